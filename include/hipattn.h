@@ -150,7 +150,8 @@ hipattn_status hipattn_sdpa(const hipattn_sdpa_desc* desc, const void* q, const 
  * side (stride[3] == 1) rides along in the tuned matrix-core kernel when the mask pointer and the
  * other strides are multiples of 16 bytes (8 elements; 16 for boolean); every other mask beside
  * 16-bit operands with a head_dim that is a multiple of 8 up to 256 takes the plain matrix-core
- * kernel; fp32 operands and larger heads take the shape-generic kernel. */
+ * kernel; fp32 operands with a head_dim that is a multiple of 4 up to 128 take the fp32 matrix-core kernel, any
+ * mask; larger heads take the shape-generic kernel. */
 typedef struct hipattn_mask_desc {
     hipattn_dtype dtype;
     int64_t stride[4];

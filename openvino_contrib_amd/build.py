@@ -18,6 +18,7 @@ SOURCES = [
     "hipattn_api.hip",
     "kv_cache_write.hip",
     "attention_generic.hip",
+    "sdpa_f32.hip",
     "paged_decode.hip",
     "paged_scores.hip",
     "flash_prefill.hip",

@@ -1,7 +1,7 @@
 // Shape-generic attention kernels: fp32 VALU arithmetic, one wavefront per (query row, head),
 // keys streamed in tiles of 64 with an online softmax.  These cover every dtype, head size
-// (<= 512) and block size the ABI accepts, serve the small f32 correctness configuration,
-// and are the on-device cross-check of the MFMA paths.  They are not tuned.
+// (<= 512) and block size the ABI accepts (dense fp32 operands up to head size 128: sdpa_f32.hip) and are the
+// on-device cross-check of the MFMA paths.  They are not tuned.
 //
 // Replaces the reference's decomposed chain MatMul -> Multiply -> Select/Add -> Softmax ->
 // MatMul (src/ops/matmul.cpp:185-227, src/ops/softmax.cpp:178-193, src/ops/select.cpp:50-91).

@@ -416,8 +416,11 @@ HIPATTN_EXPORT hipattn_status hipattn_sdpa_masked(const hipattn_sdpa_desc* desc,
         g_kernel_path = p.head_dim == 64 ? "sdpa_flash_mfma_d64" : "sdpa_flash_mfma_small";
         HIP_TRY(hipattn::launch_sdpa_flash_small(p, as_stream(stream), g_probe));
     } else {
-        g_kernel_path = "sdpa_generic";
-        HIP_TRY(hipattn::launch_sdpa_generic(p, as_stream(stream)));
+        g_kernel_path = "sdpa_generic";  // (the name of both kernels that take fp32 operands)
+        if (hipattn::sdpa_f32_supported(p))
+            HIP_TRY(hipattn::launch_sdpa_f32(p, as_stream(stream)));
+        else
+            HIP_TRY(hipattn::launch_sdpa_generic(p, as_stream(stream)));
     }
     return HIPATTN_OK;
 }

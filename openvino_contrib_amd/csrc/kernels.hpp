@@ -163,6 +163,9 @@ hipError_t launch_kv_cache_write(const KvWriteParams& p, hipStream_t stream);
 // shape-generic fp32 VALU kernels: any head_dim <= 512, any block size, every dtype
 hipError_t launch_sdpa_generic(const SdpaParams& p, hipStream_t stream);
 hipError_t launch_paged_generic(const PagedParams& p, hipStream_t stream);
+// fp32 operands on the fp32 matrix cores: head sizes up to 128 that are multiples of 4, any mask (sdpa_f32.hip)
+bool sdpa_f32_supported(const SdpaParams& p);
+hipError_t launch_sdpa_f32(const SdpaParams& p, hipStream_t stream);
 
 // MFMA flash kernels (head_dim 64 or 128, f16 / bf16)
 bool sdpa_flash_supported(const SdpaParams& p);

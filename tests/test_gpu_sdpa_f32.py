@@ -1,0 +1,39 @@
+"""fp32 attention on the fp32 matrix cores: the edges of its row and key tiles, of the split of the keys over
+wavefronts and of the head sizes, against the oracle.  Bound: 1e-4, the repository's for fp32 operands; sums of
+len_kv fp32 terms of size 1 differ from the oracle's by less than len_kv * 6e-8 of their value."""
+import numpy as np
+import pytest
+
+import helpers as H
+from openvino_contrib_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+# (batch, heads, kv heads, queries, keys, head size): one row and one key; tiles of 16 and 32 rows and keys and one
+# more; keys that leave some of the wavefronts without any; rows enough for two row tiles per wavefront; head
+# sizes at and beside the two the kernel is built for
+SHAPES = [(1, 1, 1, 1, 1, 64), (1, 2, 1, 17, 15, 64), (2, 4, 2, 16, 33, 64), (1, 8, 8, 128, 128, 64), (1, 3, 3, 31, 129, 128),
+          (3, 2, 2, 65, 64, 96), (1, 4, 1, 33, 47, 4), (2, 2, 2, 50, 17, 68), (4, 16, 16, 161, 95, 64), (3, 16, 4, 257, 260, 128),
+          (16, 16, 16, 97, 40, 32), (1, 1, 1, 5, 700, 128), (2, 12, 12, 384, 384, 64)]
+
+
+@pytest.mark.parametrize("mask", ["none", "causal", "padding", "float", "f16"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_sdpa_f32(hip, oracle, shape, mask):
+    B, Hq, Hkv, Lq, Lk, D = shape
+    case = W.make_sdpa_case(7, B, Hq, Hkv, Lq, Lk, D, W.F32)
+    rng = np.random.default_rng(3)
+    m = None
+    if mask == "padding":
+        m = np.arange(Lk)[None, None, None, :] < rng.integers(0, Lk + 1, (B, 1, 1, 1))  # (a row of zero keys gives zeros)
+    elif mask in ("float", "f16"):
+        m = rng.standard_normal((1, Hq, Lq, Lk)).astype(np.float32)
+        m[..., Lk - Lk // 3:] = -np.inf
+    if m is None:
+        out, _ = H.run_sdpa(hip, case, mask == "causal")
+        ref = oracle.sdpa(case["q"], case["k"], case["v"], causal=mask == "causal")
+    else:
+        out, _ = H.run_sdpa_masked(hip, case, m.astype(np.float16) if mask == "f16" else m)
+        ref = oracle.sdpa_masked(case["q"], case["k"], case["v"], m.astype(np.float16).astype(np.float32) if mask == "f16" else m)
+    assert np.isfinite(out).all()
+    assert H.max_abs(out, ref) <= 1e-4
