@@ -624,6 +624,21 @@ struct Line {
     }
 };
 
+// Wavefronts of `waves` that get a piece of a line of `total` units (p.min_units == 0: all of them, as the caller
+// fixed their number).  A small batch on all of them is bound by combining what they leave: every piece of a segment
+// is one more partial for the merge.  So pieces are kUnitsPerPiece units or more, except that half of the ordinary
+// count of wavefronts and two per segment are never too many, and none is empty; beyond one per compute unit only
+// whole numbers of them per compute unit (17 % more time with 1,088 than with 1,024).  One sequence of 778 tokens: 14.6 us
+// with 1,024 wavefronts, 11.2 with the 240 this gives it (12.9 with 64); of 16,384 tokens: 25.7 / 22.8 / 27.4 with
+// 1,024 / 512 / 256; 4 sequences of 256 to 4,096: 15.6 / 15.3 / 17.4; 100 sequences of 60 (800 segments): 18.9 / 22.9 with 1,024 / 512.
+constexpr int kUnitsPerPiece = 8, kFewWaves = 512;
+__device__ __forceinline__ int working_waves(const PagedParams& p, int64_t total, int waves) {
+    if (p.min_units == 0) return waves;
+    const int64_t few = max(kFewWaves, 2 * p.num_rows * p.num_heads_kv);
+    const int n = (int)min((int64_t)waves, min(total, max(few, total / p.min_units)));
+    return n > 256 ? n & ~255 : n;
+}
+
 // eight consecutive output elements, one 16-byte store for the 16-bit types
 __device__ __forceinline__ void store_out8(void* out, int64_t elem, int dtype, const float (&o)[8]) {
     if (dtype == HIPATTN_F32) {
@@ -643,24 +658,28 @@ __device__ __forceinline__ void store_out8(void* out, int64_t elem, int dtype, c
 }
 
 // Log-sum-exp reduction of the partials that pieces id_first..id_last left for query head g of
-// segment (s, h), done by one wavefront.  Pieces are taken 64 at a time: lane i fetches the
-// (max, sum) pair of piece i, the weights come out of two wavefront reductions, and the output
-// rows are then accumulated with independent loads (lane l owns head-dim 2l and 2l + 1).
+// segment (s, h), done by kParts wavefronts of a workgroup, of which `part` takes every kParts-th piece (their
+// sums meet in LDS).  Pieces are taken 64 at a time: lane i fetches the (max, sum) pair of piece i, the weights
+// come out of two wavefront reductions, and the output rows are then accumulated eight pieces at a time, the
+// eight loads ahead of the first use (lane l owns head-dim 2l and 2l + 1 and, at head size 256, 128 + 2l, 129 + 2l).
+template <int kParts>
 __device__ __forceinline__ void merge_segment_head(const PagedParams& p, const Line& line, int s, int h, int g,
-                                                   int token, int id_first, int id_last, int lane) {
+                                                   int token, int id_first, int id_last, int part, int lane,
+                                                   float4 (*shares)[64]) {
     const int Hkv = p.num_heads_kv, G = p.num_heads_q / p.num_heads_kv, D = p.head_dim;
-    // lane l owns head-dim 2l, 2l + 1 and, at head size 256, 128 + 2l, 129 + 2l
+    const int64_t seg_slot = (int64_t)s * Hkv + h;
+    const bool all_live = line.P == 0 && line.total >= line.W;  // no piece of the line is empty
+    const auto live = [&](int id) { return id <= id_last && (all_live || line.begin(id) < line.begin(id + 1)); };
     float m_run = -INFINITY, l_run = 0.0f, ox[2] = {0.0f, 0.0f}, oy[2] = {0.0f, 0.0f};
     for (int id0 = id_first; id0 <= id_last; id0 += 64) {
-        const int id = id0 + lane;
-        const bool have = id <= id_last && line.begin(id) < line.begin(id + 1);  // skip empty pieces
-        const int64_t slot = (int64_t)id + (int64_t)s * Hkv + h;
+        const bool have = live(id0 + lane);  // (empty pieces leave nothing)
         float mw = -INFINITY, lw = 0.0f;
         if (have) {
-            const float2 ml = *(const float2*)(p.part_ml + (slot * G + g) * 2);
+            const float2 ml = *(const float2*)(p.part_ml + ((seg_slot + id0 + lane) * G + g) * 2);
             mw = ml.x;
             lw = ml.y;
         }
+        const uint64_t alive = __builtin_amdgcn_ballot_w64(have);
         const float m_new = fmaxf(m_run, wave_max(mw));
         const float rescale = (m_run == -INFINITY) ? 0.0f : fast_exp2(m_run - m_new);
         const float f = (mw == -INFINITY) ? 0.0f : fast_exp2(mw - m_new);
@@ -671,21 +690,38 @@ __device__ __forceinline__ void merge_segment_head(const PagedParams& p, const L
             oy[c] *= rescale;
         }
         m_run = m_new;
-        const uint64_t live = __builtin_amdgcn_ballot_w64(have);
         const int n = min(64, id_last - id0 + 1);
-        for (int i = 0; i < n; i++) {
-            if (!((live >> i) & 1)) continue;
-            const float fi = __shfl(f, i, 64);
-            const int64_t sl = (int64_t)(id0 + i) + (int64_t)s * Hkv + h;
+        const auto rows = [&](int c) __attribute__((always_inline)) {
+            const int d = 128 * c + 2 * lane;
+            const float* const at = p.part_out + ((seg_slot + id0) * G + g) * D + (d < D ? d : 0);
+            for (int i0 = part; i0 < n; i0 += 8 * kParts) {
+                float2 v[8];
+                float fi[8];
 #pragma unroll
-            for (int c = 0; c < 2; c++) {
-                const int d = 128 * c + 2 * lane;
-                if (d < D) {
-                    const float2 v = *(const float2*)(p.part_out + (sl * G + g) * D + d);
-                    ox[c] = fmaf(fi, v.x, ox[c]);
-                    oy[c] = fmaf(fi, v.y, oy[c]);
+                for (int u = 0; u < 8; u++) {  // (a piece that does not exist: piece 0's row with weight zero)
+                    const int i = i0 + u * kParts;
+                    const bool ok = i < n && ((alive >> i) & 1) != 0;
+                    fi[u] = ok ? __shfl(f, i, 64) : 0.0f;
+                    v[u] = ok ? *(const float2*)(at + (int64_t)i * G * D) : make_float2(0.0f, 0.0f);
+                }
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    ox[c] = fmaf(fi[u], v[u].x, ox[c]);
+                    oy[c] = fmaf(fi[u], v[u].y, oy[c]);
                 }
             }
+        };
+        rows(0);
+        if (D > 128) rows(1);
+    }
+    if constexpr (kParts > 1) {
+        if (part > 0) shares[part - 1][lane] = make_float4(ox[0], oy[0], ox[1], oy[1]);
+        __syncthreads();
+        if (part > 0) return;
+#pragma unroll
+        for (int i = 0; i < kParts - 1; i++) {
+            const float4 v = shares[i][lane];
+            ox[0] += v.x, oy[0] += v.y, ox[1] += v.z, oy[1] += v.w;
         }
     }
     // (the attention sink of the head, when there is one: a logit in the denominator without a value row)
@@ -915,7 +951,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
     const int64_t total = (int64_t)prefix_at(p.num_rows) * Hkv;
     if (total <= 0) return;
     // eight to a workgroup: the plan has chosen how many of the launched wavefronts work
-    const int num_waves = kWaves == 1 ? p.num_waves : p.plan_waves[0];
+    const int num_waves = working_waves(p, total, kWaves == 1 ? p.num_waves : p.plan_waves[0]);
     if (w >= num_waves) return;
     const Line line(total, num_waves, p.dyn_pieces);
 
@@ -1480,8 +1516,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     const int Hkv = p.num_heads_kv, G = p.num_heads_q / p.num_heads_kv;
     const float c = p.scale * kLog2e;
     const int64_t total = (int64_t)p.blk_prefix[p.num_rows] * Hkv;
-    if (total <= 0 || w >= p.num_waves) return;
-    const Line line(total, p.num_waves, 0);
+    if (total <= 0) return;
+    const int num_waves = working_waves(p, total, p.num_waves);
+    if (w >= num_waves) return;
+    const Line line(total, num_waves, 0);
     const int64_t block_stride = (int64_t)(Hkv / p.kv_share) * blk * kRowBytes;
     int64_t L = line.begin(w);
     const int64_t L_end = line.begin(w + 1);
@@ -1693,22 +1731,40 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 // on.  A separate launch: the kernel boundary is what makes the partials visible, which is far
 // cheaper here than device-scope fences inside the streaming kernel (those write back and
 // invalidate whole L2 caches and cost the decode kernel almost half of its bandwidth).
-__global__ __launch_bounds__(256) void paged_merge_kernel(PagedParams p) {
+// kParts == 1: a workgroup per segment, a wavefront per query head of the group (many segments of a few pieces
+// each).  Otherwise a workgroup of kParts wavefronts per (segment, query head).
+template <int kParts>
+__global__ __launch_bounds__(kParts == 1 ? 256 : 64 * kParts) void paged_merge_kernel(PagedParams p) {
+    __shared__ float4 shares[kParts == 1 ? 1 : kParts - 1][64];
     const int Hkv = p.num_heads_kv, G = p.num_heads_q / p.num_heads_kv;
-    const int s = blockIdx.x / Hkv, h = blockIdx.x % Hkv;  // one workgroup per segment
+    const int seg = kParts == 1 ? blockIdx.x : blockIdx.x / G, s = seg / Hkv, h = seg % Hkv;
     const DecodeRange rg = ((const DecodeRange*)p.seq_info)[s];
     if (rg.nb <= 0) return;
     const int64_t total = (int64_t)p.blk_prefix[p.num_rows] * Hkv;
     if (total <= 0) return;
-    const Line line(total, p.overlap ? p.plan_waves[0] : p.num_waves, p.dyn_pieces);
+    const Line line(total, working_waves(p, total, p.overlap ? p.plan_waves[0] : p.num_waves), p.dyn_pieces);
     const int seglen = rg.nb + p.switch_cost;
     const int64_t L0 = (int64_t)p.blk_prefix[s] * Hkv + (int64_t)h * seglen + p.switch_cost, L1 = L0 + rg.nb;
     const int id_first = line.piece_at(L0), id_last = line.piece_at(L1 - 1);
     if (id_first >= id_last) return;  // a single piece covered the segment and wrote the final rows
-    for (int g = threadIdx.x >> 6; g < G; g += 4)  // one wavefront per query head of the group
-        merge_segment_head(p, line, s, h, g, rg.token, id_first, id_last, threadIdx.x & 63);
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if constexpr (kParts == 1) {
+        for (int g = wave; g < G; g += 4) merge_segment_head<1>(p, line, s, h, g, rg.token, id_first, id_last, 0, lane, shares);
+    } else {
+        merge_segment_head<kParts>(p, line, s, h, blockIdx.x % G, rg.token, id_first, id_last, wave, lane, shares);
+    }
 }
 
+static hipError_t launch_merge(const PagedParams& p, hipStream_t stream) {
+    const int segments = p.num_rows * p.num_heads_kv, G = p.num_heads_q / p.num_heads_kv;
+    // (few segments of many pieces: 16,384 tokens of one sequence, 64 pieces a segment: the step 23.8 us with four wavefronts
+    // to a query head, 23.0 with eight; one wavefront taking piece after piece, as this kernel did: 14.6 us for the merge of 25)
+    if (segments <= 128)
+        hipLaunchKernelGGL(paged_merge_kernel<8>, dim3(segments * G), dim3(512), 0, stream, p);
+    else
+        hipLaunchKernelGGL(paged_merge_kernel<1>, dim3(segments), dim3(256), 0, stream, p);
+    return hipGetLastError();
+}
 
 // Schedule options: process-wide, changed with set_option (hipattn_set_option in the C ABI).  The
 // environment variable HIPATTN_<NAME IN CAPITALS> gives an option its initial value; the
@@ -1903,6 +1959,8 @@ static unsigned long long next_merge_tag() {
 void paged_fast_plan(PagedParams& p, void* workspace) {
     const bool overlap = overlap_wanted(p);  // asks whether the caller fixed num_waves: before it is filled in
     p.overlap = overlap ? 1 : 0;
+    const bool fixed_waves = p.num_waves > 0;
+    p.min_units = fixed_waves || option(kOptDynPieces) > 0 || overlap ? 0 : kUnitsPerPiece;  // (on-demand pieces: every ticket group needs its wavefronts)
     p.num_waves = choose_num_waves(p, overlap);
     p.switch_cost = option(kOptSwitchCost);
     p.dyn_pieces = choose_dyn_pieces(p, p.num_waves, overlap);
@@ -1931,8 +1989,11 @@ void paged_fast_plan(PagedParams& p, void* workspace) {
     w += align_up(slots * sizeof(uint64_t), 256);
     // the head-256 kernel and on-demand pieces (whose order of completion is not that of their numbers) keep the merge launch
     // Built into the u8 kernels only (see kFusedBuilt).  Measured, whole steps on one machine: the 128-sequence
-    // u8 batch 0.450 ms fused against 0.454 ms with the merge launch.
-    p.fused_merge = (option(kOptFusedMerge) != 0 && p.cache_dtype == HIPATTN_U8 && p.dyn_pieces == 0 && p.head_dim <= 128) ? 1 : 0;
+    // u8 batch 0.437 ms fused against 0.440 ms with the merge launch.  Where many pieces share a segment the one wavefront that
+    // combines them in the kernel takes them two by two: one sequence of 778 tokens 36 against 12.5 us, of 16,384 88 against 24,
+    // 32 sequences of 4,000 (256 segments) 75 against 69, 64 of them (512 segments) 127 against 127: fused from there on.
+    const bool few_pieces = fixed_waves || p.num_waves <= 3 * (int64_t)p.num_rows * p.num_heads_kv;
+    p.fused_merge = (option(kOptFusedMerge) != 0 && p.cache_dtype == HIPATTN_U8 && p.dyn_pieces == 0 && p.head_dim <= 128 && few_pieces) ? 1 : 0;
     p.merge_tag = next_merge_tag();
 }
 
@@ -2151,8 +2212,7 @@ hipError_t launch_paged_fast(const PagedParams& p, const KvWriteParams* write, h
         e = hipGetLastError();
         if (probe.after) (void)hipEventRecord(probe.after, stream);
         if (e != hipSuccess || p.fused_merge) return e;
-        hipLaunchKernelGGL(paged_merge_kernel, dim3(p.num_rows * p.num_heads_kv), dim3(256), 0, stream, p);
-        return hipGetLastError();
+        return launch_merge(p, stream);
     }
     // prologue: KV-cache write of the new tokens (optional) + plan, one launch
     hipLaunchKernelGGL(paged_prologue_kernel, dim3(write_blocks + 1), dim3(256), 0, stream, wp, p, write_blocks);
@@ -2181,10 +2241,7 @@ hipError_t launch_paged_fast(const PagedParams& p, const KvWriteParams* write, h
         e = hipGetLastError();
         if (probe.after) (void)hipEventRecord(probe.after, stream);
         const hipError_t e_prefill = launch_paged_prefill(with_cache_heads(p), side->stream);
-        if (e == hipSuccess && !p.fused_merge) {
-            hipLaunchKernelGGL(paged_merge_kernel, dim3(p.num_rows * p.num_heads_kv), dim3(256), 0, stream, p);
-            e = hipGetLastError();
-        }
+        if (e == hipSuccess && !p.fused_merge) e = launch_merge(p, stream);
         // always join, also after an error, so the caller's stream never runs ahead of the side stream
         hipError_t e_join = hipEventRecord(side->join, side->stream);
         if (e_join == hipSuccess) e_join = hipStreamWaitEvent(stream, side->join, 0);
@@ -2196,8 +2253,7 @@ hipError_t launch_paged_fast(const PagedParams& p, const KvWriteParams* write, h
     if (probe.after) (void)hipEventRecord(probe.after, stream);
     if (e != hipSuccess) return e;
     if (!p.fused_merge) {
-        hipLaunchKernelGGL(paged_merge_kernel, dim3(p.num_rows * p.num_heads_kv), dim3(256), 0, stream, p);
-        e = hipGetLastError();
+        e = launch_merge(p, stream);
         if (e != hipSuccess) return e;
     }
     if (p.max_q_tiles > 0) {
