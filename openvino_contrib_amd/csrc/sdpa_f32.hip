@@ -18,7 +18,7 @@
 // taken per step.  Measured: 2 x 8 heads of 2,048 tokens at head size 64: 133 us = 129 TFLOP/s (a large fp32 matrix
 // product reaches 149 on this card); 8 x 12 heads of 384, padded: 1,660 us in the shape-generic kernel -> 37; 8 heads of
 // 128, causal: 55 -> 5.4.
-#include "device_common.hpp"
+#include "attend_row.hpp"
 #include "kernels.hpp"
 
 namespace hipattn {
@@ -319,7 +319,40 @@ __global__ __launch_bounds__(512) void sdpa_f32_kernel(SdpaParams p, int q_tiles
 #pragma unroll
     for (int nt = 0; nt < kNT; nt++) {
         const int row = row0 + 16 * nt + n;
-        if (row >= p.len_q) continue;
+        // The products multiply masked keys by a zero probability (an infinite value row would make that NaN) and let
+        // exponentials grow to 2^60 (times a value row above 1e20: infinity).  Rows that are not finite are worked again
+        // the way that skips such keys and keeps its reference at the maximum; where the inputs do ask for it they stay so.
+        float finite = 0.f;
+#pragma unroll
+        for (int cc = 0; cc < kC; cc++)
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (!kPad || 64 * cc + 16 * quarter + 4 * e < D) finite = fmaf(o[cc][t][nt][e], 0.f, finite);
+        uint64_t bad = __builtin_amdgcn_ballot_w64(finite != 0.f && row < p.len_q);
+        bad |= bad >> 32;
+        bad = (bad | bad >> 16) & 0xffff;
+        const bool again = (bad >> n) & 1;
+        while (bad != 0) {
+            const int r = row0 + 16 * nt + __builtin_ctzll(bad);
+            bad &= bad - 1;
+            const DenseKV kv{(const uint8_t*)k, (const uint8_t*)v, 4 * (int64_t)D, HIPATTN_F32};
+            const float* const q_row = q + (int64_t)r * D;
+            float x[kC];
+            if constexpr (kForm == kNoMask) {
+                attend_row_wave(q_row, kv, NoBias{}, 0, p.causal ? min(r + 1, p.len_kv) : p.len_kv, D, p.scale, x);
+            } else {
+                const int64_t at = (int64_t)b * p.mask_stride[0] + (int64_t)h * p.mask_stride[1] + (int64_t)r * p.mask_stride[2];
+                const MaskRow bias{(const uint8_t*)p.mask + at * (p.mask_dtype == HIPATTN_U8 ? 1 : dtype_bytes(p.mask_dtype)),
+                                   p.mask_stride[3], p.mask_dtype};
+                attend_row_wave(q_row, kv, bias, 0, p.len_kv, D, p.scale, x);
+            }
+#pragma unroll
+            for (int i = 0; i < kC; i++)
+                if (lane + 64 * i < D) ((float*)p.out)[((int64_t)bh * p.len_q + r) * D + lane + 64 * i] = x[i];
+        }
+        if (row >= p.len_q || again) continue;
         float* const out = (float*)p.out + ((int64_t)bh * p.len_q + row) * D;
 #pragma unroll
         for (int cc = 0; cc < kC; cc++)

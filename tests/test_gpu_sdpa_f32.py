@@ -37,3 +37,37 @@ def test_sdpa_f32(hip, oracle, shape, mask):
         ref = oracle.sdpa_masked(case["q"], case["k"], case["v"], m.astype(np.float16).astype(np.float32) if mask == "f16" else m)
     assert np.isfinite(out).all()
     assert H.max_abs(out, ref) <= 1e-4
+
+
+@pytest.mark.parametrize("shape", [(2, 4, 2, 33, 47, 64), (1, 2, 2, 20, 70, 96), (1, 4, 4, 160, 200, 128)])
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_masked_keys_may_hold_anything(hip, oracle, shape, value):
+    """Value rows of keys that a row does not attend, infinite or NaN: the row is what it is without them."""
+    B, Hq, Hkv, Lq, Lk, D = shape
+    case = W.make_sdpa_case(8, B, Hq, Hkv, Lq, Lk, D, W.F32)
+    cut = Lk - 5
+    m = np.broadcast_to(np.arange(Lk) < cut, (1, 1, 1, Lk)).copy()
+    ref = oracle.sdpa_masked(case["q"], case["k"], case["v"], m)
+    case["v"][:, :, cut:, 0] = value
+    for form in (m, np.where(m, 0.0, -np.inf).astype(np.float32)):
+        out, _ = H.run_sdpa_masked(hip, case, form)
+        assert H.max_abs(out, ref) <= 1e-4
+    case = W.make_sdpa_case(9, B, Hq, Hkv, Lq, Lk, D, W.F32)
+    ref = oracle.sdpa(case["q"], case["k"], case["v"], causal=True)
+    at = Lq // 2
+    case["v"][:, :, at, :] = value  # rows from `at` on attend it
+    out, _ = H.run_sdpa(hip, case, True)
+    assert H.max_abs(out[:, :, :at], ref[:, :, :at]) <= 1e-4
+    assert not np.isfinite(out[:, :, at:]).any()
+
+
+def test_large_values_beside_growing_scores(hip, oracle):
+    """Scores that grow by some 2^20 along the keys and values near the largest fp32: the sums stay finite."""
+    case = W.make_sdpa_case(10, 1, 2, 2, 40, 300, 64, W.F32)
+    case["q"][..., 0] = 1.0
+    case["k"][..., 0] = np.linspace(0, 160, 300, dtype=np.float32)  # (times 1 / sqrt(64))
+    case["v"] *= np.float32(2e37)
+    out, _ = H.run_sdpa(hip, case, False)
+    ref = oracle.sdpa(case["q"], case["k"], (case["v"] / np.float32(2e37)))
+    assert np.isfinite(out).all()
+    assert H.max_abs(out / np.float32(2e37), ref) <= 1e-4
