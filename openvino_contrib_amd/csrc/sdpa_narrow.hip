@@ -1,0 +1,550 @@
+// Dense attention of 16-bit operands at head sizes 64 and 72 .. 96: both products on v_mfma_f32_32x32x16, laid out
+// as in flash_prefill.hip (S^T = K Q^T with the softmax's reference in the accumulator, O^T = V^T P^T).
+//
+// What bounds it: at these head sizes a key tile has as many exponentials as at 128 and half to three quarters of
+// the matrix work, so the vector ALU is the busier unit (32 x 32 scores: 352 cycles of exp2, sum and conversion
+// against 256 of MFMAs at head size 64), and what counts is that it never waits.  So: small workgroups of four
+// wavefronts, 32 query rows each, several of them to a compute unit, which find their own phases; a wavefront computes the
+// scores of the next 32 keys and the products of the last beside the exponentials of these; no row maximum unless a sum says
+// that one is needed.  K and V tiles go straight into LDS, K in three stages (it is read half a tile ahead) and V in two.
+// Row sums are taken of the probabilities as they were rounded for the product, so that rounding them moves a row's mean less.
+//
+// Counters at 16 heads of 4,096, size 64: vector ALU 44 %, matrix cores 37 %, LDS 18 % of the cycles, no bank conflicts; the rest is
+// a step's own chain (LDS, products, exponentials, check) at two wavefronts per SIMD.
+// Measured against the head-128 kernel on padded rows: 16 x 16 heads of 577, size 64, fp16: 60 -> 33 us (660 TFLOP/s); 16 heads
+// of 4,096: 102 -> 78 (880); 8 heads of 2,048: 43 -> 19; 8 of 128: 8.6 -> 5.2; 4 x 32 of 2,048, causal: 122 -> 79; size 96,
+// 8 x 12 heads of 700: 42 -> 33; against the plain masked kernel: 4 x 12 heads of 1,100 with a bias: 135 -> 37.
+#include "device_common.hpp"
+#include "kernels.hpp"
+
+namespace hipattn {
+
+namespace narrow {
+
+constexpr int kWaves = 4;
+
+typedef __attribute__((address_space(3))) uint8_t lds_byte;
+typedef __attribute__((address_space(3))) uint4_t lds_uint4;
+typedef short short4_t __attribute__((ext_vector_type(4)));
+typedef short short8_t __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) short4_t lds_short4;
+typedef float float2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+
+template <bool kBf16>
+struct Mfma {
+    using vec8 = half8_t;
+    static __device__ __forceinline__ float16_t mma(vec8 a, vec8 b, float16_t c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
+    static __device__ __forceinline__ uint32_t cvt2(float lo, float hi) {
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector((float2_t){lo, hi}, half2_t));
+    }
+    static __device__ __forceinline__ float to_float(uint32_t bits) { return f16_bits_to_float((uint16_t)bits); }
+    // x + the two halves of w
+    static __device__ __forceinline__ float add2(uint32_t w, float x) {
+        return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, w), (half2_t){(half_t)1.0f, (half_t)1.0f}, x, false);
+    }
+    static constexpr float kSafeSum = 32768.0f;  // sixteen probabilities below it all fit fp16
+};
+template <>
+struct Mfma<true> {
+    using vec8 = bf16x8_t;
+    static __device__ __forceinline__ float16_t mma(vec8 a, vec8 b, float16_t c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+    static __device__ __forceinline__ uint32_t cvt2(float lo, float hi) {
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector((float2_t){lo, hi}, bf16x2_t));
+    }
+    static __device__ __forceinline__ float to_float(uint32_t bits) { return bf16_bits_to_float((uint16_t)bits); }
+    static __device__ __forceinline__ float add2(uint32_t w, float x) {
+        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w), (bf16x2_t){(__bf16)1.0f, (__bf16)1.0f}, x, false);
+    }
+    static constexpr float kSafeSum = 16777216.0f;
+};
+
+// 16 bytes per lane from lane_offset past a wave-uniform address to LDS byte lds_base + 16 * lane (in assembly, because the
+// compiler would wait for every load at every use of LDS; the loop waits for them before its barrier)
+__device__ __forceinline__ void load_to_lds_16(const uint8_t* base, uint32_t lane_offset, lds_byte* lds_base) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(lane_offset), "s"(base), "s"((uint32_t)(uintptr_t)lds_base)
+                 : "memory", "m0");
+}
+__device__ __forceinline__ void wait_and_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Where the 16-byte chunk c of row r of a tile lies in its row in LDS: sixteen lanes that read one chunk of sixteen rows (K)
+// and the four rows a transposing read touches (V) meet different banks.  Rows of 128 bytes: two to the width of the
+// banks; rows of 192 start in another quarter each, so that only K's need moving.
+template <int kDP>
+__device__ __forceinline__ int k_place(int r, int c) { return kDP == 64 ? c ^ ((r >> 1) & 7) : c ^ ((r >> 2) & 3); }
+template <int kDP>
+__device__ __forceinline__ int v_place(int r, int c) { return kDP == 64 ? c ^ (((r >> 1) & 1) << 2) : c; }
+
+enum MaskForm {
+    kNoMask,
+    kBoolean,   // bytes, keys side by side
+    kAdditive   // of the operands' type, keys side by side
+};
+
+// kDP: head size the kernel is built for; kPad: the call's is smaller (K's missing columns are zeros in LDS, V's whatever
+// is there: they give output columns that nobody stores).  kSplit: wavefronts that share 32 query rows, each with every
+// kSplit-th 32 keys; their results meet in LDS at the end.
+template <bool kBf16, int kDP, int kForm, bool kPad, int kSplit>
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP == 64 && kForm == kNoMask ? 3 : 2))) void sdpa_narrow_kernel(SdpaParams p, int q_tiles, int items) {
+    constexpr int kTileK = kSplit == 4 ? 128 : 64, kTileQ = 32 * kWaves / kSplit, kParts = kTileK / 32;
+    using M = Mfma<kBf16>;
+    using vec8 = typename M::vec8;
+    constexpr int kChunks = kDP / 8, kRow = kDP * 2, kStage = kTileK * kRow, kSteps = kDP / 16, kOut = kDP / 32;
+    constexpr int kLoads = kStage / 1024 / kWaves;  // load instructions per wavefront and tile
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[5 * kStage];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, n32 = lane & 31, hi = lane >> 5;
+    // workgroup ids go round the eight XCDs: consecutive items (the query tiles of a head, then those of the next head on
+    // the same K and V) stay on one and share its L2.  Causal: the longest tiles of eight heads first, so that short ones
+    // fill the end (4 x 32 heads of 2,048, size 64: 96 -> 79 us; 4 x 16 of 1,500, size 96: 51 -> 37)
+    const int G = p.num_heads_q / p.num_heads_kv, heads = p.batch * p.num_heads_q;
+    const int per_xcd = (items + 7) / 8;
+    const int item = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    if (item >= items) return;
+    int head = item / q_tiles, q0 = (q_tiles - 1 - item % q_tiles) * kTileQ;
+    if (p.causal && heads % 8 == 0) {
+        const int mine = heads / 8, at = (int)(blockIdx.x >> 3), group = at / (8 * q_tiles), in_group = at % (8 * q_tiles);
+        const int together = min(8, mine - 8 * group);
+        head = (int)(blockIdx.x & 7) * mine + 8 * group + in_group % together;
+        q0 = (q_tiles - 1 - in_group / together) * kTileQ;
+    }
+    const int part = wave % kSplit;  // which 32 keys of a tile, where several wavefronts share the rows
+    const int g = head % G, b = head / G % p.batch, hkv = head / G / p.batch, h = hkv * G + g;
+    const int D = kPad ? p.head_dim : kDP, row_bytes = 2 * D;
+    const int64_t q_off = (((int64_t)b * p.num_heads_q + h) * p.len_q) * D;
+    const int64_t kv_off = (((int64_t)b * p.num_heads_kv + hkv) * p.len_kv) * row_bytes;
+    const uint8_t* const k = (const uint8_t*)p.k + kv_off;
+    const uint8_t* const v = (const uint8_t*)p.v + kv_off;
+    const int row0 = q0 + 32 * (wave / kSplit), my_row = row0 + n32;
+    int tile0 = 0, key_end = p.causal ? min(p.len_kv, q0 + kTileQ) : p.len_kv;
+    if constexpr (kForm == kBoolean) {
+        if (p.mask_stride[2] == 0) {  // one row of keys for all queries (padding): from the first key attended to the last
+            const uint8_t* const keys = (const uint8_t*)p.mask + (int64_t)b * p.mask_stride[0] + (int64_t)h * p.mask_stride[1];
+            int first = key_end, last = -1;
+            for (int at = 4 * lane; at < p.len_kv; at += 256)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (keys[min(at + e, p.len_kv - 1)] != 0) first = min(first, at + e), last = max(last, min(at + e, p.len_kv - 1));
+#pragma unroll
+            for (int x = 32; x > 0; x >>= 1) first = min(first, __shfl_xor(first, x, 64)), last = max(last, __shfl_xor(last, x, 64));
+            tile0 = __builtin_amdgcn_readfirstlane(min(first, last + 1) / kTileK);
+            key_end = __builtin_amdgcn_readfirstlane(last + 1);
+        }
+    }
+    const int tiles = (key_end + kTileK - 1) / kTileK;
+    // steps of 32 keys before which this wavefront is done (one without rows only helps to load)
+    const int steps = row0 >= p.len_q ? 0 : ((p.causal ? min(key_end, row0 + 32) : key_end) + 31) / 32;
+
+    lds_byte* const k_lds = (lds_byte*)lds;
+    lds_byte* const v_lds = k_lds + 3 * kStage;
+    if constexpr (kPad) {  // the columns that no load writes
+        for (int i = threadIdx.x; i < 3 * kStage / 16; i += 64 * kWaves) ((lds_uint4*)k_lds)[i] = (uint4_t){0u, 0u, 0u, 0u};
+        __syncthreads();
+    }
+    // this lane's part of load instruction i (of kLoads) of a tile: a row of the tile and a chunk of it
+    int load_row[kLoads], k_chunk[kLoads], v_chunk[kLoads];
+    uint32_t k_off[kLoads], v_off[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; i++) {
+        const int place = 64 * (wave + kWaves * i) + lane;
+        load_row[i] = place / kChunks;
+        k_chunk[i] = k_place<kDP>(load_row[i], place % kChunks);
+        v_chunk[i] = v_place<kDP>(load_row[i], place % kChunks);
+        k_off[i] = (uint32_t)(load_row[i] * row_bytes + 16 * k_chunk[i]);
+        v_off[i] = (uint32_t)(load_row[i] * row_bytes + 16 * v_chunk[i]);
+    }
+    auto load_tile = [&](const uint8_t* base, const uint32_t (&off)[kLoads], const int (&chunk)[kLoads], int keys, lds_byte* stage)
+                         __attribute__((always_inline)) {
+        if (keys >= kTileK) {
+#pragma unroll
+            for (int i = 0; i < kLoads; i++)
+                if (!kPad || 8 * chunk[i] < D) load_to_lds_16(base, off[i], stage + (wave + kWaves * i) * 1024);
+        } else {  // (rows past the end repeat the last key: they are masked)
+#pragma unroll
+            for (int i = 0; i < kLoads; i++)
+                if (!kPad || 8 * chunk[i] < D)
+                    load_to_lds_16(base, off[i] - (uint32_t)(max((kPad ? load_row[i] : (int)off[i] / kRow) - (keys - 1), 0) * row_bytes), stage + (wave + kWaves * i) * 1024);
+        }
+    };
+    const int tile_bytes = kTileK * row_bytes;
+    const uint8_t* k_src = k + (int64_t)tile0 * tile_bytes;  // the next tile of K and of V to load
+    const uint8_t* v_src = v + (int64_t)tile0 * tile_bytes;
+    int k_keys = p.len_kv - tile0 * kTileK, v_keys = k_keys;
+    auto load_k = [&](lds_byte* stage) __attribute__((always_inline)) {
+        load_tile(k_src, k_off, k_chunk, k_keys, stage);
+        k_src += tile_bytes, k_keys -= kTileK;
+    };
+    auto load_v = [&](lds_byte* stage) __attribute__((always_inline)) {
+        load_tile(v_src, v_off, v_chunk, v_keys, stage);
+        v_src += tile_bytes, v_keys -= kTileK;
+    };
+    if (tile0 < tiles) {
+        load_k(k_lds);
+        load_v(v_lds);
+        if (tile0 + 1 < tiles) load_k(k_lds + kStage);
+    }
+
+    vec8 qf[kSteps];  // Q^T: lane (n32, hi) holds row n32, columns 16 i + 8 hi .. + 7, times scale * log2(e)
+    {
+        const float c = p.scale * kLog2e;
+        const uint16_t* const row = (const uint16_t*)p.q + q_off + (int64_t)min(my_row, p.len_q - 1) * D + 8 * hi;
+#pragma unroll
+        for (int i = 0; i < kSteps; i++) {
+            uint4_t raw = {0u, 0u, 0u, 0u};
+            if (!kPad || 16 * i + 8 * hi < D) raw = *(const uint4_t*)(row + 16 * i);
+            uint4_t x;
+#pragma unroll
+            for (int e = 0; e < 4; e++) x[e] = M::cvt2(M::to_float(raw[e] & 0xffffu) * c, M::to_float(raw[e] >> 16) * c);
+            qf[i] = __builtin_bit_cast(vec8, x);
+        }
+    }
+    // K fragment of key half and k-step i: chunk 2 i + hi of row n32; V^T fragment of 16 keys ks and output tile dt: two
+    // transposing reads of four rows each, eight rows apart (lane i of a group of sixteen addresses row i / 4, columns
+    // 4 (i % 4) .. + 3 and receives column i of the four rows)
+    // (chunk 2 i + hi moves by an exclusive or, so that every k-step's place is the first one's ^ 32 i at size 64, and within
+    // 64 bytes at 96)
+    const int k_at0 = n32 * kRow + 16 * k_place<kDP>(n32, hi);
+    auto k_at = [&](int i) __attribute__((always_inline)) -> int { return kDP == 64 ? k_at0 ^ (32 * i) : (k_at0 ^ (32 * (i & 1))) + 64 * (i >> 1); };
+    int v_at[kOut];
+    {
+        const int grp = lane >> 4, i16 = lane & 15, row = 4 * (grp >> 1) + (i16 >> 2);
+#pragma unroll
+        for (int dt = 0; dt < kOut; dt++) v_at[dt] = row * kRow + 16 * v_place<kDP>(row, 4 * dt + 2 * (grp & 1) + ((i16 & 3) >> 1)) + 8 * (i16 & 1);
+    }
+    float16_t neg_ref;
+#pragma unroll
+    for (int r = 0; r < 16; r++) neg_ref[r] = 0.f;
+    float16_t o[kOut];
+#pragma unroll
+    for (int dt = 0; dt < kOut; dt++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[dt][r] = 0.f;
+    float l_run = 0.f;       // this lane's half of the row's sum
+    bool started = false;    // the row has met a key that it attends
+
+    // exponents of the softmax of 32 keys: register r is key 8 (r / 4) + 4 hi + r % 4 of the half
+    auto scores = [&](const lds_byte* stage, int half, float16_t& s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kSteps; i++)
+            s = M::mma(__builtin_bit_cast(vec8, *(const lds_uint4*)(stage + k_at(i) + half * 32 * kRow)), qf[i], i == 0 ? neg_ref : s);
+    };
+    // the mask of step t for this lane's row: words of four keys (8 g + 4 hi .. + 3)
+    constexpr int kMaskWords = kForm == kAdditive ? 8 : kForm == kBoolean ? 4 : 1;
+    uint32_t mask[kMaskWords];
+    const uint8_t* mask_row = nullptr;
+    if constexpr (kForm != kNoMask) {
+        constexpr int esz = kForm == kBoolean ? 1 : 2;
+        mask_row = (const uint8_t*)p.mask + ((int64_t)b * p.mask_stride[0] + (int64_t)h * p.mask_stride[1] +
+                                             (int64_t)min(my_row, p.len_q - 1) * p.mask_stride[2]) * esz;
+    }
+    auto load_mask = [&](int t) __attribute__((always_inline)) {
+        if constexpr (kForm != kNoMask) {
+            constexpr int esz = kForm == kBoolean ? 1 : 2;
+#pragma unroll
+            for (int g4 = 0; g4 < 4; g4++) {
+                const int key = 32 * t + 8 * g4 + 4 * hi;
+                uint32_t w[esz] = {};
+                if (key + 4 <= p.len_kv) {
+                    __builtin_memcpy(w, mask_row + (int64_t)key * esz, 4 * esz);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)  // (keys past the end: masked anyway)
+                        if (key + e < p.len_kv) {
+                            if constexpr (esz == 1)
+                                w[0] |= (uint32_t)mask_row[key + e] << (8 * e);
+                            else
+                                w[e >> 1] |= (uint32_t)((const uint16_t*)mask_row)[key + e] << (16 * (e & 1));
+                        }
+                }
+#pragma unroll
+                for (int x = 0; x < esz; x++) mask[esz * g4 + x] = w[x];
+            }
+        }
+    };
+    vec8 pf[2], vf[2][kOut];  // probabilities of the step before and the V^T fragments that they meet
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+        pf[ks] = __builtin_bit_cast(vec8, (uint4_t){0u, 0u, 0u, 0u});
+#pragma unroll
+        for (int dt = 0; dt < kOut; dt++) vf[ks][dt] = pf[ks];
+    }
+    auto accumulate = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+            for (int dt = 0; dt < kOut; dt++) o[dt] = M::mma(vf[ks][dt], pf[ks], o[dt]);
+    };
+    // One step: its exponentials, and beside them on the matrix core O^T += V^T P^T of the step before and the scores of the next.
+    auto step = [&](int t, float16_t& s, float16_t& s_next, const lds_byte* k_next, int half_next, const lds_byte* v_stage, int half)
+                    __attribute__((always_inline)) {
+        if constexpr (kForm == kBoolean) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) s[r] = ((mask[r >> 2] >> (8 * (r & 3))) & 0xffu) != 0 ? s[r] : -INFINITY;
+        }
+        if constexpr (kForm == kAdditive) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) s[r] = fmaf(M::to_float((mask[r >> 1] >> (16 * (r & 1))) & 0xffffu), kLog2e, s[r]);
+        }
+        if constexpr (kForm != kNoMask) {
+            constexpr int kNext = kSplit == 1 ? 1 : kParts;  // from one step of a wavefront to its next
+            if (t + kNext < steps) load_mask(t + kNext);
+        }
+        if (32 * t + 32 > p.len_kv || (p.causal && 32 * t + 31 > row0)) {
+            const int end = (p.causal ? min(p.len_kv, my_row + 1) : p.len_kv) - 32 * t - 4 * hi;
+#pragma unroll
+            for (int r = 0; r < 16; r++) s[r] = 8 * (r >> 2) + (r & 3) < end ? s[r] : -INFINITY;
+        }
+        vec8 pn[2];
+        auto probabilities = [&](int ks) __attribute__((always_inline)) -> float {  // of sixteen keys; returns their sum
+            float sum = 0.f;
+            uint4_t w;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                w[e] = M::cvt2(fast_exp2(s[8 * ks + 2 * e]), fast_exp2(s[8 * ks + 2 * e + 1]));
+                sum = M::add2(w[e], sum);
+            }
+            pn[ks] = __builtin_bit_cast(vec8, w);
+            return sum;
+        };
+        // In this order (the compiler would read each fragment right before its use and wait for it every time), with the
+        // matrix instructions spread over the vector ones
+        vec8 kf[kSteps];
+#pragma unroll
+        for (int i = 0; i < kSteps; i++) kf[i] = __builtin_bit_cast(vec8, *(const lds_uint4*)(k_next + k_at(i) + half_next * 32 * kRow));
+        __builtin_amdgcn_sched_barrier(0);
+        accumulate();
+        float sum = probabilities(0);
+#pragma unroll
+        for (int x = 0; x < 2 * kOut; x++) {
+            __builtin_amdgcn_sched_group_barrier(0x2, 24 / (2 * kOut), 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+            for (int dt = 0; dt < kOut; dt++) {
+                const lds_byte* const at = v_stage + v_at[dt] + (2 * half + ks) * 16 * kRow;
+                const short4_t a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)at);
+                const short4_t a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(at + 8 * kRow));
+                const short8_t a = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+                vf[ks][dt] = __builtin_bit_cast(vec8, a);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < kSteps; i++) s_next = M::mma(kf[i], qf[i], i == 0 ? neg_ref : s_next);  // (after the last step: unused)
+        sum += probabilities(1);
+#pragma unroll
+        for (int x = 0; x < kSteps; x++) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, 24 / kSteps, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // The reference stays while every sum says that no probability can have overflowed; otherwise, and for the first
+        // keys of a row, it moves to the largest score (all in units of exponents to base 2).
+        if (__builtin_amdgcn_ballot_w64(!started || !(sum < M::kSafeSum)) != 0) {
+            float top = -INFINITY;
+#pragma unroll
+            for (int r = 0; r < 16; r++) top = fmaxf(top, s[r]);
+            const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(top), __float_as_uint(top), false, false);
+            top = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+            const bool seen = top != -INFINITY;
+            if (__builtin_amdgcn_ballot_w64(top > 8.0f || (seen && !started)) != 0) {
+                const float delta = started ? fmaxf(top, 0.f) : (seen ? top : 0.f);
+                const float alpha = fast_exp2(-fmaxf(delta, 0.f));
+                l_run *= alpha;
+#pragma unroll
+                for (int dt = 0; dt < kOut; dt++) o[dt] *= alpha;
+                s -= delta;
+                s_next -= delta;
+                neg_ref -= delta;
+                started = started || seen;
+            }
+            sum = probabilities(0) + probabilities(1);
+        }
+        l_run += sum;
+        pf[0] = pn[0], pf[1] = pn[1];
+    };
+
+    float16_t s0, s1;
+    lds_byte *k_now = k_lds, *k_next = k_lds + kStage, *k_fill = k_lds + 2 * kStage, *v_now = v_lds, *v_fill = v_lds + kStage;
+    const int t0 = kParts * tile0 + part;
+    if (t0 < steps) load_mask(t0);
+    wait_and_barrier();
+    scores(k_now, part, s0);
+    // One tile: K of the next tile and V of this one, loaded an iteration ago, are there for every wavefront, and the
+    // stages that are filled now were last read before the barrier
+    auto iteration = [&](int j, float16_t& a, float16_t& b) __attribute__((always_inline)) {
+        if (j > tile0) wait_and_barrier();
+        if (j + 2 < tiles) load_k(k_fill);
+        if (j + 1 < tiles) load_v(v_fill);
+        const int t = kParts * j + part;
+        if constexpr (kSplit == 1) {
+            if (t < steps) step(t, a, b, k_now, 1, v_now, 0);
+            if (t + 1 < steps) step(t + 1, b, a, k_next, 0, v_now, 1);
+        } else {
+            if (t < steps) step(t, a, b, k_next, part, v_now, part);
+        }
+        lds_byte *const k_done = k_now, *const v_done = v_now;
+        k_now = k_next, k_next = k_fill, k_fill = k_done;
+        v_now = v_fill, v_fill = v_done;
+    };
+    if constexpr (kSplit == 1) {
+        for (int j = tile0; j < tiles; j++) iteration(j, s0, s1);
+    } else {
+        for (int j = tile0; j < tiles; j += 2) {
+            iteration(j, s0, s1);
+            if (j + 1 < tiles) iteration(j + 1, s1, s0);
+        }
+    }
+    accumulate();
+
+    const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
+    float l = __uint_as_float(both[0]) + __uint_as_float(both[1]);
+    uint16_t* const out = (uint16_t*)p.out + q_off + (int64_t)my_row * D;
+    // x[0 .. 7]: columns 32 dt + 8 gg + 4 hi + r % 4 (r < 4) and eight further; lanes l and l + 32 exchange halves so that
+    // each stores eight in a row
+    auto store = [&](const float (&x)[8], int dt, int gg) __attribute__((always_inline)) {
+        const auto a = __builtin_amdgcn_permlane32_swap(M::cvt2(x[0], x[1]), M::cvt2(x[4], x[5]), false, false);
+        const auto c = __builtin_amdgcn_permlane32_swap(M::cvt2(x[2], x[3]), M::cvt2(x[6], x[7]), false, false);
+        const int d = 32 * dt + 8 * (gg + hi);
+        if (my_row < p.len_q && (!kPad || d < D)) *(uint4_t*)(out + d) = (uint4_t){a[0], c[0], a[1], c[1]};
+    };
+    if constexpr (kSplit == 1) {
+        const float inv = l > 0.f ? 1.0f / l : 0.f;
+#pragma unroll
+        for (int dt = 0; dt < kOut; dt++)
+#pragma unroll
+            for (int gg = 0; gg < 4; gg += 2) {
+                float x[8];
+#pragma unroll
+                for (int r = 0; r < 8; r++) x[r] = o[dt][4 * gg + r] * inv;
+                store(x, dt, gg);
+            }
+    } else {
+        typedef __attribute__((address_space(3))) float lds_float;
+        lds_float* const shares = (lds_float*)lds;  // [wavefront][reference, sum, accumulators][lane]
+        constexpr int kShare = (16 * kOut + 2) * 64;
+        static_assert(kWaves * kShare * 4 <= 5 * kStage, "the shares take the place of the stages");
+        __syncthreads();  // (every wavefront is done with the stages, and no load is under way)
+        lds_float* const mine = shares + wave * kShare + lane;
+        mine[0] = started ? -neg_ref[0] : -INFINITY;
+        mine[64] = l;
+#pragma unroll
+        for (int dt = 0; dt < kOut; dt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) mine[(2 + 16 * dt + r) * 64] = o[dt][r];
+        __syncthreads();
+        const lds_float* const first = shares + (wave - part) * kShare + lane;
+        float f[kSplit], top = -INFINITY, total = 0.f;
+#pragma unroll
+        for (int x = 0; x < kSplit; x++) f[x] = first[x * kShare], top = fmaxf(top, f[x]);
+#pragma unroll
+        for (int x = 0; x < kSplit; x++) {
+            f[x] = f[x] == -INFINITY ? 0.f : fast_exp2(f[x] - top);
+            total = fmaf(f[x], first[x * kShare + 64], total);
+        }
+        const float inv = total > 0.f ? 1.0f / total : 0.f;
+#pragma unroll
+        for (int i = 0; i < 2 * kOut; i++) {  // eight accumulators each: the sharers take turns
+            if (i % kSplit != part) continue;
+            float x[8];
+#pragma unroll
+            for (int r = 0; r < 8; r++) {
+                float sum = 0.f;
+#pragma unroll
+                for (int w = 0; w < kSplit; w++) sum = fmaf(f[w], first[w * kShare + (2 + 8 * i + r) * 64], sum);
+                x[r] = sum * inv;
+            }
+            store(x, i / 2, 2 * (i % 2));
+        }
+    }
+}
+
+// Wavefronts that share 32 query rows, from the time the busiest compute unit would take, in microseconds: per step 0.30 and
+// 0.14 for every workgroup beside each other on it (fitted to 0.41 / 0.59 / 0.74 with one to three), a fifth more where every
+// step has a barrier, and what a workgroup costs however few its steps are.  Measured around the lines it draws, with
+// 1 / 2 / 4: 8 heads of 2,048, size 64: 29.5 / 20.1 / 19.8 us; 12 of 800: 14.2 / 10.8 / 12.0; 48 of 800: 18.4 / 16.7 / 26.6; 96 of
+// 800: 24.8 / 27.7 / 49.2; 96 of 130: 6.4 / 7.3 / 7.7; 64 of 77 rows and 1,024 keys: 16.2 / 12.0 / 10.1; 16 of 4,096: 80 / 88 / 121.
+int choose_split(const SdpaParams& p) {
+    int best = 1;
+    double best_cost = 0;
+    for (int split = 1; split <= 4; split *= 2) {
+        const int64_t groups = (int64_t)p.batch * p.num_heads_q * ((p.len_q + 128 / split - 1) / (128 / split));
+        const int resident = p.head_dim <= 64 ? (split == 4 || p.mask ? 2 : 3) : (split == 4 ? 1 : 2);
+        const int steps = ((p.len_kv + 31) / 32 + split - 1) / split;
+        double cost = 0;
+        for (int64_t left = (groups + 255) / 256, n; left > 0; left -= n) {
+            n = left < resident ? left : resident;
+            const double round = steps * (0.30 + 0.14 * (double)n) * (split == 1 ? 1.0 : 1.2) + (split == 1 ? 1.5 : split == 2 ? 2.2 : 2.5 + 0.9 * (double)n);
+            if (left > 8 * resident) {  // (many rounds alike)
+                const int64_t rounds = left / resident - 1;
+                cost += (double)rounds * round;
+                left -= rounds * resident;
+            }
+            cost += round;
+        }
+        if (best_cost == 0 || cost < best_cost) best_cost = cost, best = split;
+    }
+    return best;
+}
+
+template <bool kBf16, int kDP, int kForm, int kSplit>
+void launch(const SdpaParams& p, hipStream_t stream) {
+    constexpr int kRows = 32 * kWaves / kSplit;
+    const int q_tiles = (p.len_q + kRows - 1) / kRows, items = p.batch * p.num_heads_q * q_tiles;
+    const dim3 grid((unsigned)((items + 7) / 8 * 8)), block(64 * kWaves);
+    if constexpr (kDP != 64)
+        if (p.head_dim < kDP) {
+            hipLaunchKernelGGL((sdpa_narrow_kernel<kBf16, kDP, kForm, true, kSplit>), grid, block, 0, stream, p, q_tiles, items);
+            return;
+        }
+    hipLaunchKernelGGL((sdpa_narrow_kernel<kBf16, kDP, kForm, false, kSplit>), grid, block, 0, stream, p, q_tiles, items);
+}
+
+template <bool kBf16, int kDP, int kForm>
+void launch(const SdpaParams& p, hipStream_t stream) {
+    const int split = choose_split(p);
+    if (split == 1)
+        launch<kBf16, kDP, kForm, 1>(p, stream);
+    else if (split == 2)
+        launch<kBf16, kDP, kForm, 2>(p, stream);
+    else
+        launch<kBf16, kDP, kForm, 4>(p, stream);
+}
+
+template <bool kBf16, int kDP>
+void launch(const SdpaParams& p, hipStream_t stream) {
+    if (!p.mask)
+        launch<kBf16, kDP, kNoMask>(p, stream);
+    else if (p.mask_dtype == HIPATTN_U8)
+        launch<kBf16, kDP, kBoolean>(p, stream);
+    else
+        launch<kBf16, kDP, kAdditive>(p, stream);
+}
+
+}  // namespace narrow
+
+// 16-bit operands at 16-byte aligned addresses; no mask, or one whose keys lie side by side, boolean or of the operands' type.
+bool sdpa_narrow_supported(const SdpaParams& p) {
+    if (p.dtype != HIPATTN_F16 && p.dtype != HIPATTN_BF16) return false;
+    if (p.head_dim != 64 && (p.head_dim < 72 || p.head_dim > 96 || p.head_dim % 8 != 0)) return false;
+    if (p.mask && (p.mask_stride[3] != 1 || (p.mask_dtype != HIPATTN_U8 && p.mask_dtype != p.dtype))) return false;
+    const int64_t tiles = (int64_t)p.batch * p.num_heads_q * (((int64_t)p.len_q + 31) / 32);
+    return p.len_q > 0 && p.len_kv > 0 && p.batch > 0 && tiles < (1 << 30) &&
+           (((uintptr_t)p.q | (uintptr_t)p.k | (uintptr_t)p.v | (uintptr_t)p.out) & 15) == 0;
+}
+
+hipError_t launch_sdpa_narrow(const SdpaParams& p, hipStream_t stream, const KernelProbe& probe) {
+    if (probe.before) (void)hipEventRecord(probe.before, stream);
+    if (p.dtype == HIPATTN_BF16)
+        p.head_dim == 64 ? narrow::launch<true, 64>(p, stream) : narrow::launch<true, 96>(p, stream);
+    else
+        p.head_dim == 64 ? narrow::launch<false, 64>(p, stream) : narrow::launch<false, 96>(p, stream);
+    const hipError_t e = hipGetLastError();
+    if (probe.after) (void)hipEventRecord(probe.after, stream);
+    return e;
+}
+
+}  // namespace hipattn
