@@ -1358,8 +1358,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 }  // namespace flash
 
 // Head size 128, and the smaller head sizes that are multiples of 8, which run the same kernel with rows of
-// fewer columns in memory, 64 and 72 .. 96 in sdpa_narrow.hip (16-byte aligned operands; the option sdpa_padded_rows = 0
-// leaves them to the plain kernels).  Measured on 4 x 2,048 tokens, 32 / 8 heads, causal: head size 64 0.079 ms there, 0.122 on
+// fewer columns in memory, 64 and 72 .. 96 and some calls of 104 .. 128 in sdpa_narrow.hip (16-byte aligned operands; the
+// option sdpa_padded_rows = 0 leaves them to the plain kernels).  Measured on 4 x 2,048 tokens, 32 / 8 heads, causal: head size 64 0.079 ms there, 0.122 on
 // padded rows, 0.153 in the plain head-64 kernel; head size 32 0.120 ms on padded rows.
 bool sdpa_flash_supported(const SdpaParams& p) {
     if (!(p.dtype == HIPATTN_F16 || p.dtype == HIPATTN_BF16)) return false;
@@ -1389,7 +1389,7 @@ bool sdpa_flash_mask_supported(const SdpaParams& p) {
 
 hipError_t launch_sdpa_flash(const SdpaParams& p, hipStream_t stream, const KernelProbe& probe) {
     if (p.batch == 0 || p.len_q == 0) return hipSuccess;
-    if (p.head_dim != flash::kD && sdpa_narrow_supported(p)) return launch_sdpa_narrow(p, stream, probe);
+    if (sdpa_narrow_supported(p) && sdpa_narrow_preferred(p)) return launch_sdpa_narrow(p, stream, probe);
     const int G = p.num_heads_q / p.num_heads_kv;
     const int n_qt = (p.len_q + flash::kTileQ - 1) / flash::kTileQ;
     const bool pair_heads = (G & 1) == 0;

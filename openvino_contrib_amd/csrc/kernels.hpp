@@ -172,8 +172,10 @@ hipError_t launch_sdpa_f32(const SdpaParams& p, hipStream_t stream);
 bool sdpa_flash_supported(const SdpaParams& p);
 bool sdpa_flash_mask_supported(const SdpaParams& p);  // p.mask can ride along in the flash kernel
 hipError_t launch_sdpa_flash(const SdpaParams& p, hipStream_t stream, const KernelProbe& probe);
-// 16-bit operands at head sizes 64 and 72 .. 96, masks with keys side by side (sdpa_narrow.hip)
+// 16-bit operands at head sizes 64 and 72 .. 128, masks with keys side by side (sdpa_narrow.hip); preferred: to the kernel
+// of flash_prefill.hip where that takes the call too
 bool sdpa_narrow_supported(const SdpaParams& p);
+bool sdpa_narrow_preferred(const SdpaParams& p);
 hipError_t launch_sdpa_narrow(const SdpaParams& p, hipStream_t stream, const KernelProbe& probe);
 
 // head sizes up to 256 that are multiples of 8 on the matrix cores (flash_small.hip)

@@ -1,7 +1,7 @@
-// Dense attention of 16-bit operands at head sizes 64 and 72 .. 96: both products on v_mfma_f32_32x32x16, laid out
+// Dense attention of 16-bit operands at head sizes 64 and 72 .. 128: both products on v_mfma_f32_32x32x16, laid out
 // as in flash_prefill.hip (S^T = K Q^T with the softmax's reference in the accumulator, O^T = V^T P^T).
 //
-// What bounds it: at these head sizes a key tile has as many exponentials as at 128 and half to three quarters of
+// What bounds it: below 128 a key tile has as many exponentials as at 128 and half to three quarters of
 // the matrix work, so the vector ALU is the busier unit (32 x 32 scores: 352 cycles of exp2, sum and conversion
 // against 256 of MFMAs at head size 64), and what counts is that it never waits.  So: small workgroups of four
 // wavefronts, 32 query rows each, several of them to a compute unit, which find their own phases; a wavefront computes the
@@ -13,7 +13,8 @@
 // a step's own chain (LDS, products, exponentials, check) at two wavefronts per SIMD.
 // Measured against the head-128 kernel on padded rows: 16 x 16 heads of 577, size 64, fp16: 60 -> 33 us (660 TFLOP/s); 16 heads
 // of 4,096: 102 -> 78 (880); 8 heads of 2,048: 43 -> 19; 8 of 128: 8.6 -> 5.2; 4 x 32 of 2,048, causal: 122 -> 79; size 96,
-// 8 x 12 heads of 700: 42 -> 33; against the plain masked kernel: 4 x 12 heads of 1,100 with a bias: 135 -> 37.
+// 8 x 12 heads of 700: 42 -> 34; against the plain masked kernel: 4 x 12 heads of 1,100 with a bias: 135 -> 37, size 128,
+// 4 x 32 heads of 1,000, padded: 454 -> 79.
 #include "device_common.hpp"
 #include "kernels.hpp"
 
@@ -73,9 +74,9 @@ __device__ __forceinline__ void wait_and_barrier() { asm volatile("s_waitcnt vmc
 // and the four rows a transposing read touches (V) meet different banks.  Rows of 128 bytes: two to the width of the
 // banks; rows of 192 start in another quarter each, so that only K's need moving.
 template <int kDP>
-__device__ __forceinline__ int k_place(int r, int c) { return kDP == 64 ? c ^ ((r >> 1) & 7) : c ^ ((r >> 2) & 3); }
+__device__ __forceinline__ int k_place(int r, int c) { return kDP == 64 ? c ^ ((r >> 1) & 7) : kDP == 96 ? c ^ ((r >> 2) & 3) : c ^ (r & 15); }
 template <int kDP>
-__device__ __forceinline__ int v_place(int r, int c) { return kDP == 64 ? c ^ (((r >> 1) & 1) << 2) : c; }
+__device__ __forceinline__ int v_place(int r, int c) { return kDP == 64 ? c ^ (((r >> 1) & 1) << 2) : kDP == 96 ? c : c ^ ((r & 3) << 2); }
 
 enum MaskForm {
     kNoMask,
@@ -202,10 +203,10 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
     // K fragment of key half and k-step i: chunk 2 i + hi of row n32; V^T fragment of 16 keys ks and output tile dt: two
     // transposing reads of four rows each, eight rows apart (lane i of a group of sixteen addresses row i / 4, columns
     // 4 (i % 4) .. + 3 and receives column i of the four rows)
-    // (chunk 2 i + hi moves by an exclusive or, so that every k-step's place is the first one's ^ 32 i at size 64, and within
-    // 64 bytes at 96)
+    // (chunk 2 i + hi moves by an exclusive or, so that every k-step's place is the first one's ^ 32 i in rows of 128 and 256 bytes, and
+    // within 64 bytes in those of 192)
     const int k_at0 = n32 * kRow + 16 * k_place<kDP>(n32, hi);
-    auto k_at = [&](int i) __attribute__((always_inline)) -> int { return kDP == 64 ? k_at0 ^ (32 * i) : (k_at0 ^ (32 * (i & 1))) + 64 * (i >> 1); };
+    auto k_at = [&](int i) __attribute__((always_inline)) -> int { return kDP != 96 ? k_at0 ^ (32 * i) : (k_at0 ^ (32 * (i & 1))) + 64 * (i >> 1); };
     int v_at[kOut];
     {
         const int grp = lane >> 4, i16 = lane & 15, row = 4 * (grp >> 1) + (i16 >> 2);
@@ -462,30 +463,30 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
     }
 }
 
-// Wavefronts that share 32 query rows, from the time the busiest compute unit would take, in microseconds: per step 0.30 and
-// 0.14 for every workgroup beside each other on it (fitted to 0.41 / 0.59 / 0.74 with one to three), a fifth more where every
-// step has a barrier, and what a workgroup costs however few its steps are.  Measured around the lines it draws, with
-// 1 / 2 / 4: 8 heads of 2,048, size 64: 29.5 / 20.1 / 19.8 us; 12 of 800: 14.2 / 10.8 / 12.0; 48 of 800: 18.4 / 16.7 / 26.6; 96 of
-// 800: 24.8 / 27.7 / 49.2; 96 of 130: 6.4 / 7.3 / 7.7; 64 of 77 rows and 1,024 keys: 16.2 / 12.0 / 10.1; 16 of 4,096: 80 / 88 / 121.
-int choose_split(const SdpaParams& p) {
-    int best = 1;
-    double best_cost = 0;
+// Wavefronts that share 32 query rows, from the time the busiest compute unit would take, in microseconds: per step 0.30 and a
+// share for every workgroup beside each other on it (fitted: size 64 0.41 / 0.59 / 0.74 with one to three, size 128 0.64 / 0.96
+// with one and two), a fifth more where every step has a barrier, and what a workgroup costs however few its steps are.
+// Measured around the lines it draws, with 1 / 2 / 4: 8 heads of 2,048, size 64: 29.5 / 20.1 / 19.8 us; 12 of 800: 14.2 / 10.8 /
+// 12.0; 48 of 800: 18.4 / 16.7 / 26.6; 96 of 800: 24.8 / 27.7 / 49.2; 96 of 130: 6.4 / 7.3 / 7.7; 64 of 77 rows and 1,024 keys:
+// 16.2 / 12.0 / 10.1; 16 of 4,096: 80 / 88 / 121; size 128, 12 of 1,000: 25.2 / 17.2 / 27.7; 12 of 500, causal: 14.6 / 11.2 / 10.2.
+struct Split {
+    int split;
+    double cost;
+};
+Split choose_split(const SdpaParams& p) {
+    Split best{1, 0};
     for (int split = 1; split <= 4; split *= 2) {
         const int64_t groups = (int64_t)p.batch * p.num_heads_q * ((p.len_q + 128 / split - 1) / (128 / split));
+        const int64_t per_cu = (groups + 255) / 256;
         const int resident = p.head_dim <= 64 ? (split == 4 || p.mask ? 2 : 3) : (split == 4 ? 1 : 2);
-        const int steps = ((p.len_kv + 31) / 32 + split - 1) / split;
-        double cost = 0;
-        for (int64_t left = (groups + 255) / 256, n; left > 0; left -= n) {
-            n = left < resident ? left : resident;
-            const double round = steps * (0.30 + 0.14 * (double)n) * (split == 1 ? 1.0 : 1.2) + (split == 1 ? 1.5 : split == 2 ? 2.2 : 2.5 + 0.9 * (double)n);
-            if (left > 8 * resident) {  // (many rounds alike)
-                const int64_t rounds = left / resident - 1;
-                cost += (double)rounds * round;
-                left -= rounds * resident;
-            }
-            cost += round;
-        }
-        if (best_cost == 0 || cost < best_cost) best_cost = cost, best = split;
+        const int steps = ((p.len_kv + 31) / 32 + split - 1) / split;  // (causal: of the longest)
+        const double share = p.head_dim <= 64 ? 0.14 : p.head_dim <= 96 ? 0.21 : 0.32;
+        const auto round = [&](int n) {
+            const double fixed = split == 1 ? (p.head_dim <= 64 ? 1.5 : 2.5 * n - 1.0) : split == 2 ? 2.2 : 2.5 + 0.9 * n;
+            return steps * (0.30 + share * n) * (split == 1 ? 1.0 : 1.2) + fixed;
+        };
+        const double cost = (double)(per_cu / resident) * round(resident) + (per_cu % resident ? round((int)(per_cu % resident)) : 0);
+        if (best.cost == 0 || cost < best.cost) best = {split, cost};
     }
     return best;
 }
@@ -505,7 +506,7 @@ void launch(const SdpaParams& p, hipStream_t stream) {
 
 template <bool kBf16, int kDP, int kForm>
 void launch(const SdpaParams& p, hipStream_t stream) {
-    const int split = choose_split(p);
+    const int split = choose_split(p).split;
     if (split == 1)
         launch<kBf16, kDP, kForm, 1>(p, stream);
     else if (split == 2)
@@ -529,19 +530,34 @@ void launch(const SdpaParams& p, hipStream_t stream) {
 // 16-bit operands at 16-byte aligned addresses; no mask, or one whose keys lie side by side, boolean or of the operands' type.
 bool sdpa_narrow_supported(const SdpaParams& p) {
     if (p.dtype != HIPATTN_F16 && p.dtype != HIPATTN_BF16) return false;
-    if (p.head_dim != 64 && (p.head_dim < 72 || p.head_dim > 96 || p.head_dim % 8 != 0)) return false;
+    if (p.head_dim != 64 && (p.head_dim < 72 || p.head_dim > 128 || p.head_dim % 8 != 0)) return false;
     if (p.mask && (p.mask_stride[3] != 1 || (p.mask_dtype != HIPATTN_U8 && p.mask_dtype != p.dtype))) return false;
     const int64_t tiles = (int64_t)p.batch * p.num_heads_q * (((int64_t)p.len_q + 31) / 32);
     return p.len_q > 0 && p.len_kv > 0 && p.batch > 0 && tiles < (1 << 30) &&
            (((uintptr_t)p.q | (uintptr_t)p.k | (uintptr_t)p.v | (uintptr_t)p.out) & 15) == 0;
 }
 
+// Head sizes above 96 share with the kernel of flash_prefill.hip, whose workgroup has a compute unit to itself, takes 256 rows
+// and needs some 1.25 us for 64 keys, 1.5 with the chip full, and 4 to 5 besides: it is faster where it fills the chip (4 x 32 heads
+// of 2,048, causal: 141 against 152 us; 4 x 8 of 1,300: 35 against 42) and slower on small calls (8 heads of 2,048: 42 against 28;
+// 12 of 500, causal: 18.4 against 10.2; 8 of 48: 7.4 against 5.6) and with a mask (4 x 8 of 1,024: 50 against 38).  Below,
+// it computes 128 columns all the same, and this one is at least as fast (size 80, 2 x 16 heads of 1,500: 38.0 and 38.3;
+// size 96, 8 x 12 of 700: 42 against 33).
+bool sdpa_narrow_preferred(const SdpaParams& p) {
+    if (p.head_dim <= 96 || p.mask) return true;
+    const int G = p.num_heads_q / p.num_heads_kv, q_tiles = (p.len_q + 127) / 128;
+    const int64_t groups = (int64_t)p.batch * p.num_heads_kv * (G % 2 == 0 ? G / 2 * q_tiles : G * ((q_tiles + 1) / 2));
+    const int64_t rounds = (groups + 255) / 256;
+    const double tiles = (p.len_kv + 63) / 64;
+    return narrow::choose_split(p).cost < 0.9 * (double)rounds * (tiles * (groups > 128 ? 1.5 : 1.25) + (rounds > 1 ? 5.0 : 4.0));
+}
+
 hipError_t launch_sdpa_narrow(const SdpaParams& p, hipStream_t stream, const KernelProbe& probe) {
     if (probe.before) (void)hipEventRecord(probe.before, stream);
     if (p.dtype == HIPATTN_BF16)
-        p.head_dim == 64 ? narrow::launch<true, 64>(p, stream) : narrow::launch<true, 96>(p, stream);
+        p.head_dim == 64 ? narrow::launch<true, 64>(p, stream) : p.head_dim <= 96 ? narrow::launch<true, 96>(p, stream) : narrow::launch<true, 128>(p, stream);
     else
-        p.head_dim == 64 ? narrow::launch<false, 64>(p, stream) : narrow::launch<false, 96>(p, stream);
+        p.head_dim == 64 ? narrow::launch<false, 64>(p, stream) : p.head_dim <= 96 ? narrow::launch<false, 96>(p, stream) : narrow::launch<false, 128>(p, stream);
     const hipError_t e = hipGetLastError();
     if (probe.after) (void)hipEventRecord(probe.after, stream);
     return e;
