@@ -1,4 +1,5 @@
-// MatMul through hipBLASLt: a plain library GEMM with fp32 accumulation.  The operator's tensors
+// MatMul: up to 16 rows in a kernel of matmul_few_rows.hip, else through hipBLASLt: a plain library GEMM with fp32
+// accumulation.  The operator's tensors
 // are row-major; hipBLASLt is column-major, so the product is taken transposed
 // (C^T = op(B)^T * op(A)^T) with the operands swapped and no data movement.  Descriptors and the
 // algorithm are kept per (device, shape), so a repeated shape costs one hipblasLtMatmul call; the
@@ -115,6 +116,7 @@ hipattn_status matmul(const hipops_matmul_desc* d, const void* a, const void* b,
     if (workspace && ((uintptr_t)workspace % 256) != 0) return fail(HIPATTN_INVALID_ARGUMENT, "matmul: workspace must be 256-byte aligned");
     int device = 0;
     if (hipGetDevice(&device) != hipSuccess) return fail(HIPATTN_NO_DEVICE, "matmul: no current device");
+    if (matmul_few_rows_supported(d, a, b, c)) return matmul_few_rows(d, a, b, c, stream);
 
     DeviceState* dev_ptr = nullptr;
     {
