@@ -13,7 +13,7 @@
 // a step's own chain (LDS, products, exponentials, check) at two wavefronts per SIMD.
 // Measured against the head-128 kernel on padded rows: 16 x 16 heads of 577, size 64, fp16: 60 -> 33 us (660 TFLOP/s); 16 heads
 // of 4,096: 102 -> 78 (880); 8 heads of 2,048: 43 -> 19; 8 of 128: 8.6 -> 5.2; 4 x 32 of 2,048, causal: 122 -> 79; size 96,
-// 8 x 12 heads of 700: 42 -> 34; against the plain masked kernel: 4 x 12 heads of 1,100 with a bias: 135 -> 37, size 128,
+// 8 x 12 heads of 700: 42 -> 34; against the plain masked kernel: 4 x 12 heads of 1,100 with a bias: 135 -> 39, size 128,
 // 4 x 32 heads of 1,000, padded: 454 -> 79.
 #include "device_common.hpp"
 #include "kernels.hpp"
@@ -180,11 +180,13 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
         load_tile(v_src, v_off, v_chunk, v_keys, stage);
         v_src += tile_bytes, v_keys -= kTileK;
     };
-    if (tile0 < tiles) {
+    auto load_first = [&]() __attribute__((always_inline)) {
+        if (tile0 >= tiles) return;
         load_k(k_lds);
         load_v(v_lds);
         if (tile0 + 1 < tiles) load_k(k_lds + kStage);
-    }
+    };
+    load_first();
 
     vec8 qf[kSteps];  // Q^T: lane (n32, hi) holds row n32, columns 16 i + 8 hi .. + 7, times scale * log2(e)
     {
@@ -223,6 +225,11 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
         for (int r = 0; r < 16; r++) o[dt][r] = 0.f;
     float l_run = 0.f;       // this lane's half of the row's sum
     bool started = false;    // the row has met a key that it attends
+    // An additive mask says "not this key" by its type's lowest value as well as by -inf.  A reference down there (94,500 in
+    // fp16) would round the scores that are computed on it to 2^-7, so a row starts with a score above this floor; below it
+    // a key counts for nothing beside any other.  Rows that have no other keys are worked in a second pass without the floor.
+    float floor = kForm == kAdditive ? -4096.f : -INFINITY;
+    bool low = false;        // the row has met keys, all of them below the floor
 
     // exponents of the softmax of 32 keys: register r is key 8 (r / 4) + 4 hi + r % 4 of the half
     auto scores = [&](const lds_byte* stage, int half, float16_t& s) __attribute__((always_inline)) {
@@ -350,7 +357,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
             for (int r = 0; r < 16; r++) top = fmaxf(top, s[r]);
             const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(top), __float_as_uint(top), false, false);
             top = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
-            const bool seen = top != -INFINITY;
+            const bool seen = top > floor;
+            if constexpr (kForm == kAdditive) low = low || top != -INFINITY;
             if (__builtin_amdgcn_ballot_w64(top > 8.0f || (seen && !started)) != 0) {
                 const float delta = started ? fmaxf(top, 0.f) : (seen ? top : 0.f);
                 const float alpha = fast_exp2(-fmaxf(delta, 0.f));
@@ -369,11 +377,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
     };
 
     float16_t s0, s1;
-    lds_byte *k_now = k_lds, *k_next = k_lds + kStage, *k_fill = k_lds + 2 * kStage, *v_now = v_lds, *v_fill = v_lds + kStage;
+    lds_byte *k_now, *k_next, *k_fill, *v_now, *v_fill;
     const int t0 = kParts * tile0 + part;
-    if (t0 < steps) load_mask(t0);
-    wait_and_barrier();
-    scores(k_now, part, s0);
     // One tile: K of the next tile and V of this one, loaded an iteration ago, are there for every wavefront, and the
     // stages that are filled now were last read before the barrier
     auto iteration = [&](int j, float16_t& a, float16_t& b) __attribute__((always_inline)) {
@@ -391,15 +396,59 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
         k_now = k_next, k_next = k_fill, k_fill = k_done;
         v_now = v_fill, v_fill = v_done;
     };
-    if constexpr (kSplit == 1) {
-        for (int j = tile0; j < tiles; j++) iteration(j, s0, s1);
+    auto all_tiles = [&]() __attribute__((always_inline)) {
+        k_now = k_lds, k_next = k_lds + kStage, k_fill = k_lds + 2 * kStage, v_now = v_lds, v_fill = v_lds + kStage;
+        if (t0 < steps) load_mask(t0);
+        wait_and_barrier();
+        scores(k_now, part, s0);
+        if constexpr (kSplit == 1) {
+            for (int j = tile0; j < tiles; j++) iteration(j, s0, s1);
+        } else {
+            for (int j = tile0; j < tiles; j += 2) {
+                iteration(j, s0, s1);
+                if (j + 1 < tiles) iteration(j + 1, s1, s0);
+            }
+        }
+        accumulate();
+    };
+    if constexpr (kForm != kAdditive) {
+        all_tiles();
     } else {
-        for (int j = tile0; j < tiles; j += 2) {
-            iteration(j, s0, s1);
-            if (j + 1 < tiles) iteration(j + 1, s1, s0);
+        for (bool again = false;; again = true) {
+            all_tiles();
+            if (again) break;
+            // does any row of the workgroup need the second pass: one with keys, none of whose wavefronts has started it
+            typedef __attribute__((address_space(3))) uint8_t lds_flag;
+            lds_flag* const flags = (lds_flag*)v_lds;  // (the stages are read by none when the first barrier is passed)
+            __syncthreads();
+            flags[32 * wave + n32] = started ? 1 : 0;
+            __syncthreads();
+            int any = 0;
+#pragma unroll
+            for (int x = 0; x < kSplit; x++) any |= flags[32 * (wave - part + x) + n32];
+            const uint64_t need = __builtin_amdgcn_ballot_w64(low && any == 0 && my_row < p.len_q);
+            if (lane == 0) flags[32 * kWaves + wave] = need != 0 ? 1 : 0;
+            __syncthreads();
+            int vote = 0;
+#pragma unroll
+            for (int x = 0; x < kWaves; x++) vote |= flags[32 * kWaves + x];
+            if (__builtin_amdgcn_readfirstlane(vote) == 0) break;
+            __syncthreads();  // (the flags' place is loaded over)
+            if (low && any == 0) floor = -INFINITY;
+            started = low = false, l_run = 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; r++) neg_ref[r] = 0.f;
+#pragma unroll
+            for (int dt = 0; dt < kOut; dt++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) o[dt][r] = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) pf[ks] = __builtin_bit_cast(vec8, (uint4_t){0u, 0u, 0u, 0u});
+            k_src = k, v_src = v;
+            k_keys = v_keys = p.len_kv;
+            load_first();
         }
     }
-    accumulate();
 
     const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
     float l = __uint_as_float(both[0]) + __uint_as_float(both[1]);
@@ -540,11 +589,14 @@ bool sdpa_narrow_supported(const SdpaParams& p) {
 // Head sizes above 96 share with the kernel of flash_prefill.hip, whose workgroup has a compute unit to itself, takes 256 rows
 // and needs some 1.25 us for 64 keys, 1.5 with the chip full, and 4 to 5 besides: it is faster where it fills the chip (4 x 32 heads
 // of 2,048, causal: 141 against 152 us; 4 x 8 of 1,300: 35 against 42) and slower on small calls (8 heads of 2,048: 42 against 28;
-// 12 of 500, causal: 18.4 against 10.2; 8 of 48: 7.4 against 5.6) and with a mask (4 x 8 of 1,024: 50 against 38).  Below,
+// 12 of 500, causal: 18.4 against 10.2; 8 of 48: 7.4 against 5.6) and with a mask.  Below,
 // it computes 128 columns all the same, and this one is at least as fast (size 80, 2 x 16 heads of 1,500: 38.0 and 38.3;
 // size 96, 8 x 12 of 700: 42 against 33).
 bool sdpa_narrow_preferred(const SdpaParams& p) {
-    if (p.head_dim <= 96 || p.mask) return true;
+    if (p.head_dim <= 96) return true;
+    // (an additive mask's second pass leaves the 128-column build short of registers: 4 x 8 heads of 1,024 44 against 50 us, but
+    // 4 x 32 of 2,048, four rounds of workgroups, 445 against 375)
+    if (p.mask) return p.mask_dtype == HIPATTN_U8 || (int64_t)p.batch * p.num_heads_q * ((p.len_q + 127) / 128) <= 512;
     const int G = p.num_heads_q / p.num_heads_kv, q_tiles = (p.len_q + 127) / 128;
     const int64_t groups = (int64_t)p.batch * p.num_heads_kv * (G % 2 == 0 ? G / 2 * q_tiles : G * ((q_tiles + 1) / 2));
     const int64_t rounds = (groups + 255) / 256;

@@ -53,3 +53,31 @@ def test_growing_scores(hip, oracle, dtype):
     ref = oracle.sdpa(case["q"], case["k"], case["v"])
     assert np.isfinite(out).all()
     assert H.max_abs(out, ref) <= (0.05 if dtype == W.F16 else 0.4)
+
+
+@pytest.mark.parametrize("dtype", [W.F16, W.BF16])
+@pytest.mark.parametrize("shape", [(2, 4, 2, 70, 300, 64), (1, 2, 2, 33, 90, 96), (1, 24, 24, 640, 200, 64), (1, 2, 1, 140, 500, 128)])
+def test_masks_of_the_lowest_value(hip, oracle, dtype, shape):
+    """Keys masked by the type's lowest value (fp16: finite after the change of base), the first ones of every row, some rows as
+    a whole: the kept keys weigh as if the others were not there, and a row of none but such keys is their mean weighted by
+    scores that the mask has rounded away (bf16: -inf after the change of base, and zeros)."""
+    B, Hq, Hkv, Lq, Lk, D = shape
+    case = W.make_sdpa_case(23, B, Hq, Hkv, Lq, Lk, D, dtype)
+    lowest = -65504.0 if dtype == W.F16 else float(np.frombuffer(np.uint32(0xff7f0000).tobytes(), np.float32)[0])
+    m = np.zeros((1, 1, Lq, Lk), np.float32)
+    m[..., :75] = lowest
+    m[:, :, Lq // 2:Lq // 2 + 3] = lowest
+    gone = m == lowest
+    case["k"][:, :, :75] *= 0.0  # (equal scores: the mean of a row of such keys is exact whatever their rounding)
+    case["k"][..., 0] = 0
+    case["q"][:, :, Lq // 2:Lq // 2 + 3] = 0
+    for n in "qk":
+        case[n + "_store"], case[n] = W.to_storage(case[n], dtype)
+    out, _ = H.run_sdpa_masked(hip, case, m, mask_dtype=dtype)
+    ref = oracle.sdpa_masked(case["q"], case["k"], case["v"], np.where(gone, -np.inf, 0).astype(np.float32))
+    rows = slice(Lq // 2, Lq // 2 + 3)
+    if dtype == W.F16:
+        ref[:, :, rows] = np.repeat(case["v"].mean(2, keepdims=True), Hq // Hkv, axis=1)
+    else:
+        ref[:, :, rows] = 0
+    assert H.scaled_bound_error(out, ref, "lowest mask") <= (2e-3 if dtype == W.F16 else 1e-2)
