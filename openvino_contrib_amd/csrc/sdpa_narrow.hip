@@ -180,13 +180,11 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
         load_tile(v_src, v_off, v_chunk, v_keys, stage);
         v_src += tile_bytes, v_keys -= kTileK;
     };
-    auto load_first = [&]() __attribute__((always_inline)) {
-        if (tile0 >= tiles) return;
+    if (tile0 < tiles) {
         load_k(k_lds);
         load_v(v_lds);
         if (tile0 + 1 < tiles) load_k(k_lds + kStage);
-    };
-    load_first();
+    }
 
     vec8 qf[kSteps];  // Q^T: lane (n32, hi) holds row n32, columns 16 i + 8 hi .. + 7, times scale * log2(e)
     {
@@ -215,7 +213,13 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
 #pragma unroll
         for (int dt = 0; dt < kOut; dt++) v_at[dt] = row * kRow + 16 * v_place<kDP>(row, 4 * dt + 2 * (grp & 1) + ((i16 & 3) >> 1)) + 8 * (i16 & 1);
     }
-    float16_t neg_ref;
+    // The reference of a row's exponents, negated: where the accumulator of its scores starts or, with an additive mask, a
+    // part of what the mask adds: fma(mask, log2(e), -reference) is rounded once, so that a constant added to a whole row,
+    // which must not change it, costs its scores nothing.  Scores start from that sum or, at size 64, have it added to
+    // them (16 heads of 4,096: 138 us against 153; size 96, 2 x 16 of 2,048: 84.5 against 82.9; size 128: 40.0 against 33.0).
+    constexpr bool kMaskStarts = kForm == kAdditive && kDP != 64;
+    float16_t neg_ref;  // (zero with an additive mask)
+    float neg_ref_add = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; r++) neg_ref[r] = 0.f;
     float16_t o[kOut];
@@ -225,19 +229,15 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
         for (int r = 0; r < 16; r++) o[dt][r] = 0.f;
     float l_run = 0.f;       // this lane's half of the row's sum
     bool started = false;    // the row has met a key that it attends
-    // An additive mask says "not this key" by its type's lowest value as well as by -inf.  A reference down there (94,500 in
-    // fp16) would round the scores that are computed on it to 2^-7, so a row starts with a score above this floor; below it
-    // a key counts for nothing beside any other.  Rows that have no other keys are worked in a second pass without the floor.
-    float floor = kForm == kAdditive ? -4096.f : -INFINITY;
-    bool low = false;        // the row has met keys, all of them below the floor
 
-    // exponents of the softmax of 32 keys: register r is key 8 (r / 4) + 4 hi + r % 4 of the half
-    auto scores = [&](const lds_byte* stage, int half, float16_t& s) __attribute__((always_inline)) {
+    // exponents of the softmax of 32 keys, from `start` on: register r is key 8 (r / 4) + 4 hi + r % 4 of the half
+    auto scores = [&](const lds_byte* stage, int half, float16_t& s, const float16_t& start) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < kSteps; i++)
-            s = M::mma(__builtin_bit_cast(vec8, *(const lds_uint4*)(stage + k_at(i) + half * 32 * kRow)), qf[i], i == 0 ? neg_ref : s);
+            s = M::mma(__builtin_bit_cast(vec8, *(const lds_uint4*)(stage + k_at(i) + half * 32 * kRow)), qf[i], i == 0 ? start : s);
     };
-    // the mask of step t for this lane's row: words of four keys (8 g + 4 hi .. + 3)
+    // the mask of a step for this lane's row, of step t or, where scores start from it, of the one after it: words of four
+    // keys (8 g + 4 hi .. + 3)
     constexpr int kMaskWords = kForm == kAdditive ? 8 : kForm == kBoolean ? 4 : 1;
     uint32_t mask[kMaskWords];
     const uint8_t* mask_row = nullptr;
@@ -270,6 +270,15 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
             }
         }
     };
+    auto addend = [&](int r) __attribute__((always_inline)) -> float {
+        return fmaf(M::to_float((mask[r >> 1] >> (16 * (r & 1))) & 0xffffu), kLog2e, neg_ref_add);
+    };
+    auto start_scores = [&](float16_t& s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[r] = addend(r);
+    };
+    constexpr int kNext = kSplit == 1 ? 1 : kParts;  // from one step of a wavefront to its next
+    bool stale = false;  // (kMaskStarts) the reference has moved far from where the next step's scores were started
     vec8 pf[2], vf[2][kOut];  // probabilities of the step before and the V^T fragments that they meet
 #pragma unroll
     for (int ks = 0; ks < 2; ks++) {
@@ -284,25 +293,46 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
             for (int dt = 0; dt < kOut; dt++) o[dt] = M::mma(vf[ks][dt], pf[ks], o[dt]);
     };
     // One step: its exponentials, and beside them on the matrix core O^T += V^T P^T of the step before and the scores of the next.
-    auto step = [&](int t, float16_t& s, float16_t& s_next, const lds_byte* k_next, int half_next, const lds_byte* v_stage, int half)
+    auto step = [&](int t, float16_t& s, float16_t& s_next, const lds_byte* k_this, const lds_byte* k_next, int half_next, const lds_byte* v_stage, int half)
                     __attribute__((always_inline)) {
         if constexpr (kForm == kBoolean) {
 #pragma unroll
             for (int r = 0; r < 16; r++) s[r] = ((mask[r >> 2] >> (8 * (r & 3))) & 0xffu) != 0 ? s[r] : -INFINITY;
         }
-        if constexpr (kForm == kAdditive) {
+        if constexpr (kForm == kAdditive && !kMaskStarts) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) s[r] = fmaf(M::to_float((mask[r >> 1] >> (16 * (r & 1))) & 0xffffu), kLog2e, s[r]);
+            for (int r = 0; r < 16; r++) s[r] += addend(r);
         }
-        if constexpr (kForm != kNoMask) {
-            constexpr int kNext = kSplit == 1 ? 1 : kParts;  // from one step of a wavefront to its next
+        if constexpr (kForm != kNoMask && !kMaskStarts) {
             if (t + kNext < steps) load_mask(t + kNext);
         }
-        if (32 * t + 32 > p.len_kv || (p.causal && 32 * t + 31 > row0)) {
-            const int end = (p.causal ? min(p.len_kv, my_row + 1) : p.len_kv) - 32 * t - 4 * hi;
-#pragma unroll
-            for (int r = 0; r < 16; r++) s[r] = 8 * (r >> 2) + (r & 3) < end ? s[r] : -INFINITY;
+        auto scores_again = [&]() __attribute__((always_inline)) {
+            load_mask(t);
+            float16_t start;
+            start_scores(start);
+            scores(k_this, half, s, start);
+        };
+        if constexpr (kMaskStarts) {
+            if (stale) {
+                scores_again();
+                if (t + kNext < steps) load_mask(t + kNext);
+                stale = false;
+            }
         }
+        auto cut_edges = [&]() __attribute__((always_inline)) {
+            if (32 * t + 32 > p.len_kv || (p.causal && 32 * t + 31 > row0)) {
+                const int end = (p.causal ? min(p.len_kv, my_row + 1) : p.len_kv) - 32 * t - 4 * hi;
+#pragma unroll
+                for (int r = 0; r < 16; r++) s[r] = 8 * (r >> 2) + (r & 3) < end ? s[r] : -INFINITY;
+            }
+        };
+        cut_edges();
+        constexpr bool kStartEarly = kDP < 128;  // (size 128 has no registers for it until half of the step is done)
+        auto start_next = [&]() __attribute__((always_inline)) {  // (after the last step: unused)
+            start_scores(s_next);
+            if (t + 2 * kNext < steps) load_mask(t + 2 * kNext);
+        };
+        if constexpr (kMaskStarts && kStartEarly) start_next();
         vec8 pn[2];
         auto probabilities = [&](int ks) __attribute__((always_inline)) -> float {  // of sixteen keys; returns their sum
             float sum = 0.f;
@@ -329,6 +359,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
             __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kMaskStarts && !kStartEarly) start_next();
 #pragma unroll
         for (int ks = 0; ks < 2; ks++)
 #pragma unroll
@@ -341,7 +372,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
             }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < kSteps; i++) s_next = M::mma(kf[i], qf[i], i == 0 ? neg_ref : s_next);  // (after the last step: unused)
+        for (int i = 0; i < kSteps; i++) s_next = M::mma(kf[i], qf[i], i == 0 && !kMaskStarts ? neg_ref : s_next);  // (after the last step: unused)
         sum += probabilities(1);
 #pragma unroll
         for (int x = 0; x < kSteps; x++) {
@@ -352,23 +383,52 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
         // The reference stays while every sum says that no probability can have overflowed; otherwise, and for the first
         // keys of a row, it moves to the largest score (all in units of exponents to base 2).
         if (__builtin_amdgcn_ballot_w64(!started || !(sum < M::kSafeSum)) != 0) {
-            float top = -INFINITY;
+            // An additive mask says "not this key" by a large negative number as well as by -inf, and a reference taken from such keys
+            // leaves the scores of the others, 94,500 above it with fp16's lowest value, rounded to 2^-7.  So after a move by
+            // more than 2^9, which leaves nothing of what a row has summed up, its scores are computed again (to 2^-15) and its
+            // reference is chosen again, off by the rounding of the last one: 2^-24 of it, so that 10^38 takes six moves.
+            constexpr float kFar = 512.0f;
+            auto move = [&]() __attribute__((always_inline)) -> bool {
+                float top = -INFINITY;
 #pragma unroll
-            for (int r = 0; r < 16; r++) top = fmaxf(top, s[r]);
-            const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(top), __float_as_uint(top), false, false);
-            top = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
-            const bool seen = top > floor;
-            if constexpr (kForm == kAdditive) low = low || top != -INFINITY;
-            if (__builtin_amdgcn_ballot_w64(top > 8.0f || (seen && !started)) != 0) {
-                const float delta = started ? fmaxf(top, 0.f) : (seen ? top : 0.f);
+                for (int r = 0; r < 16; r++) top = fmaxf(top, s[r]);
+                const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(top), __float_as_uint(top), false, false);
+                top = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+                const bool seen = top != -INFINITY;
+                if (__builtin_amdgcn_ballot_w64(top > 8.0f || (seen && !started)) == 0) return false;
+                float delta = started ? fmaxf(top, 0.f) : (seen ? top : 0.f);
+                if constexpr (kForm == kAdditive) {  // by what the new reference is, rounded, as the next steps will see it
+                    const float moved = neg_ref_add - delta;
+                    delta = neg_ref_add - moved;
+                    neg_ref_add = moved;
+                }
                 const float alpha = fast_exp2(-fmaxf(delta, 0.f));
                 l_run *= alpha;
 #pragma unroll
                 for (int dt = 0; dt < kOut; dt++) o[dt] *= alpha;
                 s -= delta;
-                s_next -= delta;
-                neg_ref -= delta;
                 started = started || seen;
+                if constexpr (kForm != kAdditive || kMaskStarts) s_next -= delta;
+                if constexpr (kForm == kAdditive) {
+                    const bool far = fabsf(delta) > kFar;
+                    started = started && !far;
+                    return __builtin_amdgcn_ballot_w64(far) != 0;
+                } else {
+                    neg_ref -= delta;
+                    return false;
+                }
+            };
+            bool again = move();
+            if constexpr (kForm == kAdditive) {
+                const bool far = again;
+                for (int tries = 0; again && tries < 8; tries++) {
+                    scores_again();
+                    cut_edges();
+                    again = move();
+                }
+                constexpr int kLoaded = kMaskStarts ? 2 * kNext : kNext;  // which step's mask has been overwritten
+                if (far && t + kLoaded < steps) load_mask(t + kLoaded);
+                if constexpr (kMaskStarts) stale = far;
             }
             sum = probabilities(0) + probabilities(1);
         }
@@ -387,68 +447,32 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
         if (j + 1 < tiles) load_v(v_fill);
         const int t = kParts * j + part;
         if constexpr (kSplit == 1) {
-            if (t < steps) step(t, a, b, k_now, 1, v_now, 0);
-            if (t + 1 < steps) step(t + 1, b, a, k_next, 0, v_now, 1);
+            if (t < steps) step(t, a, b, k_now, k_now, 1, v_now, 0);
+            if (t + 1 < steps) step(t + 1, b, a, k_now, k_next, 0, v_now, 1);
         } else {
-            if (t < steps) step(t, a, b, k_next, part, v_now, part);
+            if (t < steps) step(t, a, b, k_now, k_next, part, v_now, part);
         }
         lds_byte *const k_done = k_now, *const v_done = v_now;
         k_now = k_next, k_next = k_fill, k_fill = k_done;
         v_now = v_fill, v_fill = v_done;
     };
-    auto all_tiles = [&]() __attribute__((always_inline)) {
-        k_now = k_lds, k_next = k_lds + kStage, k_fill = k_lds + 2 * kStage, v_now = v_lds, v_fill = v_lds + kStage;
-        if (t0 < steps) load_mask(t0);
-        wait_and_barrier();
-        scores(k_now, part, s0);
-        if constexpr (kSplit == 1) {
-            for (int j = tile0; j < tiles; j++) iteration(j, s0, s1);
-        } else {
-            for (int j = tile0; j < tiles; j += 2) {
-                iteration(j, s0, s1);
-                if (j + 1 < tiles) iteration(j + 1, s1, s0);
-            }
-        }
-        accumulate();
-    };
-    if constexpr (kForm != kAdditive) {
-        all_tiles();
+    k_now = k_lds, k_next = k_lds + kStage, k_fill = k_lds + 2 * kStage, v_now = v_lds, v_fill = v_lds + kStage;
+    if (t0 < steps) load_mask(t0);
+    if constexpr (kMaskStarts) {
+        start_scores(s0);
+        if (t0 + kNext < steps) load_mask(t0 + kNext);
+    }
+    wait_and_barrier();
+    scores(k_now, part, s0, kMaskStarts ? s0 : neg_ref);
+    if constexpr (kSplit == 1) {
+        for (int j = tile0; j < tiles; j++) iteration(j, s0, s1);
     } else {
-        for (bool again = false;; again = true) {
-            all_tiles();
-            if (again) break;
-            // does any row of the workgroup need the second pass: one with keys, none of whose wavefronts has started it
-            typedef __attribute__((address_space(3))) uint8_t lds_flag;
-            lds_flag* const flags = (lds_flag*)v_lds;  // (the stages are read by none when the first barrier is passed)
-            __syncthreads();
-            flags[32 * wave + n32] = started ? 1 : 0;
-            __syncthreads();
-            int any = 0;
-#pragma unroll
-            for (int x = 0; x < kSplit; x++) any |= flags[32 * (wave - part + x) + n32];
-            const uint64_t need = __builtin_amdgcn_ballot_w64(low && any == 0 && my_row < p.len_q);
-            if (lane == 0) flags[32 * kWaves + wave] = need != 0 ? 1 : 0;
-            __syncthreads();
-            int vote = 0;
-#pragma unroll
-            for (int x = 0; x < kWaves; x++) vote |= flags[32 * kWaves + x];
-            if (__builtin_amdgcn_readfirstlane(vote) == 0) break;
-            __syncthreads();  // (the flags' place is loaded over)
-            if (low && any == 0) floor = -INFINITY;
-            started = low = false, l_run = 0.f;
-#pragma unroll
-            for (int r = 0; r < 16; r++) neg_ref[r] = 0.f;
-#pragma unroll
-            for (int dt = 0; dt < kOut; dt++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) o[dt][r] = 0.f;
-#pragma unroll
-            for (int ks = 0; ks < 2; ks++) pf[ks] = __builtin_bit_cast(vec8, (uint4_t){0u, 0u, 0u, 0u});
-            k_src = k, v_src = v;
-            k_keys = v_keys = p.len_kv;
-            load_first();
+        for (int j = tile0; j < tiles; j += 2) {
+            iteration(j, s0, s1);
+            if (j + 1 < tiles) iteration(j + 1, s1, s0);
         }
     }
+    accumulate();
 
     const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
     float l = __uint_as_float(both[0]) + __uint_as_float(both[1]);
@@ -479,7 +503,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
         static_assert(kWaves * kShare * 4 <= 5 * kStage, "the shares take the place of the stages");
         __syncthreads();  // (every wavefront is done with the stages, and no load is under way)
         lds_float* const mine = shares + wave * kShare + lane;
-        mine[0] = started ? -neg_ref[0] : -INFINITY;
+        mine[0] = started ? -(kForm == kAdditive ? neg_ref_add : neg_ref[0]) : -INFINITY;
         mine[64] = l;
 #pragma unroll
         for (int dt = 0; dt < kOut; dt++)
@@ -594,8 +618,7 @@ bool sdpa_narrow_supported(const SdpaParams& p) {
 // size 96, 8 x 12 of 700: 42 against 33).
 bool sdpa_narrow_preferred(const SdpaParams& p) {
     if (p.head_dim <= 96) return true;
-    // (an additive mask's second pass leaves the 128-column build short of registers: 4 x 8 heads of 1,024 44 against 50 us, but
-    // 4 x 32 of 2,048, four rounds of workgroups, 445 against 375)
+    // (additive masks: 4 x 8 heads of 1,024 33 against 50 us; 4 x 32 of 2,048, four rounds of workgroups: 375 there)
     if (p.mask) return p.mask_dtype == HIPATTN_U8 || (int64_t)p.batch * p.num_heads_q * ((p.len_q + 127) / 128) <= 512;
     const int G = p.num_heads_q / p.num_heads_kv, q_tiles = (p.len_q + 127) / 128;
     const int64_t groups = (int64_t)p.batch * p.num_heads_kv * (G % 2 == 0 ? G / 2 * q_tiles : G * ((q_tiles + 1) / 2));

@@ -81,3 +81,40 @@ def test_masks_of_the_lowest_value(hip, oracle, dtype, shape):
     else:
         ref[:, :, rows] = 0
     assert H.scaled_bound_error(out, ref, "lowest mask") <= (2e-3 if dtype == W.F16 else 1e-2)
+
+
+def biased_rows(Lq, Lk, dtype):
+    """(mask, the same with a constant taken off every row), row after row another kind: a constant, one of two constants on
+    either half of the keys, very low keys before and behind a constant, a falling and a rising ramp."""
+    constants, mask = np.zeros((Lq, 1), np.float32), np.zeros((Lq, Lk), np.float32)
+    fp16 = dtype == W.F16
+    step = 2 if fp16 else 16  # (the type's spacing there)
+    near = [-2800 - step * i for i in range(27 if fp16 else 8)]
+    far = [-100.0, -700.0, 96.0, 3072.0, -12288.0] + ([-65504.0, 61440.0] if fp16 else [-131072.0, 2.0 ** 40])
+    lowest = -65504.0 if fp16 else -(2.0 ** 100)
+    half = np.arange(Lk) < Lk // 2
+    kinds = [(c, 0.0 * half) for c in near + far]
+    kinds += [(c, np.where(half if flip else ~half, -float(step), 0.0)) for c in near for flip in (False, True)]
+    kinds += [(c, np.where(half if flip else ~half, -np.inf, 0.0)) for c in near + far[:4] for flip in (False, True)]
+    ramp = np.arange(Lk) * -float(step)
+    kinds += [(c, r) for c in near + far[:2] for r in (ramp, ramp[::-1])]
+    for i in range(Lq):
+        c, d = kinds[(i * 7) % len(kinds)]
+        constants[i], mask[i] = c, np.where(np.isneginf(d), lowest, c + d)
+    mask = W.to_storage(mask, dtype)[1]
+    return mask, mask - constants
+
+
+# (in the order of the wavefronts that share 32 query rows: one, two, four)
+@pytest.mark.parametrize("dtype", [W.F16, W.BF16])
+@pytest.mark.parametrize("shape", [(4, 64, 8, 130, 400, 64), (2, 64, 8, 130, 400, 96), (2, 64, 8, 130, 250, 128), (2, 24, 24, 300, 300, 64), (2, 24, 6, 300, 300, 96),
+                                   (2, 16, 16, 300, 300, 128), (1, 4, 2, 130, 1000, 64), (1, 16, 16, 300, 300, 96), (1, 8, 8, 300, 300, 104)])
+def test_a_constant_added_to_a_row_changes_nothing(hip, oracle, dtype, shape):
+    """The softmax is the same whatever is added to all scores of a row.  The constants are values of the type, so that the
+    oracle's mask without them is exact, and what the kernel takes off mask * log2(e) is the same for all keys of the row."""
+    B, Hq, Hkv, Lq, Lk, D = shape
+    case = W.make_sdpa_case(24, B, Hq, Hkv, Lq, Lk, D, dtype)
+    m, shifted = biased_rows(Lq, Lk, dtype)
+    out, _ = H.run_sdpa_masked(hip, case, m, mask_dtype=dtype)
+    ref = oracle.sdpa_masked(case["q"], case["k"], case["v"], shifted)
+    assert H.scaled_bound_error(out, ref, "row constants") <= (2e-3 if dtype == W.F16 else 1e-2)
