@@ -180,7 +180,9 @@ __global__ __launch_bounds__(512) void sdpa_f32_kernel(SdpaParams p, int q_tiles
                     gap |= ((w - 0x01010101u) & ~w & 0x80808080u) != 0;  // (one of the four bytes is zero)
                 } else {
                     const float4_t x = __builtin_bit_cast(float4_t, now[nt]);
-                    any |= fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])) > -INFINITY;
+                    // (a NaN masks nothing: it becomes the row's, so not fmaxf, which would pass over it)
+                    const auto larger = [](float a, float b) { return __builtin_elementwise_maximum(a, b); };
+                    any |= larger(larger(x[0], x[1]), larger(x[2], x[3])) != -INFINITY;
                 }
             }
             attended = __builtin_amdgcn_ballot_w64(any) != 0;

@@ -71,3 +71,25 @@ def test_large_values_beside_growing_scores(hip, oracle):
     ref = oracle.sdpa(case["q"], case["k"], (case["v"] / np.float32(2e37)))
     assert np.isfinite(out).all()
     assert H.max_abs(out / np.float32(2e37), ref) <= 1e-4
+
+
+@pytest.mark.parametrize("mask_dtype", [W.F32, W.F16])
+@pytest.mark.parametrize("shape", [(1, 2, 1, 33, 64, 64), (2, 2, 2, 20, 200, 128), (1, 4, 4, 160, 47, 32)])
+def test_nan_masks_reach_their_rows(hip, oracle, shape, mask_dtype):
+    """Sixteen keys whose mask is NaN for every row of a tile, beside -inf and beside finite values: the rows are NaN, as
+    rows with one such key are; the rows of a tile without any are what they are."""
+    B, Hq, Hkv, Lq, Lk, D = shape
+    case = W.make_sdpa_case(11, B, Hq, Hkv, Lq, Lk, D, W.F32)
+    m = np.zeros((1, 1, Lq, Lk), np.float32)
+    m[..., 16:32] = np.nan
+    m[..., 32:] = -np.inf
+    out, _ = H.run_sdpa_masked(hip, case, m, mask_dtype=mask_dtype)
+    assert np.isnan(out).all()
+    m[..., 16:32] = -np.inf
+    m[:, :, 3, 18] = np.nan
+    out, _ = H.run_sdpa_masked(hip, case, m, mask_dtype=mask_dtype)
+    assert np.isnan(out[:, :, 3]).all()
+    m[:, :, 3, 18] = -np.inf
+    ref = oracle.sdpa_masked(case["q"], case["k"], case["v"], m)
+    rest = np.arange(Lq) != 3
+    assert H.max_abs(out[:, :, rest], ref[:, :, rest]) <= 1e-4
