@@ -146,12 +146,13 @@ hipattn_status hipattn_sdpa(const hipattn_sdpa_desc* desc, const void* q, const 
  * scaled score; dtype U8: boolean, nonzero = the key takes part, zero = probability zero.  As the
  * operator specifies, the mask is ignored when desc->causal is set.  A query row whose keys are
  * all masked out yields zeros.  mask_desc and mask are both NULL or both set.
- * At head_dim 128 (and at the multiples of 8 below it) a mask of the operands' 16-bit type, or a boolean one, whose keys lie side by
- * side (stride[3] == 1) rides along in the tuned matrix-core kernel when the mask pointer and the
- * other strides are multiples of 16 bytes (8 elements; 16 for boolean); every other mask beside
- * 16-bit operands with a head_dim that is a multiple of 8 up to 256 takes the plain matrix-core
- * kernel; fp32 operands with a head_dim that is a multiple of 4 up to 128 take the fp32 matrix-core kernel, any
- * mask; larger heads take the shape-generic kernel. */
+ * Beside 16-bit operands with a head_dim of 64 or a multiple of 8 from 72 to 128, a boolean mask, or one of the operands'
+ * type, whose keys lie side by side (stride[3] == 1) rides along in the matrix-core kernel of small workgroups
+ * wherever its rows start (operands at multiples of 16 bytes).  Additive masks of large calls at head_dim 104 to 128, and both kinds at
+ * the smaller multiples of 8, ride along in the tuned head-128 kernel when the mask pointer and the other strides are multiples of
+ * 16 bytes (8 elements; 16 for boolean).  Every other mask beside 16-bit operands with a head_dim that is a multiple of 8 up
+ * to 256 takes the plain matrix-core kernel; fp32 operands with a head_dim that is a multiple of 4 up to 128 take the
+ * fp32 matrix-core kernel, any mask; the rest takes the shape-generic kernel. */
 typedef struct hipattn_mask_desc {
     hipattn_dtype dtype;
     int64_t stride[4];
@@ -345,15 +346,24 @@ hipattn_status hipattn_profile_dominant_kernel(hipattn_event before, hipattn_eve
  *   "decode_fused_merge"          where pieces of several wavefronts make up one (sequence, kv head): 1 (default):
  *                                 the u8 decode kernels combine them themselves (no merge launch); 0: a merge
  *                                 launch behind every decode kernel (what 16-bit caches always get)
- *   "sdpa_padded_rows"            1 (default): dense SDPA at head sizes below 128 (multiples of 8) runs the
- *                                 tuned head-128 kernel on rows of fewer columns; 0: the plain kernels
+ *   "sdpa_padded_rows"            1 (default): dense SDPA at head sizes below 128 (multiples of 8) runs the kernel of
+ *                                 small workgroups (64, 72 and up) or the tuned head-128 kernel on rows of fewer
+ *                                 columns; 0: the plain kernels
+ *   "sdpa_narrow"                 dense SDPA in the kernel of small workgroups: 1 (default): where it is the faster one;
+ *                                 0: never; 2: wherever it takes the call
+ *   "sdpa_narrow_split"           wavefronts of that kernel that share 32 query rows: 1, 2 or 4; 0 (default): by the
+ *                                 time they would take
  * HIPATTN_<NAME IN CAPITALS> in the environment gives an option its initial value; the
  * environment is read once per process. */
 hipattn_status hipattn_set_option(const char* name, int value);
 
 /* Name of the kernel path the last attention call on this thread dispatched to
- * ("flash_mfma", "generic", "decode_mfma+merge", ...).  Diagnostic only. */
+ * ("sdpa_flash_mfma", "sdpa_generic", "paged_mfma", ...): the family, in which several kernels may share a name.  Diagnostic only. */
 const char* hipattn_last_kernel_path(void);
+
+/* The kernel that the last dense SDPA call on this thread ran: "sdpa_narrow" (small workgroups), "sdpa_flash" (the tuned
+ * head-128 kernel), "sdpa_flash_small" (the plain matrix-core kernels), "sdpa_f32" or "sdpa_generic".  Diagnostic only. */
+const char* hipattn_last_sdpa_kernel(void);
 
 #ifdef __cplusplus
 }

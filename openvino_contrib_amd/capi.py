@@ -129,6 +129,7 @@ SYMBOLS = {
     "hipattn_rotate_key_cache": (_i, [_P(PaDesc), _vp, _vp, _i, _vp, _i, _vp, _i, _i, _vp]),
     "hipattn_cache_row_bytes": (_sz, [_i, _i]),
     "hipattn_last_kernel_path": (ctypes.c_char_p, []),
+    "hipattn_last_sdpa_kernel": (ctypes.c_char_p, []),
     "hipattn_profile_dominant_kernel": (_i, [_vp, _vp]),
 }
 
@@ -173,6 +174,10 @@ def device_info(device=0):
 
 def last_kernel_path():
     return lib().hipattn_last_kernel_path().decode()
+
+
+def last_sdpa_kernel():
+    return lib().hipattn_last_sdpa_kernel().decode()
 
 
 class Stream:

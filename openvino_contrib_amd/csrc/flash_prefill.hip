@@ -1389,7 +1389,6 @@ bool sdpa_flash_mask_supported(const SdpaParams& p) {
 
 hipError_t launch_sdpa_flash(const SdpaParams& p, hipStream_t stream, const KernelProbe& probe) {
     if (p.batch == 0 || p.len_q == 0) return hipSuccess;
-    if (sdpa_narrow_supported(p) && sdpa_narrow_preferred(p)) return launch_sdpa_narrow(p, stream, probe);
     const int G = p.num_heads_q / p.num_heads_kv;
     const int n_qt = (p.len_q + flash::kTileQ - 1) / flash::kTileQ;
     const bool pair_heads = (G & 1) == 0;

@@ -711,7 +711,6 @@ static void launch_sdpa_small(const SdpaParams& p, unsigned groups, hipStream_t 
 }
 
 hipError_t launch_sdpa_flash_small(const SdpaParams& p, hipStream_t stream, const KernelProbe& probe) {
-    if (sdpa_padded_rows_enabled() && sdpa_narrow_supported(p)) return launch_sdpa_narrow(p, stream, probe);  // (masks whose rows are not aligned)
     const int64_t q_tiles = (p.len_q + flash_small::kTileQ - 1) / flash_small::kTileQ;
     const int64_t groups = q_tiles * p.num_heads_q * p.batch;
     if (groups == 0) return hipSuccess;

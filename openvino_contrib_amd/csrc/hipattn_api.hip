@@ -18,6 +18,7 @@ namespace {
 
 thread_local char g_error[512] = "";
 thread_local const char* g_kernel_path = "none";
+thread_local const char* g_sdpa_kernel = "none";
 thread_local hipattn::KernelProbe g_probe;
 
 hipattn_status fail(hipattn_status st, const char* fmt, ...) {
@@ -155,6 +156,7 @@ HIPATTN_EXPORT const char* hipattn_status_string(hipattn_status status) {
 HIPATTN_EXPORT int hipattn_version(void) { return HIPATTN_VERSION_MAJOR * 1000 + HIPATTN_VERSION_MINOR; }
 
 HIPATTN_EXPORT const char* hipattn_last_kernel_path(void) { return g_kernel_path; }
+HIPATTN_EXPORT const char* hipattn_last_sdpa_kernel(void) { return g_sdpa_kernel; }
 
 HIPATTN_EXPORT hipattn_status hipattn_profile_dominant_kernel(hipattn_event before, hipattn_event after) {
     if ((before == nullptr) != (after == nullptr))
@@ -409,18 +411,31 @@ HIPATTN_EXPORT hipattn_status hipattn_sdpa_masked(const hipattn_sdpa_desc* desc,
         p.mask_dtype = mask_desc->dtype;
         for (int i = 0; i < 4; i++) p.mask_stride[i] = mask_desc->stride[i];
     }
-    if (hipattn::sdpa_flash_supported(p) && (!p.mask || hipattn::sdpa_flash_mask_supported(p))) {
-        g_kernel_path = p.mask ? "sdpa_flash_mfma_masked" : "sdpa_flash_mfma";
-        HIP_TRY(hipattn::launch_sdpa_flash(p, as_stream(stream), g_probe));
-    } else if (hipattn::sdpa_flash_small_supported(p)) {
-        g_kernel_path = p.head_dim == 64 ? "sdpa_flash_mfma_d64" : "sdpa_flash_mfma_small";
-        HIP_TRY(hipattn::launch_sdpa_flash_small(p, as_stream(stream), g_probe));
-    } else {
-        g_kernel_path = "sdpa_generic";  // (the name of both kernels that take fp32 operands)
-        if (hipattn::sdpa_f32_supported(p))
-            HIP_TRY(hipattn::launch_sdpa_f32(p, as_stream(stream)));
+    const bool flash = hipattn::sdpa_flash_supported(p) && (!p.mask || hipattn::sdpa_flash_mask_supported(p));
+    if (flash || hipattn::sdpa_flash_small_supported(p)) {
+        if (flash)
+            g_kernel_path = p.mask ? "sdpa_flash_mfma_masked" : "sdpa_flash_mfma";
         else
+            g_kernel_path = p.head_dim == 64 ? "sdpa_flash_mfma_d64" : "sdpa_flash_mfma_small";
+        if (hipattn::sdpa_takes_narrow(p, flash)) {
+            g_sdpa_kernel = "sdpa_narrow";
+            HIP_TRY(hipattn::launch_sdpa_narrow(p, as_stream(stream), g_probe));
+        } else if (flash) {
+            g_sdpa_kernel = "sdpa_flash";
+            HIP_TRY(hipattn::launch_sdpa_flash(p, as_stream(stream), g_probe));
+        } else {
+            g_sdpa_kernel = "sdpa_flash_small";
+            HIP_TRY(hipattn::launch_sdpa_flash_small(p, as_stream(stream), g_probe));
+        }
+    } else {
+        g_kernel_path = "sdpa_generic";
+        if (hipattn::sdpa_f32_supported(p)) {
+            g_sdpa_kernel = "sdpa_f32";
+            HIP_TRY(hipattn::launch_sdpa_f32(p, as_stream(stream)));
+        } else {
+            g_sdpa_kernel = "sdpa_generic";
             HIP_TRY(hipattn::launch_sdpa_generic(p, as_stream(stream)));
+        }
     }
     return HIPATTN_OK;
 }

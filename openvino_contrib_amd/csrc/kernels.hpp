@@ -172,10 +172,9 @@ hipError_t launch_sdpa_f32(const SdpaParams& p, hipStream_t stream);
 bool sdpa_flash_supported(const SdpaParams& p);
 bool sdpa_flash_mask_supported(const SdpaParams& p);  // p.mask can ride along in the flash kernel
 hipError_t launch_sdpa_flash(const SdpaParams& p, hipStream_t stream, const KernelProbe& probe);
-// 16-bit operands at head sizes 64 and 72 .. 128, masks with keys side by side (sdpa_narrow.hip); preferred: to the kernel
-// of flash_prefill.hip where that takes the call too
-bool sdpa_narrow_supported(const SdpaParams& p);
-bool sdpa_narrow_preferred(const SdpaParams& p);
+// 16-bit operands at head sizes 64 and 72 .. 128, masks with keys side by side (sdpa_narrow.hip).  flash: the kernel of
+// flash_prefill.hip takes the call too (otherwise those of flash_small.hip do)
+bool sdpa_takes_narrow(const SdpaParams& p, bool flash);
 hipError_t launch_sdpa_narrow(const SdpaParams& p, hipStream_t stream, const KernelProbe& probe);
 
 // head sizes up to 256 that are multiples of 8 on the matrix cores (flash_small.hip)
@@ -243,6 +242,8 @@ size_t paged_scores_workspace(int q_dtype, int cache_dtype, int head_dim, int bl
 // Schedule option by name (see paged_decode.hip); value < 0 restores the default.  false: no such option.
 bool set_option(const char* name, int value);
 bool sdpa_padded_rows_enabled();  // the option sdpa_padded_rows
+int sdpa_narrow_option();        // 0 never, 1 where it is the faster kernel, 2 wherever it takes the call
+int sdpa_narrow_split_option();  // wavefronts that share query rows: 1, 2, 4, or 0 for choose_split's choice
 // Address and size of the current device's copy of the static scratch array (resolved once per device).
 hipError_t paged_static_scratch(void** ptr, size_t* bytes);
 

@@ -1790,8 +1790,12 @@ Option g_options[] = {
     // 1: the decode kernels that have the code for it (u8 caches) combine the partials of split segments
     // themselves; 0: a merge launch behind every decode kernel
     {"decode_fused_merge", "HIPATTN_DECODE_FUSED_MERGE", 1, 0, 1, {1}},
+    // dense SDPA in the kernel of sdpa_narrow.hip: 0 never, 1 where it is the faster one, 2 wherever it takes the call
+    {"sdpa_narrow", "HIPATTN_SDPA_NARROW", 1, 0, 2, {1}},
+    // wavefronts of that kernel that share 32 query rows: 1, 2 or 4; 0: by the time they would take
+    {"sdpa_narrow_split", "HIPATTN_SDPA_NARROW_SPLIT", 0, 0, 4, {0}},
 };
-enum { kOptMixedOverlap = 0, kOptSwitchCost, kOptDynPieces, kOptSharePercent, kOptSdpaPadded, kOptFusedMerge };
+enum { kOptMixedOverlap = 0, kOptSwitchCost, kOptDynPieces, kOptSharePercent, kOptSdpaPadded, kOptFusedMerge, kOptSdpaNarrow, kOptSdpaNarrowSplit };
 
 void init_options_from_environment() {
     static std::once_flag once;
@@ -1807,6 +1811,8 @@ int option(int which) {
 }  // namespace
 
 bool sdpa_padded_rows_enabled() { return option(kOptSdpaPadded) != 0; }
+int sdpa_narrow_option() { return option(kOptSdpaNarrow); }
+int sdpa_narrow_split_option() { return option(kOptSdpaNarrowSplit); }
 
 bool set_option(const char* name, int value) {
     init_options_from_environment();

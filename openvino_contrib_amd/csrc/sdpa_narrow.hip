@@ -579,10 +579,10 @@ void launch(const SdpaParams& p, hipStream_t stream) {
 
 template <bool kBf16, int kDP, int kForm>
 void launch(const SdpaParams& p, hipStream_t stream) {
-    const int split = choose_split(p).split;
+    const int wanted = sdpa_narrow_split_option(), split = wanted > 0 ? wanted : choose_split(p).split;
     if (split == 1)
         launch<kBf16, kDP, kForm, 1>(p, stream);
-    else if (split == 2)
+    else if (split < 4)
         launch<kBf16, kDP, kForm, 2>(p, stream);
     else
         launch<kBf16, kDP, kForm, 4>(p, stream);
@@ -601,7 +601,7 @@ void launch(const SdpaParams& p, hipStream_t stream) {
 }  // namespace narrow
 
 // 16-bit operands at 16-byte aligned addresses; no mask, or one whose keys lie side by side, boolean or of the operands' type.
-bool sdpa_narrow_supported(const SdpaParams& p) {
+static bool sdpa_narrow_supported(const SdpaParams& p) {
     if (p.dtype != HIPATTN_F16 && p.dtype != HIPATTN_BF16) return false;
     if (p.head_dim != 64 && (p.head_dim < 72 || p.head_dim > 128 || p.head_dim % 8 != 0)) return false;
     if (p.mask && (p.mask_stride[3] != 1 || (p.mask_dtype != HIPATTN_U8 && p.mask_dtype != p.dtype))) return false;
@@ -616,7 +616,7 @@ bool sdpa_narrow_supported(const SdpaParams& p) {
 // 12 of 500, causal: 18.4 against 10.2; 8 of 48: 7.4 against 5.6) and with a mask.  Below,
 // it computes 128 columns all the same, and this one is at least as fast (size 80, 2 x 16 heads of 1,500: 38.0 and 38.3;
 // size 96, 8 x 12 of 700: 42 against 33).
-bool sdpa_narrow_preferred(const SdpaParams& p) {
+static bool sdpa_narrow_preferred(const SdpaParams& p) {
     if (p.head_dim <= 96) return true;
     // (additive masks: 4 x 8 heads of 1,024 33 against 50 us; 4 x 32 of 2,048, four rounds of workgroups: 375 there)
     if (p.mask) return p.mask_dtype == HIPATTN_U8 || (int64_t)p.batch * p.num_heads_q * ((p.len_q + 127) / 128) <= 512;
@@ -625,6 +625,13 @@ bool sdpa_narrow_preferred(const SdpaParams& p) {
     const int64_t rounds = (groups + 255) / 256;
     const double tiles = (p.len_kv + 63) / 64;
     return narrow::choose_split(p).cost < 0.9 * (double)rounds * (tiles * (groups > 128 ? 1.5 : 1.25) + (rounds > 1 ? 5.0 : 4.0));
+}
+
+// (sdpa_padded_rows = 0 leaves head sizes below 128 to the plain kernels)
+bool sdpa_takes_narrow(const SdpaParams& p, bool flash) {
+    const int option = sdpa_narrow_option();
+    if (option == 0 || !sdpa_narrow_supported(p)) return false;
+    return option == 2 || (flash ? sdpa_narrow_preferred(p) : sdpa_padded_rows_enabled());
 }
 
 hipError_t launch_sdpa_narrow(const SdpaParams& p, hipStream_t stream, const KernelProbe& probe) {
