@@ -93,3 +93,19 @@ def test_nan_masks_reach_their_rows(hip, oracle, shape, mask_dtype):
     ref = oracle.sdpa_masked(case["q"], case["k"], case["v"], m)
     rest = np.arange(Lq) != 3
     assert H.max_abs(out[:, :, rest], ref[:, :, rest]) <= 1e-4
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_an_infinite_value_stays_in_its_column(hip, oracle, shape, masked):
+    """Every row attends a key with one infinite value: its column is infinite, the others are what they are.  Such rows are
+    worked again by all wavefronts of a workgroup, one row after the other."""
+    B, Hq, Hkv, Lq, Lk, D = shape
+    case = W.make_sdpa_case(12, B, Hq, Hkv, Lq, Lk, D, W.F32)
+    m = np.zeros((1, 1, Lq, Lk), np.float32)
+    m[..., Lk // 2 + 1:] = -np.inf
+    ref = oracle.sdpa_masked(case["q"], case["k"], case["v"], m) if masked else oracle.sdpa(case["q"], case["k"], case["v"])
+    case["v"][:, :, Lk // 2, D - 1] = np.inf
+    out, _ = H.run_sdpa_masked(hip, case, m) if masked else H.run_sdpa(hip, case, False)
+    assert np.isposinf(out[..., D - 1]).all()
+    assert H.max_abs(out[..., :D - 1], ref[..., :D - 1]) <= 1e-4
