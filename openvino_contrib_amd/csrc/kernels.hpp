@@ -121,7 +121,7 @@ struct PagedParams {
     // decode: the batch's block-heads are cut into num_waves equal pieces (one per wavefront);
     // pieces that do not cover a whole (sequence, kv head) segment leave partials in the workspace
     int num_waves;        // wavefronts (= single-wavefront workgroups) of the decode kernel
-    int min_units;        // shortest piece worth a wavefront (working_waves in paged_decode.hip); 0: as many pieces as wavefronts
+    int few_waves;        // wavefronts that are never too many (working_waves in paged_decode.hip); 0: as many pieces as wavefronts
     int switch_cost;      // block-times a wavefront is charged for starting on a new segment
     int dyn_pieces;       // pieces of the last quarter of the work line, handed out on demand
     int dyn_groups;       // wavefront groups, each with its own ticket counter and every dyn_groups-th piece

@@ -624,19 +624,20 @@ struct Line {
     }
 };
 
-// Wavefronts of `waves` that get a piece of a line of `total` units (p.min_units == 0: all of them, as the caller
-// fixed their number).  A small batch on all of them is bound by combining what they leave: every piece of a segment
-// is one more partial for the merge.  So pieces are kUnitsPerPiece units or more, except that half of the ordinary
-// count of wavefronts and two per segment are never too many, and none is empty; beyond one per compute unit only
-// whole numbers of them per compute unit (17 % more time with 1,088 than with 1,024).  One sequence of 778 tokens: 14.6 us
-// with 1,024 wavefronts, 11.2 with the 240 this gives it (12.9 with 64); of 16,384 tokens: 25.7 / 22.8 / 27.4 with
-// 1,024 / 512 / 256; 4 sequences of 256 to 4,096: 15.6 / 15.3 / 17.4; 100 sequences of 60 (800 segments): 18.9 / 22.9 with 1,024 / 512.
-constexpr int kUnitsPerPiece = 8, kFewWaves = 512;
-__device__ __forceinline__ int working_waves(const PagedParams& p, int64_t total, int waves) {
-    if (p.min_units == 0) return waves;
-    const int64_t few = max(kFewWaves, 2 * p.num_rows * p.num_heads_kv);
-    const int n = (int)min((int64_t)waves, min(total, max(few, total / p.min_units)));
-    return n > 256 ? n & ~255 : n;
+// Wavefronts of `waves` that get a piece of a line of `total` units (p.few_waves == 0: all of them).  A small batch on all of
+// them is bound by combining what they leave: every piece of a segment is one more partial for the merge.  So pieces
+// are eight units or more, except that half of the ordinary count of wavefronts and two per segment are never too many
+// (p.few_waves), and none is empty; beyond one per compute unit only whole numbers of them per compute unit (17 % more
+// time with 1,088 than with 1,024).  One sequence of 778 tokens: 13.7 us with 1,024 wavefronts, 11.7 with the 240 this gives
+// it (64: 12.9); of 4,000: 14.3 / 13.1 with 1,024 / 512; u8, 16 sequences of 300 (128 segments): 22.5 / 17.1 with 1,536 / 512.
+__host__ __device__ __forceinline__ int working_waves(const PagedParams& p, int64_t total, int waves) {
+    if (p.few_waves == 0) return waves;
+    const int eighth = total >= 8 * (int64_t)waves ? waves : (int)(total >> 3);  // (no division: it took 0.3 us of both kernels)
+    int n = eighth > p.few_waves ? eighth : p.few_waves;
+    if (n > 256) n = (n + 128) & ~255;
+    if (n > waves) n = waves;
+    if (n > total) n = total > 256 ? (int)total & ~255 : (int)total;
+    return n;
 }
 
 // eight consecutive output elements, one 16-byte store for the 16-bit types
@@ -698,7 +699,7 @@ __device__ __forceinline__ void merge_segment_head(const PagedParams& p, const L
                 float2 v[8];
                 float fi[8];
 #pragma unroll
-                for (int u = 0; u < 8; u++) {  // (a piece that does not exist: piece 0's row with weight zero)
+                for (int u = 0; u < 8; u++) {  // (a piece that does not exist: zeros with weight zero)
                     const int i = i0 + u * kParts;
                     const bool ok = i < n && ((alive >> i) & 1) != 0;
                     fi[u] = ok ? __shfl(f, i, 64) : 0.0f;
@@ -1755,11 +1756,22 @@ __global__ __launch_bounds__(kParts == 1 ? 256 : 64 * kParts) void paged_merge_k
     }
 }
 
+// The most 32-token blocks of a row, and pieces of one segment, that the caller's bound on the contexts allows.
+static int64_t most_blocks(const PagedParams& p) {
+    int64_t tokens = p.max_context_len > 0 ? p.max_context_len : 0x7fffffff;
+    if (p.sliding_window > 0) tokens = std::min(tokens, (int64_t)p.sliding_window + 31);
+    return (tokens + 31) / 32;
+}
+static int64_t most_waves(const PagedParams& p) {
+    return working_waves(p, (int64_t)p.num_rows * p.num_heads_kv * (most_blocks(p) + p.switch_cost), p.num_waves);
+}
+
 static hipError_t launch_merge(const PagedParams& p, hipStream_t stream) {
     const int segments = p.num_rows * p.num_heads_kv, G = p.num_heads_q / p.num_heads_kv;
     // (few segments of many pieces: 16,384 tokens of one sequence, 64 pieces a segment: the step 23.8 us with four wavefronts
-    // to a query head, 23.0 with eight; one wavefront taking piece after piece, as this kernel did: 14.6 us for the merge of 25)
-    if (segments <= 128)
+    // to a query head, 23.0 with eight; one wavefront taking piece after piece, as this kernel did: 14.6 us for the merge of 25.
+    // Up to eight pieces one wavefront has under way at once: 16 sequences of 100 tokens 13.5 us with eight of them to a head, 12.8 with one)
+    if (segments <= 128 && std::min(most_blocks(p), most_waves(p) / segments + 2) > 8)
         hipLaunchKernelGGL(paged_merge_kernel<8>, dim3(segments * G), dim3(512), 0, stream, p);
     else
         hipLaunchKernelGGL(paged_merge_kernel<1>, dim3(segments), dim3(256), 0, stream, p);
@@ -1966,7 +1978,6 @@ void paged_fast_plan(PagedParams& p, void* workspace) {
     const bool overlap = overlap_wanted(p);  // asks whether the caller fixed num_waves: before it is filled in
     p.overlap = overlap ? 1 : 0;
     const bool fixed_waves = p.num_waves > 0;
-    p.min_units = fixed_waves || option(kOptDynPieces) > 0 || overlap ? 0 : kUnitsPerPiece;  // (on-demand pieces: every ticket group needs its wavefronts)
     p.num_waves = choose_num_waves(p, overlap);
     p.switch_cost = option(kOptSwitchCost);
     p.dyn_pieces = choose_dyn_pieces(p, p.num_waves, overlap);
@@ -1975,6 +1986,11 @@ void paged_fast_plan(PagedParams& p, void* workspace) {
     const int G = p.num_heads_q / p.num_heads_kv;
     p.max_q_tiles = query_tile_bound(p);
     p.num_rows = plan_rows(p);
+    const int64_t segments = (int64_t)p.num_rows * p.num_heads_kv;
+    // 16-bit caches: from 128 segments on all wavefronts (24 sequences of 400: 16.1 us against 17.4 with 512; 63 of 300, 504
+    // segments: 23.1 against 23.8 with 768).  (On-demand pieces: every ticket group needs its wavefronts.)
+    const bool all = fixed_waves || option(kOptDynPieces) > 0 || overlap || (p.cache_dtype != HIPATTN_U8 && segments >= 128);
+    p.few_waves = all ? 0 : (int)std::max<int64_t>(512, 2 * segments);
     const size_t slots = (size_t)p.num_waves + p.dyn_pieces + (size_t)p.num_rows * p.num_heads_kv;
     uint8_t* w = (uint8_t*)workspace;
     p.dyn_counter = (int32_t*)w;
@@ -1997,8 +2013,10 @@ void paged_fast_plan(PagedParams& p, void* workspace) {
     // Built into the u8 kernels only (see kFusedBuilt).  Measured, whole steps on one machine: the 128-sequence
     // u8 batch 0.437 ms fused against 0.440 ms with the merge launch.  Where many pieces share a segment the one wavefront that
     // combines them in the kernel takes them two by two: one sequence of 778 tokens 36 against 12.5 us, of 16,384 88 against 24,
-    // 32 sequences of 4,000 (256 segments) 75 against 69, 64 of them (512 segments) 127 against 127: fused from there on.
-    const bool few_pieces = fixed_waves || p.num_waves <= 3 * (int64_t)p.num_rows * p.num_heads_kv;
+    // 32 sequences of 4,000 (256 segments) 75 against 69, 64 of them (512 segments) 127 against 127: fused up to three pieces to a
+    // segment, and up to four blocks, of which each may be one (49 sequences of 300: 20.4 against 22.4; 40 of 100: 15.0 against 17.6).
+    // Beside a chunk kernel the launch costs the host 8 us: up to eight blocks (a prompt of 60 tokens 35.5 against 44.5).
+    const bool few_pieces = fixed_waves || most_blocks(p) <= (overlap ? 8 : 4) || most_waves(p) <= 3 * segments;
     p.fused_merge = (option(kOptFusedMerge) != 0 && p.cache_dtype == HIPATTN_U8 && p.dyn_pieces == 0 && p.head_dim <= 128 && few_pieces) ? 1 : 0;
     p.merge_tag = next_merge_tag();
 }
