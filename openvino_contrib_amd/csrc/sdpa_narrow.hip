@@ -15,6 +15,8 @@
 // of 4,096: 102 -> 78 (880); 8 heads of 2,048: 43 -> 19; 8 of 128: 8.6 -> 5.2; 4 x 32 of 2,048, causal: 122 -> 79; size 96,
 // 8 x 12 heads of 700: 42 -> 34; against the plain masked kernel: 4 x 12 heads of 1,100 with a bias: 135 -> 39, size 128,
 // 4 x 32 heads of 1,000, padded: 454 -> 79.
+#include <algorithm>
+
 #include "device_common.hpp"
 #include "kernels.hpp"
 
@@ -541,7 +543,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kDP
 // with one and two), a fifth more where every step has a barrier, and what a workgroup costs however few its steps are.
 // Measured around the lines it draws, with 1 / 2 / 4: 8 heads of 2,048, size 64: 29.5 / 20.1 / 19.8 us; 12 of 800: 14.2 / 10.8 /
 // 12.0; 48 of 800: 18.4 / 16.7 / 26.6; 96 of 800: 24.8 / 27.7 / 49.2; 96 of 130: 6.4 / 7.3 / 7.7; 64 of 77 rows and 1,024 keys:
-// 16.2 / 12.0 / 10.1; 16 of 4,096: 80 / 88 / 121; size 128, 12 of 1,000: 25.2 / 17.2 / 27.7; 12 of 500, causal: 14.6 / 11.2 / 10.2.
+// 16.2 / 12.0 / 10.1; 16 of 4,096: 80 / 88 / 121; size 128, 12 of 1,000: 25.2 / 17.2 / 27.7; 12 of 500, causal: 14.6 / 11.2 / 10.2;
+// 16 x 32 of 150, causal, three rounds of workgroups where two share the rows: 18.5 / 24.2 (23.2 in the head-128 kernel).
 struct Split {
     int split;
     double cost;
@@ -558,7 +561,8 @@ Split choose_split(const SdpaParams& p) {
             const double fixed = split == 1 ? (p.head_dim <= 64 ? 1.5 : 2.5 * n - 1.0) : split == 2 ? 2.2 : 2.5 + 0.9 * n;
             return steps * (0.30 + share * n) * (split == 1 ? 1.0 : 1.2) + fixed;
         };
-        const double cost = (double)(per_cu / resident) * round(resident) + (per_cu % resident ? round((int)(per_cu % resident)) : 0);
+        double cost = (double)(per_cu / resident) * round(resident) + (per_cu % resident ? round((int)(per_cu % resident)) : 0);
+        if (split == 2 && p.head_dim > 96) cost += 2.2 * (double)((per_cu - 1) / resident);
         if (best.cost == 0 || cost < best.cost) best = {split, cost};
     }
     return best;
@@ -610,21 +614,23 @@ static bool sdpa_narrow_supported(const SdpaParams& p) {
            (((uintptr_t)p.q | (uintptr_t)p.k | (uintptr_t)p.v | (uintptr_t)p.out) & 15) == 0;
 }
 
-// Head sizes above 96 share with the kernel of flash_prefill.hip, whose workgroup has a compute unit to itself, takes 256 rows
-// and needs some 1.25 us for 64 keys, 1.5 with the chip full, and 4 to 5 besides: it is faster where it fills the chip (4 x 32 heads
-// of 2,048, causal: 141 against 152 us; 4 x 8 of 1,300: 35 against 42) and slower on small calls (8 heads of 2,048: 42 against 28;
-// 12 of 500, causal: 18.4 against 10.2; 8 of 48: 7.4 against 5.6) and with a mask.  Below,
-// it computes 128 columns all the same, and this one is at least as fast (size 80, 2 x 16 heads of 1,500: 38.0 and 38.3;
-// size 96, 8 x 12 of 700: 42 against 33).
+// Head sizes above 64 share with the kernel of flash_prefill.hip, whose workgroup has a compute unit to itself, takes 256 rows
+// and needs some 1.25 us for 64 keys, 1.5 to 1.8 with the chip full, and 4 to 7 besides.  Above 96 it is faster where it fills the chip (4 x 32
+// heads of 2,048, causal: 136 against 142 us; 4 x 8 of 1,300: 35 against 42) and slower on small calls (8 heads of 2,048: 42 against 28;
+// 12 of 500, causal: 18.4 against 10.2; 8 of 48: 7.4 against 5.6) and with a mask.  Up to 96 it computes 128 columns all the
+// same and is the faster one only without a mask or the causal flag, where its workgroups come out as one round and these as a
+// little more than one (size 80, 2 x 12 heads of 1,390: 33.2 against 35.2; 2 x 16 of 1,500: 38.0 and 38.3; 4 x 16 of 1,024: 33.8 against
+// 31.7; 8 x 12 of 700: 42 against 33).
 static bool sdpa_narrow_preferred(const SdpaParams& p) {
-    if (p.head_dim <= 96) return true;
-    // (additive masks: 4 x 8 heads of 1,024 33 against 50 us; 4 x 32 of 2,048, four rounds of workgroups: 375 there)
+    if (p.head_dim == 64 || (p.head_dim <= 96 && (p.mask || p.causal))) return true;
+    // (additive masks: 4 x 8 heads of 1,024 33 against 50 us; 4 x 32 of 2,048, four rounds of workgroups: 368 against 375)
     if (p.mask) return p.mask_dtype == HIPATTN_U8 || (int64_t)p.batch * p.num_heads_q * ((p.len_q + 127) / 128) <= 512;
     const int G = p.num_heads_q / p.num_heads_kv, q_tiles = (p.len_q + 127) / 128;
     const int64_t groups = (int64_t)p.batch * p.num_heads_kv * (G % 2 == 0 ? G / 2 * q_tiles : G * ((q_tiles + 1) / 2));
     const int64_t rounds = (groups + 255) / 256;
-    const double tiles = (p.len_kv + 63) / 64;
-    return narrow::choose_split(p).cost < 0.9 * (double)rounds * (tiles * (groups > 128 ? 1.5 : 1.25) + (rounds > 1 ? 5.0 : 4.0));
+    const double tiles = (p.len_kv + 63) / 64, cost = narrow::choose_split(p).cost;
+    if (p.head_dim <= 96) return cost < 1.02 * (double)rounds * (tiles * (1.25 + 0.55 / 128 * (double)std::clamp<int64_t>(groups - 128, 0, 128)) + 5.0);
+    return cost < 0.9 * (double)rounds * (tiles * (groups > 128 ? 1.5 : 1.25) + (rounds > 1 ? 7.0 : 4.0));
 }
 
 // (sdpa_padded_rows = 0 leaves head sizes below 128 to the plain kernels)

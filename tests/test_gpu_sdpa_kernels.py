@@ -180,6 +180,7 @@ def test_which_kernel_the_rule_takes(hip, oracle):
     for (B, Hq, Hkv, Lq, Lk, D, dtype, causal), kernel in [
             ((1, 4, 4, 64, 64, 64, W.F16, False), "sdpa_narrow"), ((1, 4, 4, 64, 64, 96, W.BF16, True), "sdpa_narrow"),
             ((1, 8, 8, 48, 48, 128, W.F16, True), "sdpa_narrow"), ((4, 32, 8, 1024, 1024, 128, W.BF16, True), "sdpa_flash"),
+            ((2, 12, 12, 1390, 1390, 80, W.F16, False), "sdpa_flash"), ((2, 12, 12, 1390, 1390, 80, W.F16, True), "sdpa_narrow"),
             ((1, 4, 4, 64, 64, 56, W.F16, False), "sdpa_flash"), ((1, 4, 4, 64, 64, 256, W.F16, False), "sdpa_flash_small"),
             ((1, 4, 4, 64, 64, 64, W.F32, False), "sdpa_f32"), ((1, 4, 4, 64, 64, 136, W.F32, False), "sdpa_generic")]:
         H.run_sdpa(hip, W.make_sdpa_case(28, B, Hq, Hkv, Lq, Lk, D, dtype), causal)
