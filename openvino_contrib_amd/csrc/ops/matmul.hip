@@ -1,6 +1,5 @@
-// MatMul: up to 16 rows in a kernel of matmul_few_rows.hip, else through hipBLASLt: a plain library GEMM with fp32
-// accumulation.  The operator's tensors
-// are row-major; hipBLASLt is column-major, so the product is taken transposed
+// MatMul: few rows (up to six, up to 16 on small weights) in the kernel of matmul_few_rows.hip, else through hipBLASLt: a
+// plain library GEMM with fp32 accumulation.  The operator's tensors are row-major; hipBLASLt is column-major, so the product is taken transposed
 // (C^T = op(B)^T * op(A)^T) with the operands swapped and no data movement.  Descriptors and the
 // algorithm are kept per (device, shape), so a repeated shape costs one hipblasLtMatmul call; the
 // algorithm is the fastest of the heuristic's candidates, timed once when the shape is first seen

@@ -1,5 +1,5 @@
-// Products of up to 16 activation rows with a weight matrix stored [n, k] -- the projections of a decode step of few
-// sequences -- on v_mfma_f32_16x16x32 with fp32 accumulation, instead of the library's kernels.
+// Products of few activation rows -- up to six, up to 16 on small weights -- with a weight matrix stored [n, k], the
+// projections of a decode step of few sequences, on v_mfma_f32_16x16x32 with fp32 accumulation, instead of the library's kernels.
 //
 // What bounds it: the weights, read once.  A workgroup takes 16 weight rows and its eight wavefronts an eighth of k each;
 // a lane's loads are the matrix operands as they stand (weight row lane % 16, eight k of quarter lane / 16; activations
@@ -101,15 +101,24 @@ __global__ __launch_bounds__(64 * kWaves) void matmul_few_rows_kernel(const uint
 // 16-bit operands, one matrix, the weights' rows along k, whole steps of k, 16-byte aligned rows.
 // Every activation row costs load instructions of its own and the library's kernels, built for tiles of 16, do not mind them,
 // so it is up to 6 rows, or 16 where the weights are small enough for the launch to be most of the time (library -> this,
-// 16 rows: 512 x 2,048 10.1 -> 5.6 us, 1,024 x 4,096 10.0 -> 9.1, 4,096 x 4,096 10.2 -> 10.6; 8 rows: 3,072 x 8,192 14.0 -> 14.6).
+// 16 rows: 512 x 2,048 10.1 -> 5.6 us, 1,024 x 4,096 10.0 -> 9.1, 4,096 x 4,096 10.2 -> 10.6; 8 rows: 3,072 x 8,192 14.0 -> 14.6), and
+// up to 4 on the largest (128,256 x 4,096, 1 / 4 / 6 rows: 173 / 174 / 175 -> 166 / 175 / 184).
+// A wavefront goes through its eighth of k alone, so k must not be long where n is short: a chain of 6,144 takes as long as the
+// library's split one (4 rows: 512 x 6,144 10.2 -> 9.6, 16 x 6,144 9.9 -> 9.1, but 64 x 8,192 10.1 -> 11.8, 256 x 16,384 13.3 -> 21.9;
+// 16 rows: 512 x 6,144 11.0 -> 12.5), beyond it n bounds k (2,048 x 7,168 12.4 -> 11.1, 4,096 x 14,336 25.5 -> 22.3,
+// but 2,048 x 8,192 12.0 -> 12.7, 3,072 x 12,288 19.0 -> 19.4, 4,096 x 16,384 29.8 -> 34.4, 8,192 x 28,672 85.1 -> 87.0).
 // Large weights only where every wavefront's k is whole rounds of two groups (4 rows: 8,192 x 4,096 15.8 -> 15.2, 14,336 x
 // 2,048 15.6 -> 15.1, but 21,504 x 3,072 27.4 -> 28.9 and 5,120 x 5,120 16.1 -> 17.1).
 bool matmul_few_rows_supported(const hipops_matmul_desc* d, const void* a, const void* b, const void* c) {
     const auto aligned16 = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
     const int64_t weights = d->n * d->k;
-    return (d->ab_dtype == HIPATTN_F16 || d->ab_dtype == HIPATTN_BF16) && d->batch == 1 && !d->transpose_a && d->transpose_b &&
-           d->n % 4 == 0 && d->k % 32 == 0 &&
-           (d->m <= 6 ? weights <= (1 << 24) || d->k % (2 * 32 * kGroup * kWaves) == 0 : d->m <= 16 && weights <= (1 << 22)) && aligned16(a) && aligned16(b) && aligned16(c);
+    if ((d->ab_dtype != HIPATTN_F16 && d->ab_dtype != HIPATTN_BF16) || d->batch != 1 || d->transpose_a || !d->transpose_b || d->n % 4 != 0 ||
+        d->k % 32 != 0 || !aligned16(a) || !aligned16(b) || !aligned16(c))
+        return false;
+    if (d->m > 6) return d->m <= 16 && weights <= (1 << 22) && d->k <= 4096;
+    if (d->m > 4 && weights > (1 << 27)) return false;
+    if (d->k > 6144 && (2 * d->k > 7 * d->n || weights > (1 << 27))) return false;
+    return weights <= (1 << 24) || d->k % (2 * 32 * kGroup * kWaves) == 0;
 }
 
 hipattn_status matmul_few_rows(const hipops_matmul_desc* d, const void* a, const void* b, void* c, hipStream_t stream) {

@@ -29,7 +29,7 @@ hipattn_status convert(const void* in, void* out, int64_t count, int from_dtype,
 hipattn_status binary(int op, const void* a, const void* b, void* out, int rank, const int64_t* out_dims, const int64_t* a_dims,
                       const int64_t* b_dims, int dtype, hipStream_t stream);
 hipattn_status softmax(const void* x, void* out, int64_t outer, int64_t length, int64_t inner, int dtype, hipStream_t stream);
-// up to 16 rows against weights stored [n, k] (matmul_few_rows.hip)
+// few rows against weights stored [n, k] (matmul_few_rows.hip)
 bool matmul_few_rows_supported(const hipops_matmul_desc* d, const void* a, const void* b, const void* c);
 hipattn_status matmul_few_rows(const hipops_matmul_desc* d, const void* a, const void* b, void* c, hipStream_t stream);
 hipattn_status matmul_workspace_size(const hipops_matmul_desc* desc, size_t* bytes);

@@ -23,3 +23,9 @@ def test_matmul_few_rows(hip, ops, oracle, m, n, k, dtype):  # noqa: F811
         ops.matmul(ops.MatmulDesc(dtype, c_dtype, m, n, k, 1, 0, 1, 0, 0), da, db, dc, None)
         got = download(hip, dc, c_dtype, (1, m, n))
         assert scaled_error(got, ref) <= (ROUND[dtype] if c_dtype == dtype else 0) + 1e-6 * np.sqrt(k)
+
+
+# either side of where the rule leaves a long k to the library: any n, n against k, and 16 rows
+@pytest.mark.parametrize("m,n,k", [(6, 16, 6144), (6, 16, 6176), (4, 2048, 7168), (4, 2044, 7168), (16, 64, 4096), (16, 64, 4128)])
+def test_matmul_lines_of_the_rule(hip, ops, oracle, m, n, k):  # noqa: F811
+    test_matmul_few_rows(hip, ops, oracle, m, n, k, BF16)
