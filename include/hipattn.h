@@ -186,7 +186,8 @@ hipattn_status hipattn_sdpa_masked(const hipattn_sdpa_desc* desc, const void* q,
  * Step 2: that token attends cache positions j, max(0, p - sliding_window + 1) <= j <= p
  * (all of 0..p when sliding_window <= 0).
  * All index arrays live in device memory and are only read there; the split of the work is
- * planned on the device.  max_context_len (>= max_s(past_lens[s] + q_len[s])) is advisory.
+ * planned on the device.  max_context_len (>= max_s(past_lens[s] + q_len[s])) is advisory: short contexts are scheduled
+ * by it, except in a call that is being captured, whose replays may see longer ones; 0 means not known.
  * A sequence may contribute any number of tokens to a batch, none included.  A batch with
  * num_tokens == num_seqs is planned per token (the host cannot see the lengths, and a decode
  * step should not pay for a prefill launch that finds nothing to do): every token is a decode

@@ -533,6 +533,10 @@ hipattn_status paged_attention_impl(const hipattn_pa_desc* desc, const void* q, 
     p.subsequence_begins = subsequence_begins;
     p.block_indices = block_indices;
     p.block_indices_begins = block_indices_begins;
+    // (a recorded call is replayed while the contexts grow past the bound it was recorded with: the schedule, which is all
+    // that the bound decides here, is then one for contexts of any length)
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (stream && (hipStreamIsCapturing(as_stream(stream), &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone)) p.max_context_len = 0;
     p.out = out;
     p.no_side_stream = static_scratch ? 1 : 0;  // (creating the side stream of a mixed batch allocates)
     // the caller's workspace, or the static scratch, checked against what the chosen path needs

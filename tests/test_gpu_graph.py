@@ -96,3 +96,48 @@ def test_paged_attention_replays_from_a_graph(hip, oracle, batch, cache_dtype, D
         ws.free()
         dev.free()
         stream.close()
+
+
+@pytest.mark.parametrize("cache_dtype", [W.U8, W.F16])
+def test_replays_outgrow_the_context_bound_of_the_recording(hip, oracle, cache_dtype):
+    """A decode step recorded while its contexts were short (bound 100) and replayed when they are long: the rows of the long ones."""
+    short = W.make_paged_case(96, [(60, 1), (99, 1), (5, 1)], 16, 4, 128, 32, W.F16, W.F16, cache_dtype)
+    case = W.make_paged_case(97, [(2000, 1), (99, 1), (700, 1)], 16, 4, 128, 32, W.F16, W.F16, cache_dtype)
+    ref, okc, ovc = H.oracle_paged(oracle, case)
+    rt = hip_runtime()
+    stream = hip.Stream()
+    dev = H.PagedDeviceCase(hip, case)
+    desc = H.pa_desc(hip, case, max_context_len=100)
+    ws = hip.DeviceBuffer(hip.paged_attention_workspace_size(desc))
+    lengths = hip.DeviceBuffer.from_numpy(short["past_lens"])  # (the short lengths fit the long sequences' tables)
+
+    def call(d):
+        hip.paged_attention(d, dev.q, dev.k_new, dev.v_new, dev.key_cache, dev.value_cache, lengths, dev.subsequence_begins,
+                            dev.block_indices, dev.block_indices_begins, dev.out, ws, stream)
+
+    call(H.pa_desc(hip, case, flags=hip.PA_SKIP_CACHE_WRITE, max_context_len=100))  # eager: whatever a device's first call sets up
+    graph, graph_exec = ctypes.c_void_p(), ctypes.c_void_p()
+    assert rt.hipStreamBeginCapture(stream.handle, CAPTURE_MODE_RELAXED) == 0
+    try:
+        call(desc)
+    finally:
+        status = rt.hipStreamEndCapture(stream.handle, ctypes.byref(graph))
+    assert status == 0 and graph.value
+    assert rt.hipGraphInstantiate(ctypes.byref(graph_exec), graph, None, None, 0) == 0
+    try:
+        lengths.upload(case["past_lens"], stream)
+        for replay in range(3):
+            dev.out.fill(0xFF, stream)
+            assert rt.hipGraphLaunch(graph_exec, stream.handle) == 0
+            got = H.storage_to_f32(dev.out.download(np.uint16, (case["T"], case["Hq"] * case["D"]), stream), W.F16)
+            assert H.max_abs(got, ref) <= (1e-2 if cache_dtype == W.U8 else 2e-3), replay
+        kc, vc = dev.caches()
+        np.testing.assert_array_equal(kc, okc)
+        np.testing.assert_array_equal(vc, ovc)
+    finally:
+        rt.hipGraphExecDestroy(graph_exec)
+        rt.hipGraphDestroy(graph)
+        for b in (ws, lengths):
+            b.free()
+        dev.free()
+        stream.close()
