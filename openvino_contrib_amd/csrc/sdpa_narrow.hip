@@ -9,12 +9,12 @@
 // that one is needed.  K and V tiles go straight into LDS, K in three stages (it is read half a tile ahead) and V in two.
 // Row sums are taken of the probabilities as they were rounded for the product, so that rounding them moves a row's mean less.
 //
-// Counters at 16 heads of 4,096, size 64: vector ALU 44 %, matrix cores 37 %, LDS 18 % of the cycles, no bank conflicts; the rest is
-// a step's own chain (LDS, products, exponentials, check) at two wavefronts per SIMD.
+// Counters at 16 heads of 4,096, size 64: vector ALU 45 %, matrix cores 40 % of the busy cycles (16 x 16 of 577: 53 %, 36 %), no bank
+// conflicts; the rest is a step's own chain (LDS, products, exponentials, check) at two wavefronts per SIMD.
 // Measured against the head-128 kernel on padded rows: 16 x 16 heads of 577, size 64, fp16: 60 -> 33 us (660 TFLOP/s); 16 heads
 // of 4,096: 102 -> 78 (880); 8 heads of 2,048: 43 -> 19; 8 of 128: 8.6 -> 5.2; 4 x 32 of 2,048, causal: 122 -> 79; size 96,
 // 8 x 12 heads of 700: 42 -> 34; against the plain masked kernel: 4 x 12 heads of 1,100 with a bias: 135 -> 39, size 128,
-// 4 x 32 heads of 1,000, padded: 454 -> 79.
+// 2 x 12 of 1,001 with a bias: 263 -> 33; 4 x 32 heads of 1,000, padded: 454 -> 79.
 #include <algorithm>
 
 #include "device_common.hpp"
