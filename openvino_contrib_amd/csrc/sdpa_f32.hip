@@ -323,6 +323,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDP == 128 
 #pragma unroll
                 for (int i = 0; i < kRegs; i++) o[i / (4 * kNT)][i / kNT % 4][i % kNT] += shares[(wave * kRegs + i) * 64 + lane];
         }
+        if (wave != 0) return;
     } else {
 #pragma unroll
         for (int nt = 0; nt < kNT; nt++) {
@@ -333,51 +334,28 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDP == 128 
                 for (int t = 0; t < 4; t++) o[cc][t][nt] *= f;
         }
     }
-    // The products multiply masked keys by a zero probability (an infinite value row would make that NaN) and let
-    // exponentials grow to 2^60 (times a value row above 1e20: infinity).  Rows that are not finite are worked again, the workgroup's
-    // wavefronts in turn, the way that skips such keys and keeps its reference at the maximum; where the inputs do ask
-    // for it they stay so.
-    uint32_t* const bad_rows = (uint32_t*)lds;  // (over the shares, which this wavefront has read)
-    uint32_t bad[kNT];
-    if (wave == 0) {
+    // lane (row n, q): register e of o[cc][t] is column 64 cc + 16 q + 4 e + t, sixteen in a row
 #pragma unroll
-        for (int nt = 0; nt < kNT; nt++) {
-            // lane (row n, q): register e of o[cc][t] is column 64 cc + 16 q + 4 e + t, sixteen in a row
-            const int row = row0 + 16 * nt + n;
-            float finite = 0.f;
+    for (int nt = 0; nt < kNT; nt++) {
+        const int row = row0 + 16 * nt + n;
+        // The products multiply masked keys by a zero probability (an infinite value row would make that NaN) and let
+        // exponentials grow to 2^60 (times a value row above 1e20: infinity).  Rows that are not finite are worked again
+        // the way that skips such keys and keeps its reference at the maximum; where the inputs do ask for it they stay so.
+        float finite = 0.f;
 #pragma unroll
-            for (int cc = 0; cc < kC; cc++)
+        for (int cc = 0; cc < kC; cc++)
 #pragma unroll
-                for (int t = 0; t < 4; t++)
+            for (int t = 0; t < 4; t++)
 #pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        if (!kPad || 64 * cc + 16 * quarter + 4 * e < D) finite = fmaf(o[cc][t][nt][e], 0.f, finite);
-            uint64_t rows = __builtin_amdgcn_ballot_w64(finite != 0.f && row < p.len_q);
-            rows |= rows >> 32;
-            bad[nt] = (uint32_t)(rows | rows >> 16) & 0xffffu;
-            if (waves > 1 && lane == 0) bad_rows[nt] = bad[nt];
-            if (row >= p.len_q || ((bad[nt] >> n) & 1)) continue;
-            float* const out = (float*)p.out + ((int64_t)bh * p.len_q + row) * D;
-#pragma unroll
-            for (int cc = 0; cc < kC; cc++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int d = 64 * cc + 16 * quarter + 4 * e;
-                    if (!kPad || d < D) *(float4_t*)(out + d) = (float4_t){o[cc][0][nt][e], o[cc][1][nt][e], o[cc][2][nt][e], o[cc][3][nt][e]};
-                }
-        }
-    }
-    if (waves > 1) {
-        __syncthreads();
-#pragma unroll
-        for (int nt = 0; nt < kNT; nt++) bad[nt] = __builtin_amdgcn_readfirstlane(bad_rows[nt]);
-    }
-    int turn = 0;
-#pragma unroll
-    for (int nt = 0; nt < kNT; nt++)
-        for (uint32_t left = bad[nt]; left != 0; left &= left - 1, turn++) {
-            if (turn % waves != wave) continue;
-            const int r = row0 + 16 * nt + __builtin_ctz(left);
+                for (int e = 0; e < 4; e++)
+                    if (!kPad || 64 * cc + 16 * quarter + 4 * e < D) finite = fmaf(o[cc][t][nt][e], 0.f, finite);
+        uint64_t bad = __builtin_amdgcn_ballot_w64(finite != 0.f && row < p.len_q);
+        bad |= bad >> 32;
+        bad = (bad | bad >> 16) & 0xffff;
+        const bool again = (bad >> n) & 1;
+        while (bad != 0) {
+            const int r = row0 + 16 * nt + __builtin_ctzll(bad);
+            bad &= bad - 1;
             const DenseKV kv{(const uint8_t*)k, (const uint8_t*)v, 4 * (int64_t)D, HIPATTN_F32};
             const float* const q_row = q + (int64_t)r * D;
             float x[kC];
@@ -393,6 +371,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDP == 128 
             for (int i = 0; i < kC; i++)
                 if (lane + 64 * i < D) ((float*)p.out)[((int64_t)bh * p.len_q + r) * D + lane + 64 * i] = x[i];
         }
+        if (row >= p.len_q || again) continue;
+        float* const out = (float*)p.out + ((int64_t)bh * p.len_q + row) * D;
+#pragma unroll
+        for (int cc = 0; cc < kC; cc++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int d = 64 * cc + 16 * quarter + 4 * e;
+                if (!kPad || d < D) *(float4_t*)(out + d) = (float4_t){o[cc][0][nt][e], o[cc][1][nt][e], o[cc][2][nt][e], o[cc][3][nt][e]};
+            }
+    }
 }
 
 template <int kDP, int kNT>

@@ -99,7 +99,7 @@ def test_nan_masks_reach_their_rows(hip, oracle, shape, mask_dtype):
 @pytest.mark.parametrize("shape", SHAPES)
 def test_an_infinite_value_stays_in_its_column(hip, oracle, shape, masked):
     """Every row attends a key with one infinite value: its column is infinite, the others are what they are.  Such rows are
-    worked again by all wavefronts of a workgroup, one row after the other."""
+    worked again, one after the other."""
     B, Hq, Hkv, Lq, Lk, D = shape
     case = W.make_sdpa_case(12, B, Hq, Hkv, Lq, Lk, D, W.F32)
     m = np.zeros((1, 1, Lq, Lk), np.float32)
