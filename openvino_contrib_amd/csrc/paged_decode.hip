@@ -635,6 +635,7 @@ __host__ __device__ __forceinline__ int working_waves(const PagedParams& p, int6
     const int eighth = total >= 8 * (int64_t)waves ? waves : (int)(total >> 3);  // (no division: it took 0.3 us of both kernels)
     int n = eighth > p.few_waves ? eighth : p.few_waves;
     if (n > 256) n = (n + 128) & ~255;
+    if (n > 1024) n &= ~511;  // (five wavefronts to a compute unit's four SIMDs: u8, 79 sequences of 40 to 335, 24.8 us with 1,280, 24.0 with 1,024)
     if (n > waves) n = waves;
     if (n > total) n = total > 256 ? (int)total & ~255 : (int)total;
     return n;
@@ -2014,9 +2015,12 @@ void paged_fast_plan(PagedParams& p, void* workspace) {
     // u8 batch 0.437 ms fused against 0.440 ms with the merge launch.  Where many pieces share a segment the one wavefront that
     // combines them in the kernel takes them two by two: one sequence of 778 tokens 36 against 12.5 us, of 16,384 88 against 24,
     // 32 sequences of 4,000 (256 segments) 75 against 69, 64 of them (512 segments) 127 against 127: fused up to three pieces to a
-    // segment, and up to four blocks, of which each may be one (49 sequences of 300: 20.4 against 22.4; 40 of 100: 15.0 against 17.6).
-    // Beside a chunk kernel the launch costs the host 8 us: up to eight blocks (a prompt of 60 tokens 35.5 against 44.5).
-    const bool few_pieces = fixed_waves || most_blocks(p) <= (overlap ? 8 : 4) || most_waves(p) <= 3 * segments;
+    // segment (49 sequences of 300: 20.4 against 22.4), two and a half at head size 64 (172 segments of 283: 21.0 against 19.3 with
+    // three), and up to two blocks, of which each may be a piece, or four in many segments (40 of 100: 15.0 against 17.6; 16 heads' 32
+    // segments of 81: 13.3 against 12.6).  Beside a chunk kernel the launch costs the host 8 us: up to eight blocks (a prompt of
+    // 60 tokens 35.5 against 44.5).
+    const bool few_pieces = fixed_waves || most_blocks(p) <= (overlap ? 8 : segments >= 128 ? 4 : 2) ||
+                            2 * most_waves(p) <= (p.head_dim <= 64 ? 5 : 6) * segments;
     p.fused_merge = (option(kOptFusedMerge) != 0 && p.cache_dtype == HIPATTN_U8 && p.dyn_pieces == 0 && p.head_dim <= 128 && few_pieces) ? 1 : 0;
     p.merge_tag = next_merge_tag();
 }
