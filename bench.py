@@ -278,7 +278,7 @@ RECORDED_TRAFFIC = {
     "c3": ((563582.6 * 2.0 + 3258.4) * 1024, "profiles/paged_decode_kernel_config3_fp16.txt"),
     "c4": ((1225872.7 * 2.0 + 12671.2) * 1024, "profiles/paged_decode_kernel_config4_u8.txt"),
     "c2": ((49302.7 * 2.0 + 65536.0) * 1024, "profiles/sdpa_flash_kernel_config2_bf16.txt"),
-    "c5": ((786147.1 * 2.0 + 6318.8) * 1024, "profiles/paged_attention_config5_mixed.txt"),  # the decode kernel of the mixed step
+    "c5": ((786147.1 * 2.0 + 6318.8) * 1024, "profiles/paged_attention_config5_mixed.txt"),  # the decode part of the mixed step
 }
 
 
@@ -291,7 +291,7 @@ def roofline_hbm(res, w):
     a = res["decode_kv_bytes"] / (res["dominant_kernel_ms"] * 1e-3) / 1e9
     traffic, source = recorded_traffic(w)
     return {"bound": "hbm", "achieved": a, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": a / HBM_PEAK_GBS,
-            "traffic": traffic, "traffic_source": source, "kernel": "paged_decode_kernel"}
+            "traffic": traffic, "traffic_source": source, "kernel": "paged_mixed_kernel" if w == "c5" else "paged_decode_kernel"}
 
 
 def roofline_mfma(res):

@@ -205,12 +205,13 @@ hipattn_status hipattn_sdpa_masked(const hipattn_sdpa_desc* desc, const void* q,
  * (probability zero in every kernel; a new token that falls there is not stored), and a row left with
  * nothing to attend is zeros.  No kernel reads outside the cache for such an entry.
  * A mixed batch (single-token and multi-token sequences) with decode_waves == 0 runs its two
- * parts side by side: the call forks from `stream` onto a side stream that the library keeps for
+ * parts side by side, in one launch at head size 128 and, with 16-bit caches on 16-byte aligned rows, between 64 and
+ * 128.  Other shapes (and calls with sinks): the call forks from `stream` onto a side stream that the library keeps for
  * that stream (created by the first such call on it, default priority, destroyed by
  * hipattn_stream_destroy; the library keeps at most 32, further streams share one) and joins before
  * it returns, so `stream` order is all the caller has to know, also under stream capture (make the
  * first such call on a stream outside a capture: creating a stream is not a capturable operation).  The
- * option "mixed_overlap" = 0 (hipattn_set_option) switches that off. */
+ * option "mixed_overlap" = 0 (hipattn_set_option) switches both off. */
 enum {
     HIPATTN_PA_SKIP_CACHE_WRITE = 1, /* attention only; k_new / v_new may be NULL */
     HIPATTN_PA_FORCE_GENERIC = 2,    /* use the shape-generic kernels (testing aid) */
@@ -331,8 +332,8 @@ size_t hipattn_cache_row_bytes(hipattn_dtype cache_dtype, int head_dim);
  * Execute calls with events, src/cuda_profiler.hpp:141-146).  While a pair of events is set
  * on the calling thread, hipattn_sdpa / hipattn_paged_attention record `before` immediately
  * ahead of and `after` immediately behind the launch of their dominant kernel (the flash
- * kernel, or the split-context decode kernel when the batch has decode sequences), on the
- * call's stream.  Pass NULLs to switch it off. */
+ * kernel, or the split-context decode kernel when the batch has decode sequences -- with the chunks
+ * of a mixed batch, where one launch does both), on the call's stream.  Pass NULLs to switch it off. */
 hipattn_status hipattn_profile_dominant_kernel(hipattn_event before, hipattn_event after);
 
 /* Process-wide schedule options (no reference counterpart; the reference's knobs are OpenVINO

@@ -21,6 +21,7 @@ SOURCES = [
     "sdpa_f32.hip",
     "sdpa_narrow.hip",
     "paged_decode.hip",
+    "paged_mixed.hip",
     "paged_scores.hip",
     "flash_prefill.hip",
     "flash_small.hip",

@@ -197,6 +197,9 @@ void release_side_stream(hipStream_t owner);  // drops the side stream mixed bat
 // write == nullptr skips the KV-cache write of the new tokens
 hipError_t launch_paged_fast(const PagedParams& p, const KvWriteParams* write, hipStream_t stream,
                              const KernelProbe& probe);
+// decode rows and chunks of a mixed batch in one launch (needs the plan, with p.overlap); chunk_heads_kv: the cache's own kv heads
+bool paged_mixed_supported(const PagedParams& p);
+hipError_t launch_paged_mixed(const PagedParams& p, int chunk_heads_kv, hipStream_t stream);
 hipError_t launch_paged_prefill(const PagedParams& p, hipStream_t stream);  // flash over the block table (needs the plan)
 hipError_t launch_paged_prefill_small(const PagedParams& p, hipStream_t stream);  // the same at head size 64 (flash_small.hip)
 
