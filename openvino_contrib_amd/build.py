@@ -82,7 +82,7 @@ def build_library(verbose=False, extra_flags=(), jobs=4):
 
 
 OPS_LIB_PATH = os.path.join(CSRC, "libhipops.so")
-OPS_SOURCES = ["ops/hipops_api.hip", "ops/layer_ops.hip", "ops/format_ops.hip", "ops/math_ops.hip", "ops/matmul.hip", "ops/matmul_few_rows.hip"]
+OPS_SOURCES = ["ops/hipops_api.hip", "ops/layer_ops.hip", "ops/format_ops.hip", "ops/math_ops.hip", "ops/matmul.hip", "ops/matmul_few_rows.hip", "ops/matmul_mid_rows.hip"]
 
 
 def build_ops_library(verbose=False, extra_flags=(), jobs=4):
