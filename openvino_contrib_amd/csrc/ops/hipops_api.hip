@@ -101,6 +101,11 @@ HIPOPS_API hipattn_status hipops_softmax(const void* x, void* out, int64_t outer
     return guarded("hipops_softmax", [&] { return softmax(x, out, outer, length, inner, dtype, (hipStream_t)stream); });
 }
 
+HIPOPS_API hipattn_status hipops_projection(const hipops_projection_desc* desc, const hipops_projection_args* tensors, void* workspace,
+                                            size_t workspace_bytes, hipattn_stream stream) {
+    return guarded("hipops_projection", [&] { return projection(desc, tensors, workspace, workspace_bytes, (hipStream_t)stream); });
+}
+
 HIPOPS_API hipattn_status hipops_glu(const void* x, void* out, int64_t rows, int64_t width, int activation, int gate_first,
                                      int dtype, hipattn_stream stream) {
     return guarded("hipops_glu", [&] { return glu(x, out, rows, width, activation, gate_first, dtype, (hipStream_t)stream); });

@@ -210,14 +210,6 @@ __global__ __launch_bounds__(256) void rope_scalar_kernel(RopeParams p) {
 }
 
 // ------------------------------------------------------------------------------ Swish, Multiply, GLU
-__device__ __forceinline__ float activate(float x, int activation, float beta) {
-    switch (activation) {
-        case HIPOPS_GLU_GELU: return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f));
-        case HIPOPS_GLU_GELU_TANH: return 0.5f * x * (1.0f + tanhf(0.79788456080286536f * (x + 0.044715f * x * x * x)));
-        default: return x / (1.0f + __expf(-beta * x));
-    }
-}
-
 struct EltwiseParams {
     const void* a;  // x (swish), a (multiply), the gate half's row 0 (glu)
     const void* b;  // multiply: b; glu: the other half's row 0

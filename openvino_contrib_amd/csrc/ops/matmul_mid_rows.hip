@@ -57,35 +57,49 @@ __device__ __forceinline__ void barrier_keeping() {
     asm volatile("" ::: "memory");
 }
 
+constexpr int kMaxWeights = 3;
+
 struct MidRowsParams {
-    const uint16_t* a;  // [m, k]
-    const uint16_t* b;  // [n, k]
-    void* c;            // [m, n] of the operands' type or fp32; sums of a part of k: [parts][m][n] fp32
-    int m, n;
+    const uint16_t* a;               // [m, k]
+    const uint16_t* b[kMaxWeights];  // [n[i], k]
+    void* c[kMaxWeights];            // [m, n[i]] of the operands' type or fp32; not written where there are sums
+    float* sums;                     // null, or the parts' sums: [parts][m][sum of n] fp32
+    int n[kMaxWeights];
+    int begin[kMaxWeights];          // the first tile of weights i
+    int offset[kMaxWeights];         // their first column in a row of sums
+    int m, columns, tiles, parts, c_is_f32;
+    int activation, gate_first;      // kGlu
     int64_t k;
-    int tiles, parts, c_is_f32;
 };
 
-template <bool kBf16, int kM, int kWaves, int kRing>
+// kGlu: the weight rows are the two halves of a gated MLP; a wavefront's 16 are eight of the gate's and the same eight of the other half,
+// c is [m, n / 2].
+template <bool kBf16, bool kGlu, int kM, int kWaves, int kRing>
 __global__ __launch_bounds__(64 * kWaves) void matmul_mid_rows_kernel(MidRowsParams p) {
     constexpr int kTileN = 16 * kWaves, kRows = kTileN + 16 * kM, kSlot = kRows * kStageBytes;
     constexpr int kXLoads = (2 * kM + kWaves - 1) / kWaves, kLoads = 2 + kXLoads;  // loads of a wavefront for a stage, eight rows each
     __shared__ __attribute__((aligned(128))) uint8_t lds[kRing * kSlot];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, row = lane & 15, quarter = lane >> 4;
-    const int tile = (int)blockIdx.x % p.tiles, part = (int)blockIdx.x / p.tiles;
+    const int tile_of_all = (int)blockIdx.x % p.tiles, part = (int)blockIdx.x / p.tiles;
+    const int which = (tile_of_all >= p.begin[1]) + (tile_of_all >= p.begin[2]);  // (absent weights begin behind the last tile)
+    const int tile = tile_of_all - p.begin[which], n = p.n[which];
     const int stages = (int)(p.k / 64);
     const int first = (int)((int64_t)stages * part / p.parts), count = (int)((int64_t)stages * (part + 1) / p.parts) - first;
     // lane l loads piece (l % 8) ^ (row % 8) of row l / 8, so that the pieces a fragment reads lie on different banks
     const int lrow = lane >> 3, piece = (lane & 7) ^ lrow;
     // workgroups begin at different stages of their part: rows whose distance is a power of two would have all of them wait for the same
     // memory channels
-    int stage = (int)((uint32_t)tile * 37u % (uint32_t)max(count, 1));
-    const char* const wbase = (const char*)(p.b + (int64_t)(kTileN * tile) * p.k + 64 * (int64_t)first);
+    int stage = (int)((uint32_t)tile_of_all * 37u % (uint32_t)max(count, 1));
+    const char* const wbase = (const char*)(p.b[which] + 64 * (int64_t)first);
     const char* const xbase = (const char*)(p.a + 64 * (int64_t)first);
     uint32_t w[2], x[kXLoads];
     int xrow[kXLoads];
 #pragma unroll
-    for (int i = 0; i < 2; i++) w[i] = (uint32_t)min(16 * wave + 8 * i + lrow, p.n - 1 - kTileN * tile) * (uint32_t)(2 * p.k) + 16 * piece;
+    for (int i = 0; i < 2; i++) {
+        int r = min(kTileN * tile + 16 * wave + 8 * i + lrow, n - 1);
+        if constexpr (kGlu) r = min((kTileN * tile + 16 * wave) / 2 + lrow, n / 2 - 1) + (p.gate_first ? i : 1 - i) * (n / 2);
+        w[i] = (uint32_t)r * (uint32_t)(2 * p.k) + 16 * piece;
+    }
 #pragma unroll
     for (int i = 0; i < kXLoads; i++) {
         xrow[i] = 8 * ((kXLoads * wave + i) % (2 * kM));  // (some twice)
@@ -126,18 +140,42 @@ __global__ __launch_bounds__(64 * kWaves) void matmul_mid_rows_kernel(MidRowsPar
         fill = fill + 1 == kRing ? 0 : fill + 1;
     }
     // register r: weight row 4 quarter + r of the wavefront's 16, activation row lane % 16
+    if constexpr (kGlu) {
+        const int at = (kTileN * tile + 16 * wave) / 2 + 4 * quarter;  // (of quarters 0 and 1; n / 2 is a multiple of 4)
+#pragma unroll
+        for (int i = 0; i < kM; i++) {
+            float4_t other, o;
+#pragma unroll
+            for (int r = 0; r < 4; r++) other[r] = __shfl_xor(acc[i][r], 32);
+            const int out_row = 16 * i + row;
+            if (quarter > 1 || at >= n / 2 || out_row >= p.m) continue;
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[r] = activate(acc[i][r], p.activation, 1.0f) * other[r];
+            *(uint2_t*)((uint16_t*)p.c[0] + (int64_t)out_row * (n / 2) + at) = (uint2_t){cvt2<kBf16>(o[0], o[1]), cvt2<kBf16>(o[2], o[3])};
+        }
+        return;
+    }
     const int at = kTileN * tile + 16 * wave + 4 * quarter;  // (n is a multiple of 4)
-    if (at >= p.n) return;
+    if (at >= n) return;
 #pragma unroll
     for (int i = 0; i < kM; i++) {
         const int out_row = 16 * i + row;
         if (out_row >= p.m) break;
-        const int64_t o = ((int64_t)part * p.m + out_row) * p.n + at;
-        if (p.parts > 1 || p.c_is_f32)
-            *(float4_t*)((float*)p.c + o) = acc[i];
+        const int64_t o = (int64_t)out_row * n + at;
+        if (p.sums != nullptr)
+            *(float4_t*)(p.sums + ((int64_t)part * p.m + out_row) * p.columns + p.offset[which] + at) = acc[i];
+        else if (p.c_is_f32)
+            *(float4_t*)((float*)p.c[which] + o) = acc[i];
         else
-            *(uint2_t*)((uint16_t*)p.c + o) = (uint2_t){cvt2<kBf16>(acc[i][0], acc[i][1]), cvt2<kBf16>(acc[i][2], acc[i][3])};
+            *(uint2_t*)((uint16_t*)p.c[which] + o) = (uint2_t){cvt2<kBf16>(acc[i][0], acc[i][1]), cvt2<kBf16>(acc[i][2], acc[i][3])};
     }
+}
+
+__device__ __forceinline__ float4_t add_parts(const float* sums, int64_t part_stride, int parts) {
+    float4_t sum = *(const float4_t*)sums;
+#pragma unroll 4
+    for (int p = 1; p < parts; p++) sum += *(const float4_t*)(sums + p * part_stride);
+    return sum;
 }
 
 // The parts' sums, in their order; four elements a lane.
@@ -145,13 +183,111 @@ template <bool kBf16>
 __global__ __launch_bounds__(256) void matmul_sum_parts_kernel(const float* sums, void* c, int64_t count, int parts, int c_is_f32) {
     const int64_t i = 4 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
     if (i >= count) return;
-    float4_t sum = *(const float4_t*)(sums + i);
-#pragma unroll 4
-    for (int p = 1; p < parts; p++) sum += *(const float4_t*)(sums + p * count + i);
+    const float4_t sum = add_parts(sums + i, count, parts);
     if (c_is_f32)
         *(float4_t*)((float*)c + i) = sum;
     else
         *(uint2_t*)((uint16_t*)c + i) = (uint2_t){cvt2<kBf16>(sum[0], sum[1]), cvt2<kBf16>(sum[2], sum[3])};
+}
+
+struct FinishParams {
+    const float* sums;
+    void* out[kMaxWeights];
+    int n[kMaxWeights], offset[kMaxWeights];
+    int m, columns, parts, dtype;
+    int rotated, head_size;  // rotated: a bit for each output
+    const void *cos, *sin;
+    const int32_t* positions;
+    int64_t table_row_stride;
+    int table_dtype, gamma_dtype;
+    const void *residual, *gamma;
+    void* normalised;
+    float eps;
+};
+
+// What follows the products, on the parts' sums: a rotary embedding of some outputs, or a residual; eight elements a lane, of a rotated
+// head four of each half.  Replaces a launch for each, which is most of what these cost (4 to 5 us each for a serving batch).
+__global__ __launch_bounds__(256) void projection_finish_kernel(FinishParams p) {
+    const int item = (int)blockIdx.x * 256 + threadIdx.x, row = (int)blockIdx.y;
+    if (8 * item >= p.columns) return;
+    const int which = (8 * item >= p.offset[1]) + (8 * item >= p.offset[2]);
+    const int local = item - p.offset[which] / 8;
+    const bool rotate = (p.rotated >> which) & 1;
+    int c0 = 8 * local, c1 = c0 + 4, i = 0;
+    const int half = p.head_size / 2;
+    if (rotate) {
+        const int head = local / (p.head_size / 8);
+        i = 4 * (local - head * (p.head_size / 8));
+        c0 = head * p.head_size + i, c1 = c0 + half;
+    }
+    const int64_t stride = (int64_t)p.m * p.columns;
+    const float* const s = p.sums + (int64_t)row * p.columns + p.offset[which];
+    const float4_t lo = add_parts(s + c0, stride, p.parts), hi = add_parts(s + c1, stride, p.parts);
+    float4_t ol = lo, oh = hi;
+    const int64_t base = (int64_t)row * p.n[which];
+    if (rotate) {
+        const int64_t tb = (p.positions ? (int64_t)p.positions[row] : row) * p.table_row_stride + i;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            ol[k] = lo[k] * load_scalar(p.cos, tb + k, p.table_dtype) - hi[k] * load_scalar(p.sin, tb + k, p.table_dtype);
+            oh[k] = hi[k] * load_scalar(p.cos, tb + half + k, p.table_dtype) + lo[k] * load_scalar(p.sin, tb + half + k, p.table_dtype);
+        }
+    } else if (p.residual != nullptr) {
+        const Float8 r = load8(p.residual, base + c0, p.dtype);
+#pragma unroll
+        for (int k = 0; k < 4; k++) ol[k] += r.v[k], oh[k] += r.v[4 + k];
+    }
+    const auto store = [&](int64_t at, const float4_t& v) {
+        *(uint2_t*)((uint16_t*)p.out[which] + at) = p.dtype == HIPATTN_BF16 ? (uint2_t){cvt2<true>(v[0], v[1]), cvt2<true>(v[2], v[3])}
+                                                                            : (uint2_t){cvt2<false>(v[0], v[1]), cvt2<false>(v[2], v[3])};
+    };
+    store(base + c0, ol);
+    store(base + c1, oh);
+}
+
+constexpr int kNormThreads = 512, kNormKeep = 4;  // chunks of eight elements that a lane keeps: rows of up to 16,384
+
+// The residual added to the parts' sums, and the RMS norm of the rounded result; a workgroup to a row.
+__global__ __launch_bounds__(kNormThreads) void projection_norm_kernel(FinishParams p) {
+    __shared__ float partial[kNormThreads / 64];
+    const int64_t base = (int64_t)blockIdx.x * p.columns, stride = (int64_t)p.m * p.columns;
+    const int chunks = p.columns / 8;
+    Float8 keep[kNormKeep];
+    float sq = 0.f;
+#pragma unroll
+    for (int c = 0; c < kNormKeep; c++) {
+        const int ch = threadIdx.x + c * kNormThreads;
+        if (ch < chunks) {
+            const float4_t lo = add_parts(p.sums + base + 8 * ch, stride, p.parts), hi = add_parts(p.sums + base + 8 * ch + 4, stride, p.parts);
+            Float8 r = load8(p.residual, base + 8 * ch, p.dtype);
+#pragma unroll
+            for (int k = 0; k < 4; k++) r.v[k] += lo[k], r.v[4 + k] += hi[k];
+            store8(p.out[0], base + 8 * ch, p.dtype, r);
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                keep[c].v[k] = p.dtype == HIPATTN_BF16 ? (float)(__bf16)r.v[k] : (float)(_Float16)r.v[k];
+                sq = fmaf(keep[c].v[k], keep[c].v[k], sq);
+            }
+        }
+    }
+    sq = wave_sum(sq);
+    if ((threadIdx.x & 63) == 0) partial[threadIdx.x / 64] = sq;
+    __syncthreads();
+    sq = 0.f;
+#pragma unroll
+    for (int w = 0; w < kNormThreads / 64; w++) sq += partial[w];
+    const float inv = 1.0f / sqrtf(sq / (float)p.columns + p.eps);
+#pragma unroll
+    for (int c = 0; c < kNormKeep; c++) {
+        const int ch = threadIdx.x + c * kNormThreads;
+        if (ch < chunks) {
+            const Float8 g = load8(p.gamma, 8 * ch, p.gamma_dtype);
+            Float8 o;
+#pragma unroll
+            for (int k = 0; k < 8; k++) o.v[k] = (keep[c].v[k] * inv) * g.v[k];
+            store8(p.normalised, base + 8 * ch, p.dtype, o);
+        }
+    }
 }
 
 struct Split {
@@ -160,70 +296,161 @@ struct Split {
 // Wavefronts to a workgroup and parts of k, by the bytes that the busiest compute unit moves: its share of the weights and, with parts, the
 // chip's traffic of their sums.  A part is five stages or more (64 rows: 1,024 x 4,096 in 16 / 12 parts 11.2 / 10.5 us; 2,048 x 2,048 in
 // 8 / 6 9.4 / 8.9), four wavefronts unless six deal the rows out better (22,016 x 4,096: 45.8 -> 39.6; 6,144 x 4,096: 17.0 -> 15.3).
-Split split_of(int64_t m, int64_t n, int64_t k, size_t workspace_bytes) {
+Split split_of(int64_t m, const int64_t* n, int count, int64_t k, size_t workspace_bytes, bool whole_k) {
     constexpr int64_t kUnits = 256;
     Split best{4, 1};
-    int64_t least = INT64_MAX;
+    int64_t least = INT64_MAX, columns = 0;
+    for (int i = 0; i < count; i++) columns += n[i];
     for (int waves = 4; waves <= 6; waves += 2) {
-        const int64_t tiles = (n + 16 * waves - 1) / (16 * waves);
-        for (int64_t parts = 1; parts <= 16 && (parts == 1 || (parts * 5 <= k / 64 && parts * tiles <= 2 * kUnits)); parts++) {
-            if (parts > 1 && (size_t)(parts * m * n * 4) > workspace_bytes) break;
-            const int64_t cost = (tiles * parts + kUnits - 1) / kUnits * (16 * waves) * (2 * k / parts) + (parts > 1 ? parts * m * n * 8 / kUnits : 0);
+        int64_t tiles = 0;
+        for (int i = 0; i < count; i++) tiles += (n[i] + 16 * waves - 1) / (16 * waves);
+        for (int64_t parts = 1; parts <= 16 && (parts == 1 || (!whole_k && parts * 5 <= k / 64 && parts * tiles <= 2 * kUnits)); parts++) {
+            if (parts > 1 && (size_t)(parts * m * columns * 4) > workspace_bytes) break;
+            const int64_t cost = (tiles * parts + kUnits - 1) / kUnits * (16 * waves) * (2 * k / parts) + (parts > 1 ? parts * m * columns * 8 / kUnits : 0);
             if (cost < least) least = cost, best = {waves, (int)parts};
         }
     }
     return best;
 }
 
-template <bool kBf16, int kM>
+template <bool kBf16, bool kGlu, int kM>
 void launch(const MidRowsParams& p, int waves, hipStream_t stream) {
     const dim3 grid((unsigned)(p.tiles * p.parts));
     constexpr int kRing4 = kM == 1 ? 5 : 4, kRing6 = kM == 4 ? 4 : 5;  // (two workgroups to a compute unit, or three)
     if (waves == 4)
-        hipLaunchKernelGGL((matmul_mid_rows_kernel<kBf16, kM, 4, kRing4>), grid, dim3(256), 0, stream, p);
+        hipLaunchKernelGGL((matmul_mid_rows_kernel<kBf16, kGlu, kM, 4, kRing4>), grid, dim3(256), 0, stream, p);
     else
-        hipLaunchKernelGGL((matmul_mid_rows_kernel<kBf16, kM, 6, kRing6>), grid, dim3(384), 0, stream, p);
+        hipLaunchKernelGGL((matmul_mid_rows_kernel<kBf16, kGlu, kM, 6, kRing6>), grid, dim3(384), 0, stream, p);
 }
 
-template <bool kBf16>
+template <bool kBf16, bool kGlu>
 void launch(const MidRowsParams& p, int waves, hipStream_t stream) {
     if (p.m <= 16)
-        launch<kBf16, 1>(p, waves, stream);
+        launch<kBf16, kGlu, 1>(p, waves, stream);
     else if (p.m <= 32)
-        launch<kBf16, 2>(p, waves, stream);
+        launch<kBf16, kGlu, 2>(p, waves, stream);
     else
-        launch<kBf16, 4>(p, waves, stream);
+        launch<kBf16, kGlu, 4>(p, waves, stream);
+}
+
+// the products of one input with `count` weights, as tiles of split.waves wavefronts
+MidRowsParams params_of(const void* a, const void* const* b, void* const* c, const int64_t* n, int count, int64_t m, int64_t k, const Split& split,
+                        float* sums) {
+    MidRowsParams p{};
+    p.a = (const uint16_t*)a, p.sums = sums, p.m = (int)m, p.k = k, p.parts = split.parts;
+    for (int i = 0; i < kMaxWeights; i++) {
+        p.begin[i] = INT32_MAX;
+        if (i >= count) continue;
+        p.b[i] = (const uint16_t*)b[i], p.c[i] = c[i], p.n[i] = (int)n[i];
+        p.begin[i] = p.tiles, p.offset[i] = p.columns;
+        p.tiles += (int)((n[i] + 16 * split.waves - 1) / (16 * split.waves)), p.columns += (int)n[i];
+    }
+    return p;
+}
+
+bool aligned16(const void* x) { return ((uintptr_t)x & 15) == 0; }
+bool sizes_supported(int dtype, int64_t n, int64_t k) {
+    return (dtype == HIPATTN_F16 || dtype == HIPATTN_BF16) && k % 64 == 0 && k < (1 << 24) && n * k <= (1 << 28);
 }
 
 }  // namespace
 
-// 16-bit operands, one matrix, the weights' rows along k in whole stages (and 96 rows within 32 bits of offset), 16-byte
+// 16-bit operands, one matrix, the weights' rows along k in whole stages (and all of them within 32 bits of offset), 16-byte
 // aligned rows.  The sums of the parts need a workspace; without one k stays whole.  The largest weights are the library's
 // (128,256 x 4,096 with 7 / 16 / 64 rows: 180 / 191 / 202 us there, 186 / 188 / 206 here).
 bool matmul_mid_rows_supported(const hipops_matmul_desc* d, const void* a, const void* b, const void* c) {
-    const auto aligned16 = [](const void* x) { return ((uintptr_t)x & 15) == 0; };
-    return (d->ab_dtype == HIPATTN_F16 || d->ab_dtype == HIPATTN_BF16) && d->batch == 1 && !d->transpose_a && d->transpose_b && d->m > 6 && d->m <= 64 &&
-           d->n % 4 == 0 && d->k % 64 == 0 && d->k < (1 << 24) && d->n * d->k <= (1 << 28) && aligned16(a) && aligned16(b) && aligned16(c);
+    return sizes_supported(d->ab_dtype, d->n, d->k) && d->batch == 1 && !d->transpose_a && d->transpose_b && d->m > 6 && d->m <= 64 && d->n % 4 == 0 &&
+           aligned16(a) && aligned16(b) && aligned16(c);
 }
 
 hipattn_status matmul_mid_rows(const hipops_matmul_desc* d, const void* a, const void* b, void* c, void* workspace, size_t workspace_bytes,
                                hipStream_t stream) {
-    const Split split = split_of(d->m, d->n, d->k, workspace ? workspace_bytes : 0);
+    const Split split = split_of(d->m, &d->n, 1, d->k, workspace ? workspace_bytes : 0, false);
     const bool bf16 = d->ab_dtype == HIPATTN_BF16;
-    const int c_is_f32 = d->c_dtype == HIPATTN_F32 ? 1 : 0, rows = 16 * split.waves;
-    const MidRowsParams p{(const uint16_t*)a, (const uint16_t*)b, split.parts > 1 ? workspace : c, (int)d->m, (int)d->n, d->k,
-                          (int)((d->n + rows - 1) / rows), split.parts, c_is_f32};
+    MidRowsParams p = params_of(a, &b, &c, &d->n, 1, d->m, d->k, split, split.parts > 1 ? (float*)workspace : nullptr);
+    p.c_is_f32 = d->c_dtype == HIPATTN_F32 ? 1 : 0;
     if (bf16)
-        launch<true>(p, split.waves, stream);
+        launch<true, false>(p, split.waves, stream);
     else
-        launch<false>(p, split.waves, stream);
+        launch<false, false>(p, split.waves, stream);
     if (split.parts > 1) {
         const int64_t count = d->m * d->n;
         const dim3 grid((unsigned)((count / 4 + 255) / 256));
         const auto kernel = bf16 ? matmul_sum_parts_kernel<true> : matmul_sum_parts_kernel<false>;
-        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, (const float*)workspace, c, count, split.parts, c_is_f32);
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, p.sums, c, count, split.parts, p.c_is_f32);
     }
     if (const hipError_t e = hipGetLastError(); e != hipSuccess) return fail(HIPATTN_HIP_ERROR, "matmul: %s", hipGetErrorString(e));
+    return HIPATTN_OK;
+}
+
+// Up to 64 rows: one launch for all the products of an input and one for what follows them, where the operators one by one are a
+// launch each.  Bounded by the weights, once launches are few: us, 4 / 64 rows of hidden 4,096, 32 / 8 heads of 128, MLP 14,336: q, k, v and
+// two rotary embeddings in five to eight launches 33 / 62 -> 15.6 / 20.1; o, residual and norm 18 / 34 -> 13.7 / 16.2; gate|up and SwiGLU
+// 47 / 57 -> 42.0 / 54.4; down and residual 26 / 42 -> 25.8 / 31.8.
+hipattn_status projection(const hipops_projection_desc* d, const hipops_projection_args* t, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+    if (!d || !t) return fail(HIPATTN_INVALID_ARGUMENT, "projection: null descriptor");
+    const auto refuse = [](const char* why) { return fail(HIPATTN_UNSUPPORTED, "projection: %s", why); };
+    if (d->num_weights < 1 || d->num_weights > kMaxWeights) return refuse("one to three weights");
+    if (d->rows < 1 || d->rows > 64) return refuse("1 to 64 rows");
+    const bool glu = d->kind == HIPOPS_PROJECTION_GLU, add = d->kind == HIPOPS_PROJECTION_ADD, rope = d->kind == HIPOPS_PROJECTION_ROPE;
+    if (!glu && !add && !rope) return fail(HIPATTN_INVALID_ARGUMENT, "projection: kind %d", d->kind);
+    if ((glu || add) && d->num_weights != 1) return refuse("several weights go with a rotary embedding only");
+    int64_t columns = 0;
+    for (int i = 0; i < d->num_weights; i++) {
+        if (d->n[i] < 1 || d->n[i] % 8 != 0 || !sizes_supported(d->dtype, d->n[i], d->k) || d->k < 64) return refuse("types or sizes");
+        if (!t->weights[i] || !t->outs[i]) return fail(HIPATTN_INVALID_ARGUMENT, "projection: null pointer");
+        if (!aligned16(t->weights[i]) || !aligned16(t->outs[i])) return refuse("operands off 16 bytes");
+        columns += d->n[i];
+    }
+    if (!t->x) return fail(HIPATTN_INVALID_ARGUMENT, "projection: null pointer");
+    if (!aligned16(t->x)) return refuse("operands off 16 bytes");
+    const bool bf16 = d->dtype == HIPATTN_BF16;
+    if (glu) {
+        if (d->glu_activation < HIPOPS_GLU_SWISH || d->glu_activation > HIPOPS_GLU_GELU_TANH)
+            return fail(HIPATTN_INVALID_ARGUMENT, "projection: activation %d", d->glu_activation);
+        const Split split = split_of(d->rows, d->n, 1, d->k, 0, true);
+        MidRowsParams p = params_of(t->x, t->weights, t->outs, d->n, 1, d->rows, d->k, split, nullptr);
+        p.activation = d->glu_activation, p.gate_first = d->glu_gate_first ? 1 : 0;
+        if (bf16)
+            launch<true, true>(p, split.waves, stream);
+        else
+            launch<false, true>(p, split.waves, stream);
+    } else {
+        const auto float_type = [](int x) { return x == HIPATTN_F32 || x == HIPATTN_F16 || x == HIPATTN_BF16; };
+        if (add && (!t->residual || (t->gamma == nullptr) != (t->normalised == nullptr))) return fail(HIPATTN_INVALID_ARGUMENT, "projection: null pointer");
+        if (add && (!aligned16(t->residual) || !aligned16(t->gamma) || !aligned16(t->normalised))) return refuse("operands off 16 bytes");
+        if (t->gamma && (!float_type(d->gamma_dtype) || columns > 8 * kNormThreads * kNormKeep)) return refuse("gamma or row length of the norm");
+        if (rope && d->rotated_outputs) {
+            if (!t->cos || !t->sin) return fail(HIPATTN_INVALID_ARGUMENT, "projection: null pointer");
+            if (d->head_size < 8 || d->head_size % 8 != 0 || !float_type(d->table_dtype)) return refuse("head size or table type");
+            for (int i = 0; i < d->num_weights; i++)
+                if (((d->rotated_outputs >> i) & 1) && d->n[i] % d->head_size != 0) return refuse("rows of no whole heads");
+        }
+        if (!workspace || !aligned16(workspace) || workspace_bytes < (size_t)(d->rows * columns * 4)) return refuse("no workspace for the sums");
+        const Split split = split_of(d->rows, d->n, d->num_weights, d->k, workspace_bytes, false);
+        const MidRowsParams p = params_of(t->x, t->weights, t->outs, d->n, d->num_weights, d->rows, d->k, split, (float*)workspace);
+        if (bf16)
+            launch<true, false>(p, split.waves, stream);
+        else
+            launch<false, false>(p, split.waves, stream);
+        FinishParams f{};
+        f.sums = p.sums, f.m = p.m, f.columns = p.columns, f.parts = p.parts, f.dtype = d->dtype;
+        for (int i = 0; i < kMaxWeights; i++) {
+            f.out[i] = p.c[i], f.n[i] = p.n[i];
+            f.offset[i] = i < d->num_weights ? p.offset[i] : INT32_MAX;
+        }
+        if (add) {
+            f.residual = t->residual, f.gamma = t->gamma, f.normalised = t->normalised, f.gamma_dtype = d->gamma_dtype, f.eps = d->eps;
+        } else {
+            f.rotated = d->rotated_outputs, f.head_size = d->head_size, f.cos = t->cos, f.sin = t->sin, f.positions = t->positions;
+            f.table_row_stride = d->table_row_stride, f.table_dtype = d->table_dtype;
+        }
+        if (f.gamma)
+            hipLaunchKernelGGL(projection_norm_kernel, dim3((unsigned)p.m), dim3(kNormThreads), 0, stream, f);
+        else
+            hipLaunchKernelGGL(projection_finish_kernel, dim3((unsigned)((columns / 8 + 255) / 256), (unsigned)p.m), dim3(256), 0, stream, f);
+    }
+    if (const hipError_t e = hipGetLastError(); e != hipSuccess) return fail(HIPATTN_HIP_ERROR, "projection: %s", hipGetErrorString(e));
     return HIPATTN_OK;
 }
 

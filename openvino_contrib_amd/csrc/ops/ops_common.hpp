@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "hipops.h"
+#include "ops/projection.h"
 
 namespace hipops {
 
@@ -36,6 +37,8 @@ hipattn_status matmul_few_rows(const hipops_matmul_desc* d, const void* a, const
 bool matmul_mid_rows_supported(const hipops_matmul_desc* d, const void* a, const void* b, const void* c);
 hipattn_status matmul_mid_rows(const hipops_matmul_desc* d, const void* a, const void* b, void* c, void* workspace, size_t workspace_bytes,
                                hipStream_t stream);
+hipattn_status projection(const hipops_projection_desc* desc, const hipops_projection_args* tensors, void* workspace, size_t workspace_bytes,
+                          hipStream_t stream);
 hipattn_status matmul_workspace_size(const hipops_matmul_desc* desc, size_t* bytes);
 hipattn_status matmul(const hipops_matmul_desc* desc, const void* a, const void* b, void* c, void* workspace,
                       size_t workspace_bytes, hipStream_t stream);

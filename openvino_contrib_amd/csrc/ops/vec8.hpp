@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "device_common.hpp"
+#include "hipops.h"
 
 namespace hipops {
 
@@ -67,6 +68,15 @@ __device__ __forceinline__ void store8(void* base, int64_t idx, int dtype, const
                 raw[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, bf16x2_t));
         }
         *(uint4_t*)((uint16_t*)base + idx) = raw;
+    }
+}
+
+// the gated MLP's activations (HIPOPS_GLU_*)
+__device__ __forceinline__ float activate(float x, int activation, float beta) {
+    switch (activation) {
+        case HIPOPS_GLU_GELU: return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f));
+        case HIPOPS_GLU_GELU_TANH: return 0.5f * x * (1.0f + tanhf(0.79788456080286536f * (x + 0.044715f * x * x * x)));
+        default: return x / (1.0f + __expf(-beta * x));
     }
 }
 

@@ -8,9 +8,13 @@
 // RMS and RoPE, which the reference would receive unfused (VariadicSplit / Swish / Multiply,
 // Power / ReduceMean / Sqrt / Multiply, and Slice / Multiply / Concat / Add).  As everywhere in this plugin a constructor that throws is how
 // an unsupported node is reported (src/cuda_plugin.cpp:171-188).
+#include <algorithm>
 #include <cstring>
+#include <map>
+#include <set>
 
 #include "hip_operation.hpp"
+#include "../../ops/projection.h"
 #include "hipops.h"
 #include "openvino/op/concat.hpp"
 #include "openvino/op/constant.hpp"
@@ -76,6 +80,11 @@ public:
                           "gamma " + shape_str(in[1].shape) + " must hold one value per element of the last axis of " + shape_str(x));
         HIP_OPS_CHECK(hipops_rms_norm(in[0].device, in[1].device, out[0].device, (int64_t)(hidden ? ov::shape_size(x) / hidden : 0),
                                       (int64_t)hidden, eps_, x_dtype_, gamma_dtype_, out_dtype_, context.stream.get()));
+    }
+
+    bool describe_for_projection(Inputs in, hipops_projection_desc& d) const {
+        d.gamma_dtype = gamma_dtype_, d.eps = eps_;
+        return x_dtype_ == d.dtype && out_dtype_ == d.dtype && ov::shape_size(in[1].shape) == in[0].shape.back();
     }
 
 private:
@@ -202,6 +211,21 @@ public:
         }
     }
 
+    // Rotates whole heads of a [tokens, heads * size] input by halves, a table row for each token or position: what a projection's
+    // epilogue does.  Fills in the descriptor, or false.
+    bool describe_for_projection(Inputs in, hipops_projection_desc& d) const {
+        if (rank_ != 2 || cfg_.is_interleaved || cfg_.slice_start != 0 || dtype_ != d.dtype) return false;
+        const Geometry g = geometry(in[0].shape);
+        const ov::Shape& cs = in[1].shape;
+        if (in[0].shape.back() != g.heads * g.size || (cfg_.rotary_ndims != 0 && cfg_.rotary_ndims != g.size) || cs.empty() || cs.back() != g.size ||
+            in[2].shape != cs)
+            return false;
+        if (has_positions_ ? ov::shape_size(in[3].shape) != g.length : ov::shape_size(cs) / g.size != g.length) return false;
+        d.head_size = (int)g.size, d.table_dtype = table_dtype_, d.table_row_stride = (int64_t)g.size;
+        return true;
+    }
+    bool has_positions() const { return has_positions_; }
+
 private:
     ov::op::internal::RoPE::Config cfg_;
     size_t num_inputs_ = 3, rank_ = 4;
@@ -277,6 +301,9 @@ public:
         const size_t ws_bytes = wb.mutable_sizes.empty() ? 0 : wb.mutable_sizes[0];
         HIP_OPS_CHECK(hipops_matmul(&d, in[0].device, in[1].device, out[0].device, ws, ws_bytes, context.stream.get()));
     }
+
+    // x [rows, k] times weights stored [n, k], 16-bit throughout
+    bool is_projection() const { return !transpose_a_ && transpose_b_ && ab_dtype_ == c_dtype_ && ab_dtype_ != HIPATTN_F32; }
 
 private:
     int ab_dtype_ = 0, c_dtype_ = 0;
@@ -445,13 +472,151 @@ public:
         HIP_OPS_CHECK(hipops_glu(in[0].device, out[0].device, rows, width_, activation_, gate_first_, dtype_, context.stream.get()));
     }
 
+    bool describe_for_projection(hipops_projection_desc& d) const {
+        d.glu_activation = activation_, d.glu_gate_first = gate_first_;
+        return dtype_ == d.dtype;
+    }
+
 private:
     int dtype_ = 0, activation_ = 0;
     int64_t width_ = 0;
     bool gate_first_ = true;
 };
 
+// ------------------------------------------------------------------------------ projections with what follows them
+// The MatMuls of one input (q, k and v) and the RoPEs of their results; or one MatMul with the Add of a residual and the RMS norm of
+// that; or one MatMul with the GLU of its result.  Nothing else reads what is between, which is then not written.
+class ProjectionGroup : public OperationGroup {
+public:
+    int kind = HIPOPS_PROJECTION_ROPE;
+    std::vector<const MatMulOp*> products;
+    std::vector<size_t> product_at;                        // position of each in steps()
+    const RopeOp* rope[3] = {nullptr, nullptr, nullptr};  // of product i
+    size_t rope_at[3] = {0, 0, 0};
+    const GluOp* glu = nullptr;
+    const RmsOp* norm = nullptr;
+    size_t residual_input = 0;  // of the Add
+    void add(size_t step) { steps_.push_back(step); }
+
+    bool Execute(const InferenceRequestContext& context, const std::vector<Tensors>& t) const override {
+        hipops_projection_desc d{};
+        hipops_projection_args a{};
+        d.kind = kind, d.num_weights = (int)products.size();
+        for (size_t i = 0; i < products.size(); i++) {
+            const auto& in = *t[product_at[i]].in;
+            const hipops_matmul_desc m = products[i]->describe(in, nullptr);
+            if (m.batch != 1 || m.m < 1 || m.m > 64) return false;
+            d.dtype = m.ab_dtype, d.rows = m.m, d.k = m.k, d.n[i] = m.n;
+            a.x = in[0].device, a.weights[i] = in[1].device, a.outs[i] = (*t[product_at[i]].out)[0].device;
+        }
+        if (kind == HIPOPS_PROJECTION_ROPE) {
+            for (size_t i = 0; i < products.size(); i++) {
+                if (!rope[i]) continue;
+                const auto& in = *t[rope_at[i]].in;
+                const int head_size = d.head_size;
+                if (!rope[i]->describe_for_projection(in, d) || (head_size && head_size != d.head_size)) return false;
+                d.rotated_outputs |= 1 << i;
+                a.outs[i] = (*t[rope_at[i]].out)[0].device;
+                a.cos = in[1].device, a.sin = in[2].device, a.positions = rope[i]->has_positions() ? (const int32_t*)in[3].device : nullptr;
+            }
+        } else if (kind == HIPOPS_PROJECTION_GLU) {
+            if (!glu->describe_for_projection(d)) return false;
+            a.outs[0] = (*t[1].out)[0].device;
+        } else {
+            const auto& in = *t[1].in;
+            if (in[0].shape != in[1].shape || in[0].type != (*t[0].out)[0].type || in[1].type != in[0].type) return false;
+            a.residual = in[residual_input].device, a.outs[0] = (*t[1].out)[0].device;
+            if (norm) {
+                if (!norm->describe_for_projection(*t[2].in, d)) return false;
+                a.gamma = (*t[2].in)[1].device, a.normalised = (*t[2].out)[0].device;
+            }
+        }
+        const Workbuffers& wb = *t[0].workbuffers;
+        if (wb.mutable_buffers.empty()) return false;
+        const hipattn_status st = hipops_projection(&d, &a, wb.mutable_buffers[0], wb.mutable_sizes[0], context.stream.get());
+        if (st == HIPATTN_UNSUPPORTED) return false;
+        HIP_OPS_CHECK(st);
+        return true;
+    }
+};
+
 }  // namespace
+
+std::vector<std::shared_ptr<OperationGroup>> find_projection_groups(const std::vector<const OperationBase*>& sequence) {
+    std::map<TensorID, std::vector<size_t>> readers;
+    for (size_t i = 0; i < sequence.size(); i++)
+        for (TensorID id : sequence[i]->GetInputIds()) readers[id].push_back(i);
+    const auto only_reader = [&](TensorID id, size_t step) { return readers[id].size() == 1 && readers[id][0] == step; };
+    const auto next = [&](size_t i) {
+        for (i++; i < sequence.size(); i++)
+            if (sequence[i]->GetTypeName() != "Parameter" && sequence[i]->GetTypeName() != "Constant") break;
+        return i;
+    };
+    const auto as_projection = [&](size_t i) -> const MatMulOp* {
+        const auto* mm = i < sequence.size() ? dynamic_cast<const MatMulOp*>(sequence[i]) : nullptr;
+        return mm && mm->is_projection() ? mm : nullptr;
+    };
+    std::vector<std::shared_ptr<OperationGroup>> groups;
+    for (size_t i = 0; i < sequence.size(); i++) {
+        const MatMulOp* const first = as_projection(i);
+        if (!first) continue;
+        const TensorID x = first->GetInputIds()[0], y = first->GetOutputIds()[0];
+        auto g = std::make_shared<ProjectionGroup>();
+        const auto take_product = [&](size_t step) {
+            g->product_at.push_back(g->steps().size());
+            g->products.push_back(as_projection(step));
+            g->add(step);
+        };
+        take_product(i);
+        const size_t then = next(i);
+        if (then < sequence.size() && sequence[then]->GetTypeName() == "Add" && only_reader(y, then)) {
+            g->kind = HIPOPS_PROJECTION_ADD;
+            g->residual_input = sequence[then]->GetInputIds()[0] == y ? 1 : 0;
+            g->add(then);
+            const size_t last = next(then);
+            const auto* rms = last < sequence.size() ? dynamic_cast<const RmsOp*>(sequence[last]) : nullptr;
+            if (rms && rms->GetInputIds()[0] == sequence[then]->GetOutputIds()[0]) g->norm = rms, g->add(last);
+        } else if (const auto* glu = then < sequence.size() ? dynamic_cast<const GluOp*>(sequence[then]) : nullptr; glu && only_reader(y, then)) {
+            g->kind = HIPOPS_PROJECTION_GLU;
+            g->glu = glu;
+            g->add(then);
+        } else {
+            const RopeOp* any = nullptr;  // (all of a group turn by one table)
+            for (size_t step = then; step < sequence.size(); step = next(step)) {
+                if (const MatMulOp* mm = as_projection(step); mm && g->products.size() < 3 && mm->GetInputIds()[0] == x && mm->GetInputIds()[1] != x) {
+                    take_product(step);
+                    continue;
+                }
+                const auto* rope = dynamic_cast<const RopeOp*>(sequence[step]);
+                size_t of = 0;
+                while (rope && of < g->products.size() && g->products[of]->GetOutputIds()[0] != rope->GetInputIds()[0]) of++;
+                if (!rope || of == g->products.size() || !only_reader(rope->GetInputIds()[0], step)) break;
+                if (any && (any->GetInputIds().size() != rope->GetInputIds().size() ||
+                            !std::equal(any->GetInputIds().begin() + 1, any->GetInputIds().end(), rope->GetInputIds().begin() + 1) ||
+                            any->has_positions() != rope->has_positions()))
+                    break;
+                any = rope;
+                g->rope[of] = rope, g->rope_at[of] = g->steps().size();
+                g->add(step);
+            }
+        }
+        if (g->steps().size() < 2) continue;
+        // nothing that a group reads beside its chain may come from within it (a weight computed by a neighbour)
+        std::set<TensorID> made;
+        for (size_t step : g->steps())
+            for (TensorID id : sequence[step]->GetOutputIds()) made.insert(id);
+        bool closed = true;
+        for (size_t k = 0; k < g->steps().size(); k++) {
+            const auto& ids = sequence[g->steps()[k]]->GetInputIds();
+            const size_t chain = g->kind == HIPOPS_PROJECTION_ADD && k == 1 ? 1 - g->residual_input : 0;
+            for (size_t n = 0; n < ids.size(); n++) closed = closed && (n == chain || !made.count(ids[n]));
+        }
+        if (!closed) continue;
+        groups.push_back(g);
+        i = g->steps().back();
+    }
+    return groups;
+}
 
 }  // namespace hip_gpu
 }  // namespace ov

@@ -148,6 +148,27 @@ protected:
     const IndexCollection output_ids_;
 };
 
+// Neighbouring operators that one call serves for some shapes (projections of few rows with what follows them).  The request
+// decides nothing: it asks the group at its last step and, where the group declines, runs the steps one by one.
+class OperationGroup {
+public:
+    struct Tensors {
+        const std::vector<TensorView>* in;
+        const std::vector<TensorView>* out;
+        const Workbuffers* workbuffers;
+    };
+    virtual ~OperationGroup() = default;
+    // steps of the execution sequence, ascending, nothing but Parameters and Constants between them
+    const std::vector<size_t>& steps() const { return steps_; }
+    // Enqueues all of it, or nothing (false).  tensors: of the steps, in their order.
+    virtual bool Execute(const InferenceRequestContext& context, const std::vector<Tensors>& tensors) const = 0;
+
+protected:
+    std::vector<size_t> steps_;
+};
+// the groups of a sequence (hip_layer_ops.cpp); a step is in one at most
+std::vector<std::shared_ptr<OperationGroup>> find_projection_groups(const std::vector<const OperationBase*>& sequence);
+
 class OperationRegistry final {
 public:
     using IndexCollection = OperationBase::IndexCollection;

@@ -475,6 +475,12 @@ CompiledModel::CompiledModel(const std::shared_ptr<const ov::Model>& model, cons
         auto op = OperationRegistry::getInstance().createOperation(ctx, node, std::move(in), std::move(out));
         exec_sequence_.push_back({node, op});
     }
+    std::vector<const OperationBase*> operators;
+    for (const auto& step : exec_sequence_) operators.push_back(step.op.get());
+    groups_ = find_projection_groups(operators);
+    group_of_step_.assign(exec_sequence_.size(), -1);
+    for (size_t g = 0; g < groups_.size(); g++)
+        for (size_t step : groups_[g]->steps()) group_of_step_[step] = (int)g;
     // outputs nothing consumes (neither an operator nor a Result) need not be produced
     std::set<std::pair<const ov::Node*, size_t>> consumed;
     for (const auto& node : ordered)
@@ -835,9 +841,13 @@ void InferRequest::prepare_steps(const ThreadContext& thread_context, const Infe
             ps.out.push_back(v);
             continue;
         }
+        // (a group runs as a whole at its last step, and its results may be written before the last of its inputs is read)
+        const int group = compiled_->group_of(si);
+        const int begins = group < 0 ? (int)si : (int)compiled_->groups()[group]->steps().front();
+        const int ends = group < 0 ? (int)si : (int)compiled_->groups()[group]->steps().back();
         for (TensorID id : step.op->GetInputIds()) {
             ps.in.push_back(views_[id]);
-            last_use[owner[id]] = std::max(last_use[owner[id]], (int)si);
+            last_use[owner[id]] = std::max(last_use[owner[id]], ends);
         }
         const std::vector<ov::Shape> out_shapes = step.op->InferOutputShapes(ps.in, context);
         for (size_t o = 0; o < out_ids.size(); o++) {
@@ -860,7 +870,8 @@ void InferRequest::prepare_steps(const ThreadContext& thread_context, const Infe
                 v.host = host;
                 if (v.byte_size() && constants_on_device_.insert(out_ids[o]).second) stream.upload(v.device, host, v.byte_size());
             } else {
-                packed.push_back({out_ids[o], std::max<size_t>(v.byte_size(), 16), (int)si});
+                packed.push_back({out_ids[o], std::max<size_t>(v.byte_size(), 16), begins});
+                last_use[out_ids[o]] = std::max(last_use[out_ids[o]], ends);
             }
             ps.out.push_back(v);
             views_[out_ids[o]] = v;
@@ -926,9 +937,8 @@ void InferRequest::prepare_steps(const ThreadContext& thread_context, const Infe
 
 void InferRequest::execute_steps(const InferenceRequestContext& context, bool profiling) {
     const auto& sequence = compiled_->exec_sequence();
-    for (size_t si = 0; si < sequence.size(); si++) {
+    const auto run = [&](size_t si) {
         const auto& step = sequence[si];
-        if (ov::as_type<const ov::op::v0::Parameter>(step.node.get())) continue;
         if (cancellation_.is_cancelled()) throw ov::Cancelled("Infer Request was canceled");
         if (profiling) {
             ev_begin_.emplace_back(new Event());
@@ -939,6 +949,21 @@ void InferRequest::execute_steps(const InferenceRequestContext& context, bool pr
         step.op->Execute(context, prepared_[si].in, prepared_[si].out, prepared_[si].workbuffers);
         for (const auto& c : prepared_[si].copies) context.stream.transfer(c.to, c.from, c.bytes);
         if (profiling) ev_end_.back()->record(context.stream);
+    };
+    for (size_t si = 0; si < sequence.size(); si++) {
+        if (ov::as_type<const ov::op::v0::Parameter>(sequence[si].node.get())) continue;
+        const int index = profiling ? -1 : compiled_->group_of(si);  // (timed operators run each by itself)
+        if (index < 0) {
+            run(si);
+            continue;
+        }
+        const OperationGroup& group = *compiled_->groups()[index];
+        if (si != group.steps().back()) continue;
+        if (cancellation_.is_cancelled()) throw ov::Cancelled("Infer Request was canceled");
+        std::vector<OperationGroup::Tensors> tensors;
+        for (size_t s : group.steps()) tensors.push_back({&prepared_[s].in, &prepared_[s].out, &prepared_[s].workbuffers});
+        if (group.Execute(context, tensors)) continue;
+        for (size_t s : group.steps()) run(s);
     }
 }
 

@@ -178,6 +178,9 @@ public:
         OperationBase::Ptr op;
     };
     const std::vector<ExecStep>& exec_sequence() const { return exec_sequence_; }
+    // operators that one call may serve; group_of: the index of a step's, -1 for none
+    const std::vector<std::shared_ptr<OperationGroup>>& groups() const { return groups_; }
+    int group_of(size_t step) const { return group_of_step_[step]; }
     size_t num_tensors() const { return num_tensors_; }
     const std::vector<TensorID>& output_ids(const ov::Node* node) const { return output_ids_.at(node); }
     // no consumer of this tensor reads it on the device (OperationBase::InputIsHostOnly)
@@ -200,6 +203,8 @@ private:
     std::shared_ptr<ov::threading::ITaskExecutor> wait_executor_;
     bool loaded_from_cache_;
     std::vector<ExecStep> exec_sequence_;
+    std::vector<std::shared_ptr<OperationGroup>> groups_;
+    std::vector<int> group_of_step_;
     std::map<const ov::Node*, std::vector<TensorID>> output_ids_;  // per node: one TensorID per output port
     std::set<TensorID> host_only_tensors_;
     std::set<TensorID> advisory_value_tensors_;

@@ -52,6 +52,18 @@ class MatmulDesc(ctypes.Structure):
     ]
 
 
+class ProjectionDesc(ctypes.Structure):
+    _fields_ = [("kind", _i), ("dtype", _i), ("num_weights", _i), ("rotated_outputs", _i), ("head_size", _i), ("table_dtype", _i), ("gamma_dtype", _i),
+                ("eps", _f), ("glu_activation", _i), ("glu_gate_first", _i), ("rows", _i64), ("k", _i64), ("n", _i64 * 3), ("table_row_stride", _i64)]
+
+
+class ProjectionArgs(ctypes.Structure):
+    _fields_ = [("x", _vp), ("weights", _vp * 3), ("outs", _vp * 3), ("cos", _vp), ("sin", _vp), ("positions", _vp), ("residual", _vp), ("gamma", _vp),
+                ("normalised", _vp)]
+
+
+PROJECTION_ROPE, PROJECTION_ADD, PROJECTION_GLU = 0, 1, 2
+
 SYMBOLS = {
     "hipops_last_error_string": (ctypes.c_char_p, []),
     "hipops_version": (_i, []),
@@ -126,6 +138,19 @@ def matmul_workspace_size(desc):
 def matmul(desc, a, b, c, workspace=None, stream=None):
     check(lib().hipops_matmul(ctypes.byref(desc), _ptr(a), _ptr(b), _ptr(c), _ptr(workspace),
                               workspace.nbytes if workspace is not None else 0, _h(stream)))
+
+
+def projection(kind, dtype, rows, k, n, x, weights, outs, workspace=None, stream=None, rotated=0, head_size=0, table_dtype=0, table_row_stride=0,
+               cos=None, sin=None, positions=None, residual=None, gamma=None, gamma_dtype=0, normalised=None, eps=0.0, activation=0, gate_first=True):
+    """One to three products of x with weights [n[i], k], and a rotary embedding, a residual (and its RMS norm) or a GLU behind them."""
+    address = lambda b: _vp(0) if b is None else b.ptr
+    three = lambda bs: (_vp * 3)(*[address(bs[i] if i < len(bs) else None) for i in range(3)])
+    d = ProjectionDesc(kind, dtype, len(n), rotated, head_size, table_dtype, gamma_dtype, eps, activation, int(gate_first), rows, k,
+                       (_i64 * 3)(*n), table_row_stride)
+    a = ProjectionArgs(address(x), three(weights), three(outs), *[address(b) for b in (cos, sin, positions, residual, gamma, normalised)])
+    entry = lib().hipops_projection  # (not of the public header: the plugin's)
+    entry.restype, entry.argtypes = _i, [_P(ProjectionDesc), _P(ProjectionArgs), _vp, _sz, _vp]
+    check(entry(ctypes.byref(d), ctypes.byref(a), _ptr(workspace), workspace.nbytes if workspace is not None else 0, _h(stream)))
 
 
 GLU_SWISH, GLU_GELU, GLU_GELU_TANH = 0, 1, 2

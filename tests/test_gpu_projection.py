@@ -1,0 +1,140 @@
+"""Projections of few rows with what follows them (hipops_projection) against the oracle's operators one after the other, and the
+plugin's groups against the same model run operator by operator.
+Bounds: one rounding of the result and 1e-6 sqrt(k) for the fp32 sum of k products (three times that behind the SwiGLU, whose slope
+stays below 1.1 and whose factors reach 2.5 here); the norm divides by a root mean square that carries the sum's error once more, and is
+taken of the rounded sum, of which the last bit may fall either way: one more rounding."""
+import numpy as np
+import pytest
+
+import openvino_contrib_amd.plugin_capi as P
+from openvino_contrib_amd import device_case as H
+from test_gpu_layer_ops import BF16, F16, F32, ROUND, download, ops, rope_tables, scaled_error, upload  # noqa: F401
+from test_gpu_plugin_layer import storage
+
+pytestmark = pytest.mark.gpu
+
+
+def _weights(hip, rng, n, k, dtype):
+    return [upload(hip, rng.standard_normal((x, k)) / np.sqrt(k), dtype) for x in n]
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("m,n,k,head,rotated", [(1, (64, 64, 64), 64, 64, 3), (4, (4096, 1024, 1024), 4096, 128, 3), (16, (256, 64, 64), 704, 64, 1),
+                                                (17, (512, 128), 320, 128, 2), (64, (1024, 256, 256), 1024, 128, 3), (33, (192,), 192, 24, 1),
+                                                (5, (104, 8), 128, 8, 0)])
+def test_products_with_rotary_embedding(hip, ops, oracle, m, n, k, head, rotated, dtype):  # noqa: F811
+    rng = np.random.default_rng(m + k)
+    dx, x = upload(hip, rng.standard_normal((m, k)), dtype)
+    w = _weights(hip, rng, n, k, dtype)
+    cos, sin = rope_tables(rng, 2 * m + 3, head, False, head)
+    positions = rng.permutation(2 * m + 3)[:m].astype(np.int32)
+    dcos, dsin, dpos = (hip.DeviceBuffer.from_numpy(t) for t in (cos.astype(np.float32), sin.astype(np.float32), positions))
+    workspace = hip.DeviceBuffer(32 << 20)
+    for with_positions in (True, False):
+        outs = [hip.DeviceBuffer(m * i * 2) for i in n]
+        for o in outs:
+            o.fill(0xFF)
+        ops.projection(ops.PROJECTION_ROPE, dtype, m, k, n, dx, [b for b, _ in w], outs, workspace, rotated=rotated, head_size=head, table_dtype=F32,
+                       table_row_stride=head, cos=dcos, sin=dsin, positions=dpos if with_positions else None)
+        for i, size in enumerate(n):
+            ref = oracle.matmul(x, w[i][1], False, True)
+            if (rotated >> i) & 1:
+                ref = oracle.rope(ref.reshape(m, size // head, head), cos, sin, positions if with_positions else None).reshape(m, size)
+            assert scaled_error(download(hip, outs[i], dtype, (m, size)), ref) <= ROUND[dtype] + 2e-6 * np.sqrt(k)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("m,n,k", [(1, 8, 64), (4, 4096, 4096), (15, 1000, 448), (64, 4096, 1024), (33, 16384, 128), (49, 264, 5376)])
+def test_product_residual_and_norm(hip, ops, oracle, m, n, k, dtype):  # noqa: F811
+    rng = np.random.default_rng(m + n + k)
+    dx, x = upload(hip, rng.standard_normal((m, k)), dtype)
+    (dw, w), = _weights(hip, rng, (n,), k, dtype)
+    dr, r = upload(hip, rng.standard_normal((m, n)), dtype)
+    dg, g = upload(hip, 1 + 0.1 * rng.standard_normal(n), dtype)
+    workspace = hip.DeviceBuffer(32 << 20)
+    ref = oracle.matmul(x, w, False, True) + r
+    for norm in (True, False):
+        out, normalised = hip.DeviceBuffer(m * n * 2), hip.DeviceBuffer(m * n * 2)
+        out.fill(0xFF), normalised.fill(0xFF)
+        ops.projection(ops.PROJECTION_ADD, dtype, m, k, (n,), dx, [dw], [out], workspace, residual=dr, gamma=dg if norm else None, gamma_dtype=dtype,
+                       normalised=normalised if norm else None, eps=1e-5)
+        assert scaled_error(download(hip, out, dtype, (m, n)), ref) <= ROUND[dtype] + 1e-6 * np.sqrt(k)
+        if norm:
+            assert scaled_error(download(hip, normalised, dtype, (m, n)), oracle.rms_norm(ref, g, 1e-5)) <= 3 * ROUND[dtype] + 2e-6 * np.sqrt(k)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("m,width,k,activation,gate_first", [(1, 4, 64, 0, True), (4, 14336, 4096, 0, True), (16, 100, 320, 1, False), (33, 1376, 512, 2, True),
+                                                             (64, 11008, 256, 0, False), (20, 44, 704, 0, True)])
+def test_product_and_glu(hip, ops, oracle, m, width, k, activation, gate_first, dtype):  # noqa: F811
+    rng = np.random.default_rng(m + width + k)
+    dx, x = upload(hip, rng.standard_normal((m, k)), dtype)
+    (dw, w), = _weights(hip, rng, (2 * width,), k, dtype)
+    out = hip.DeviceBuffer(m * width * 2)
+    out.fill(0xFF)
+    ops.projection(ops.PROJECTION_GLU, dtype, m, k, (2 * width,), dx, [dw], [out], activation=activation, gate_first=gate_first)
+    ref = oracle.glu(oracle.matmul(x, w, False, True), activation, gate_first)
+    assert scaled_error(download(hip, out, dtype, (m, width)), ref) <= ROUND[dtype] + 3e-6 * np.sqrt(k)
+
+
+def test_what_the_kernels_do_not_take_is_refused(hip, ops):  # noqa: F811
+    buf, ws = hip.DeviceBuffer(1 << 20), hip.DeviceBuffer(1 << 20)
+    for kwargs, status in ((dict(rows=65), hip.UNSUPPORTED), (dict(k=96), hip.UNSUPPORTED), (dict(n=(12,)), hip.UNSUPPORTED), (dict(dtype=F32), hip.UNSUPPORTED),
+                           (dict(workspace=None), hip.UNSUPPORTED), (dict(residual=None), hip.INVALID_ARGUMENT), (dict(kind=7), hip.INVALID_ARGUMENT),
+                           (dict(gamma=buf, normalised=None), hip.INVALID_ARGUMENT)):
+        call = dict(dict(kind=ops.PROJECTION_ADD, dtype=BF16, rows=8, k=64, n=(64,), x=buf, weights=[buf], outs=[buf], workspace=ws, residual=buf), **kwargs)
+        with pytest.raises(ops.HipOpsError) as e:
+            ops.projection(**call)
+        assert e.value.status == status, kwargs
+
+
+def _model(tokens, hidden, ffn, heads, kv_heads, size, extra_reader):
+    """norm -> q, k, v -> RoPE of q and k -> (their parts put together, as far as they are wide) -> o -> Add -> norm -> gate|up -> GLU -> down -> Add."""
+    rng = np.random.default_rng(tokens + hidden)
+    g = P.GraphText("projections")
+    const = lambda name, shape, std: g.constant(name, storage(rng.standard_normal(shape) * std, BF16)[0], "bf16")
+    weight = lambda name, rows, cols: const(name, (rows, cols), cols ** -0.5)
+    mm = lambda name, x, w: g.add("MatMul", name, [x, w], transpose_a=False, transpose_b=True)
+    rms = lambda name, x: g.add("RMS", name, [x, const(name + "_gamma", (hidden,), 1.0)], epsilon=1e-5, output_type="dynamic")
+    x = g.parameter("x", BF16, [-1, hidden])
+    cos, sin, pos = g.parameter("cos", F32, [-1, size]), g.parameter("sin", F32, [-1, size]), g.parameter("positions", P.I32, [-1])
+    n1 = rms("norm1", x)
+    q, k, v = (mm(n, n1, weight("w" + n, h * size, hidden)) for n, h in (("q", heads), ("k", kv_heads), ("v", kv_heads)))
+    rope = dict(head_size=size, rotary_ndims=size, gather_position_arg_id=3)
+    qr = g.add("RoPE", "rope_q", [q, cos, sin, pos], head_cnt=heads, **rope)
+    kr = g.add("RoPE", "rope_k", [k, cos, sin, pos], head_cnt=kv_heads, **rope)
+    kv = g.add("Multiply", "kv", [kr, v])
+    if extra_reader:
+        g.result("q_before", q)  # (read outside: what is between must be written)
+    o = g.add("Add", "residual1", [mm("o", qr, weight("wo", hidden, heads * size)), x])
+    act = g.add("GLU", "glu", [mm("gate_up", rms("norm2", o), weight("wgu", 2 * ffn, hidden))], axis=-1, split_lengths=ffn, glu_type=0, split_to_glu_idx=0,
+                output_type="dynamic")
+    g.result("out", g.add("Add", "residual2", [o, mm("down", act, weight("wd", hidden, ffn))]))
+    g.result("kv_out", kv)
+    return g.model()
+
+
+@pytest.mark.parametrize("extra_reader", [False, True])
+@pytest.mark.parametrize("hidden,ffn,heads,kv_heads,size", [(256, 704, 4, 2, 64), (384, 320, 3, 3, 128)])
+def test_groups_of_the_plugin(hip, extra_reader, hidden, ffn, heads, kv_heads, size):
+    """One compiled model over batches that a group takes, declines and takes again (the third and fourth infer of a size replay a graph),
+    against the operators one by one (a model compiled for profiling).  Both round to bf16 at most eleven times on the way to an output;
+    the norms keep every intermediate at one or below, so that three roundings' worth is ample."""
+    plugin, timed = P.Plugin(), P.Plugin()
+    timed.set_property("PERF_COUNT", "YES")
+    text = _model(0, hidden, ffn, heads, kv_heads, size, extra_reader)
+    requests = [p.compile_model(text).create_infer_request() for p in (plugin, timed)]
+    rng = np.random.default_rng(1)
+    for tokens in (1, 6, 7, 64, 65, 33, 64):
+        x = storage(rng.standard_normal((tokens, hidden)), BF16)[0]
+        cos, sin = rope_tables(rng, tokens + 9, size, False, size)
+        pos = rng.permutation(tokens + 9)[:tokens].astype(np.int32)
+        results = []
+        for request in requests:
+            for _ in range(4):
+                for i, value in enumerate(((x, BF16), (cos.astype(np.float32), F32), (sin.astype(np.float32), F32), (pos, P.I32))):
+                    request.set_input(i, *value)
+                request.infer()
+            results.append([H.storage_to_f32(request.output(i)[0], BF16) for i in range(3 if extra_reader else 2)])
+        for got, ref in zip(*results):
+            assert np.isfinite(ref).all() and scaled_error(got, ref) <= 6 * ROUND[BF16], tokens
