@@ -151,6 +151,7 @@ private:
     std::mutex mutex_;
     std::condition_variable wake_;
     std::deque<ov::threading::Task> queue_;
+    std::atomic<size_t> queued_{0};  // of queue_, to be looked at without the lock
     bool stopping_ = false;
     std::vector<std::thread> threads_;
 };
@@ -278,6 +279,7 @@ private:
     Graph graph_;
     size_t graph_launches_ = 0, graphs_captured_ = 0;
     bool graph_allowed_ = false;
+    bool outlasts_its_launches() const;
     std::vector<uint64_t> make_signature() const;
     void prepare_steps(const ThreadContext& thread_context, const InferenceRequestContext& context);
     void execute_steps(const InferenceRequestContext& context, bool profiling);
