@@ -149,4 +149,20 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// two bytes of a word (selected by `sel`) as fp16 numbers 1024 + byte
+__device__ __forceinline__ half2_t biased_half2(uint32_t w, uint32_t sel) {
+    return __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, w, sel));
+}
+// 8 payload bytes -> 8 dequantised fp16 values: (byte - zp) * scale, as (byte) * scale + off in
+// packed fp16 (1024 + byte is exact in fp16, and so is the subtraction of 1024)
+__device__ __forceinline__ uint4_t dequant8(uint2_t w, half2_t scale, half2_t off) {
+    const half2_t bias = {(half_t)1024.0f, (half_t)1024.0f};
+    uint4_t r;
+    r[0] = __builtin_bit_cast(uint32_t, (biased_half2(w[0], 0x04010400u) - bias) * scale + off);
+    r[1] = __builtin_bit_cast(uint32_t, (biased_half2(w[0], 0x04030402u) - bias) * scale + off);
+    r[2] = __builtin_bit_cast(uint32_t, (biased_half2(w[1], 0x04010400u) - bias) * scale + off);
+    r[3] = __builtin_bit_cast(uint32_t, (biased_half2(w[1], 0x04030402u) - bias) * scale + off);
+    return r;
+}
+
 }  // namespace hipattn

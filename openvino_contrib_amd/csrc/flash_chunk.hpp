@@ -148,22 +148,6 @@ struct U8Rows {
     float2 k_sz, v_sz;               // the rows' (scale, zero-point)
     int jk, jv;                      // tiles they belong to (-1: none)
 };
-// two bytes of a word (selected by `sel`) as fp16 numbers 1024 + byte
-__device__ __forceinline__ half2_t biased_half2(uint32_t w, uint32_t sel) {
-    return __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, w, sel));
-}
-// 8 payload bytes -> 8 dequantised fp16 values: (byte - zp) * scale, as (byte) * scale + off in
-// packed fp16 (1024 + byte is exact in fp16, and so is the subtraction of 1024)
-__device__ __forceinline__ uint4_t dequant8(uint2_t w, half2_t scale, half2_t off) {
-    const half2_t bias = {(half_t)1024.0f, (half_t)1024.0f};
-    uint4_t r;
-    r[0] = __builtin_bit_cast(uint32_t, (biased_half2(w[0], 0x04010400u) - bias) * scale + off);
-    r[1] = __builtin_bit_cast(uint32_t, (biased_half2(w[0], 0x04030402u) - bias) * scale + off);
-    r[2] = __builtin_bit_cast(uint32_t, (biased_half2(w[1], 0x04010400u) - bias) * scale + off);
-    r[3] = __builtin_bit_cast(uint32_t, (biased_half2(w[1], 0x04030402u) - bias) * scale + off);
-    return r;
-}
-
 // Keys [lo, hi) a tile has to visit, lo rounded down to a tile boundary.
 __device__ __forceinline__ void key_range(const Tile& t, int& lo, int& hi) {
     if (t.rows <= 0) {
@@ -1211,7 +1195,8 @@ __device__ __forceinline__ Tile paged_group_tile(const PagedParams& p, int s, in
 }
 
 // kPad: a head size between 64 and 128 (p.head_dim, a multiple of 8; 16-bit caches).
-template <bool kBf16, bool kU8, bool kPad>
+// kShadow: sequences that begin with this call take their rows from the prologue's dequantised copy (p.shadow_table), where there is one.
+template <bool kBf16, bool kU8, bool kPad, bool kShadow = false>
 __device__ __forceinline__ void paged_prefill_item(const PagedParams& p, int index, uint8_t* lds) {
     // Launch index (a workgroup's number on the device modulo 8) -> work item.  The workgroups that run on one XCD at a time should share K/V in
     // its L2, and the XCDs should get equal work although sequences differ in length.  With a
@@ -1253,6 +1238,24 @@ __device__ __forceinline__ void paged_prefill_item(const PagedParams& p, int ind
     if (!pair_heads && (qt & 1)) return;
     const Tile t0 = paged_group_tile<kPad>(p, s, qt, h0, true);
     const Tile t1 = pair_heads ? paged_group_tile<kPad>(p, s, qt, h0 + 1, true) : paged_group_tile<kPad>(p, s, qt + 1, h0, qt + 1 < tiles_s);
+    if constexpr (kShadow) {
+        const int begin = p.subsequence_begins[s], end = p.subsequence_begins[s + 1];
+        if (p.shadow_table != nullptr && p.past_lens[s] == 0 && end - begin >= kShadowTokens && begin >= 0 && end <= p.num_tokens &&
+            t0.table_len > 0) {
+            const int64_t block = shadow_block(begin, s, p.block_size), stride = (int64_t)p.num_heads_kv * p.block_size * kRowBytes;
+            const int64_t off = block * stride + (int64_t)hkv * p.block_size * kRowBytes;
+            const auto in_shadow = [&](Tile t) {
+                t.k = (const uint8_t*)p.shadow_k + off;
+                t.v = (const uint8_t*)p.shadow_v + off;
+                t.table = p.shadow_table + block;
+                t.num_blocks = t.table_len = min(t.table_len, (end - begin + p.block_size - 1) / p.block_size);
+                t.block_stride = stride;
+                return t;
+            };
+            run_both<false, false, true, 0, false>(in_shadow(t0), in_shadow(t1), lds, p.scale);
+            return;
+        }
+    }
     run_both<kBf16, kU8, true, 0, kPad>(t0, t1, lds, p.scale);
 }
 

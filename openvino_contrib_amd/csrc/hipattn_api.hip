@@ -502,7 +502,7 @@ HIPATTN_EXPORT hipattn_status hipattn_paged_attention_workspace_size(const hipat
     hipattn::PagedParams p = make_paged_params(desc);
     if (desc->flags & HIPATTN_PA_FORCE_GENERIC) return HIPATTN_OK;
     if (hipattn::paged_fast_supported(p))
-        *bytes = hipattn::paged_fast_workspace_bytes(p);
+        *bytes = hipattn::paged_fast_workspace_bytes(p) + hipattn::paged_shadow_bytes(p);
     else if (hipattn::paged_tiles_supported(p))  // (pointers are not known here: a call with unaligned ones needs none)
         *bytes = hipattn::paged_tiles_workspace_bytes(p);
     return HIPATTN_OK;
@@ -558,7 +558,7 @@ hipattn_status paged_attention_impl(const hipattn_pa_desc* desc, const void* q, 
     const bool forced_generic = (desc->flags & HIPATTN_PA_FORCE_GENERIC) != 0;
     if (!forced_generic && hipattn::paged_fast_supported(p)) {
         if (hipattn_status st = take_workspace(hipattn::paged_fast_workspace_bytes(p))) return st;
-        hipattn::paged_fast_plan(p, workspace);
+        hipattn::paged_fast_plan(p, workspace, workspace_bytes);
         g_kernel_path = "paged_mfma";
         HIP_TRY(hipattn::launch_paged_fast(p, do_write ? &w : nullptr, as_stream(stream), g_probe));
     } else if (!forced_generic && hipattn::paged_tiles_supported(p)) {

@@ -32,6 +32,10 @@ struct KvWriteParams {
     // head size 128, 16-bit new rows, 16-byte aligned pointers (set by kv_write_wavefronts): a
     // wavefront writes four kv heads of a token with 16-byte loads
     int vector_rows;
+    // nullptr, or where the rows of sequences that begin with this call also go, quantised and back to fp16 (PagedParams)
+    uint16_t* shadow_k;
+    uint16_t* shadow_v;
+    int32_t* shadow_table;
 };
 
 // The operator's cache rotation: the key rows of the listed blocks turned by the angles of their table rows.
@@ -150,8 +154,20 @@ struct PagedParams {
                           // chunked-prefill kernel too (HIPATTN_PA_ANY_LENGTHS); without it such a batch is
                           // planned per token and every token is a decode row
     int no_side_stream;   // mixed batches run one kernel after the other on the caller's stream
+    // u8 caches, nullptr or: what the writer left of the new rows of sequences without cached tokens and with kShadowTokens or more, as a chunk
+    // kernel finds them in the cache but in fp16 -- [blocks, num_heads_kv, block_size, head_dim], a sequence's blocks from shadow_block()
+    // on, and a block table that counts from there (-1: the cache's table names no block, whose rows are zeros here)
+    uint16_t* shadow_k;
+    uint16_t* shadow_v;
+    int32_t* shadow_table;
     int tiles_only;       // (flash_small.hip) tile_prefix counts single-token sequences too: there are no decode rows
 };
+
+// A shorter prompt is read by few query tiles and costs the writer as much (32 heads on 8, us without -> with: 8 prompts of 100 21.2 -> 23.0, of 300
+// 49.3 -> 49.8, of 500 66.3 -> 62.9, of 1,000 149 -> 132).
+constexpr int kShadowTokens = 384;
+// First block of a sequence in the shadow: blocks of sequences before it fill no more (begin, its first token; s, its number).
+__host__ __device__ inline int64_t shadow_block(int begin, int s, int block_size) { return (int64_t)(begin / block_size) + s; }
 
 // Optional event pair recorded around the dominant kernel of a call (measurement aid).
 struct KernelProbe {
@@ -192,7 +208,8 @@ bool paged_fast_supported(const PagedParams& p);
 // within the stream-K kernels' reach (paged_fast_supported of the result), else p as it is.
 PagedParams split_kv_heads(const PagedParams& p);
 size_t paged_fast_workspace_bytes(const PagedParams& p);
-void paged_fast_plan(PagedParams& p, void* workspace);  // fills chunking fields and workspace pointers
+size_t paged_shadow_bytes(const PagedParams& p);  // behind those, where the caller has them: the shadow of u8 chunks (0: none)
+void paged_fast_plan(PagedParams& p, void* workspace, size_t workspace_bytes);  // fills chunking fields and workspace pointers
 void release_side_stream(hipStream_t owner);  // drops the side stream mixed batches on `owner` used, if any
 // write == nullptr skips the KV-cache write of the new tokens
 hipError_t launch_paged_fast(const PagedParams& p, const KvWriteParams* write, hipStream_t stream,

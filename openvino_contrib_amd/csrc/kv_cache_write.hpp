@@ -27,10 +27,12 @@ __device__ __forceinline__ int locate_sequence(const int32_t* __restrict__ prefi
 // Where token t goes: physical block and position inside it; false when it has no valid target
 // (padding tokens outside every sequence, positions beyond the sequence's block table, block
 // numbers outside the pool).  A chain of dependent loads, done once per wavefront.
-__device__ __forceinline__ bool kv_write_slot(const KvWriteParams& p, int t, int lane, int& pb, int& pos) {
+// s: the token's sequence, -1 for a token outside every one.
+__device__ __forceinline__ bool kv_write_slot(const KvWriteParams& p, int t, int lane, int& pb, int& pos, int& s) {
+    s = -1;
     if (t >= p.num_tokens) return false;
     if (t < p.subsequence_begins[0] || t >= p.subsequence_begins[p.num_seqs]) return false;
-    const int s = locate_sequence(p.subsequence_begins, p.num_seqs, t, lane);
+    s = locate_sequence(p.subsequence_begins, p.num_seqs, t, lane);
     pos = p.past_lens[s] + (t - p.subsequence_begins[s]);
     if (pos < 0) return false;
     const int lb = pos / p.block_size;
@@ -38,6 +40,11 @@ __device__ __forceinline__ bool kv_write_slot(const KvWriteParams& p, int t, int
     if (lb >= p.block_indices_begins[s + 1] - tb0) return false;
     pb = p.block_indices[tb0 + lb];
     return pb >= 0 && pb < p.num_blocks;
+}
+
+__device__ __forceinline__ bool kv_write_slot(const KvWriteParams& p, int t, int lane, int& pb, int& pos) {
+    int s;
+    return kv_write_slot(p, t, lane, pb, pos, s);
 }
 
 __device__ __forceinline__ float bits16_to_float(uint32_t bits, int dtype) {
@@ -68,7 +75,7 @@ __device__ __forceinline__ float row16_reduce(float x) {
 // in the reduction, store nothing).  The arithmetic is that of the element-wise path below, value
 // for value (the quantiser's minimum and maximum do not depend on the order of the reduction).
 __device__ __forceinline__ void kv_store_row8(const KvWriteParams& p, uint4_t raw, uint8_t* row, int d0, bool active,
-                                              int lane) {
+                                              int lane, uint16_t* shadow = nullptr) {
     if (p.cache_dtype == p.kv_dtype) {
         if (active) *(uint4_t*)(row + d0 * 2) = raw;
         return;
@@ -100,6 +107,10 @@ __device__ __forceinline__ void kv_store_row8(const KvWriteParams& p, uint4_t ra
         if (active) {
             *(uint2_t*)(row + 8 + d0) = packed;
             if ((lane & 15) == 0) *(float2*)row = make_float2(scale, zp);
+            if (shadow != nullptr) {
+                const half_t sc = (half_t)scale, of = (half_t)(-zp * scale);
+                *(uint4_t*)(shadow + d0) = dequant8(packed, half2_t{sc, sc}, half2_t{of, of});
+            }
         }
     } else {  // the other 16-bit type
         uint4_t out;
@@ -119,17 +130,30 @@ __device__ __forceinline__ void kv_cache_write_rows128(const KvWriteParams& p, i
     const int t = (int)(wv / chunks);
     const int h = (int)(wv % chunks) * 4 + (lane >> 4);
     const int d0 = (lane & 15) * 8;
-    int pb = 0, pos = 0;
-    if (!kv_write_slot(p, t, lane, pb, pos)) return;  // wavefront-uniform
+    int pb = 0, pos = 0, s = -1;
+    const bool valid = kv_write_slot(p, t, lane, pb, pos, s);  // wavefront-uniform
     const bool active = h < p.num_heads_kv;
     const int hh = active ? h : 0;  // idle lanes follow head 0 and store nothing
+    uint16_t *sk = nullptr, *sv = nullptr;
+    if (p.shadow_table != nullptr && s >= 0 && p.past_lens[s] == 0) {
+        const int begin = p.subsequence_begins[s], lb = pos / p.block_size;
+        if (begin >= 0 && p.subsequence_begins[s + 1] - begin >= kShadowTokens && lb < p.block_indices_begins[s + 1] - p.block_indices_begins[s]) {
+            const int64_t block = shadow_block(begin, s, p.block_size) + lb;
+            const int64_t row = ((block * p.num_heads_kv + hh) * p.block_size + pos % p.block_size) * 128;
+            sk = p.shadow_k + row;
+            sv = p.shadow_v + row;
+            if (pos % p.block_size == 0 && wv % chunks == 0 && lane == 0) p.shadow_table[block] = valid ? lb : -1;
+            if (!valid && active) *(uint4_t*)(sk + d0) = *(uint4_t*)(sv + d0) = uint4_t{0u, 0u, 0u, 0u};
+        }
+    }
+    if (!valid) return;
     const int64_t src_off = ((int64_t)t * p.num_heads_kv + hh) * 128 + d0;
     const uint4_t kraw = *(const uint4_t*)((const uint16_t*)p.k_new + src_off);
     const uint4_t vraw = *(const uint4_t*)((const uint16_t*)p.v_new + src_off);
     const int64_t rb = cache_row_bytes(p.cache_dtype, 128);
     const int64_t row_off = (((int64_t)pb * p.num_heads_kv + hh) * p.block_size + pos % p.block_size) * rb;
-    kv_store_row8(p, kraw, p.key_cache + row_off, d0, active, lane);
-    kv_store_row8(p, vraw, p.value_cache + row_off, d0, active, lane);
+    kv_store_row8(p, kraw, p.key_cache + row_off, d0, active, lane, sk);
+    kv_store_row8(p, vraw, p.value_cache + row_off, d0, active, lane, sv);
 }
 
 // The K row and the V row of ONE (token, kv head) pair, head size 128, 16-bit new rows, written by

@@ -930,6 +930,21 @@ size_t paged_fast_workspace_bytes(const PagedParams& p) {
            align_up(slots * sizeof(uint64_t), 256);
 }
 
+// The chunks of a u8 batch read rows that the prologue has just quantised, 128 query rows at a time, and dequantise them through
+// registers in the phase that bounds the chunk kernel.  The rows of sequences without cached tokens are therefore kept in fp16 as
+// well, the values that dequantisation gives, at 5 us more for the prologue of 9,000 tokens.  Measured (us a step, 32 heads on 8, without -> with):
+// six prompts of 100 to 3,000 tokens 166 -> 149, two of 3,000 205 -> 181, one of 1,000 46 -> 40, eight of 512 beside 120 decode rows (64
+// heads) 283 -> 274.  Up to 256 MiB (65,536 tokens of 8 heads).
+static int64_t shadow_blocks(const PagedParams& p) { return (int64_t)(p.num_tokens / p.block_size) + p.num_seqs + 1; }
+
+size_t paged_shadow_bytes(const PagedParams& p) {
+    if (p.cache_dtype != HIPATTN_U8 || p.head_dim != 128 || !overlap_wanted(p) || !paged_mixed_supported(p)) return 0;
+    if (p.num_tokens < kShadowTokens || (p.max_context_len > 0 && p.max_context_len < kShadowTokens)) return 0;
+    const int64_t kv_heads = p.num_heads_kv / p.kv_share;
+    const size_t rows = (size_t)(shadow_blocks(p) * kv_heads * p.block_size) * 128 * sizeof(uint16_t);
+    return rows > (size_t)128 << 20 ? 0 : 256 + 2 * rows + align_up((size_t)shadow_blocks(p) * sizeof(int32_t), 256);
+}
+
 // A value no earlier call of this process used and that memory which was never written is unlikely to hold.
 static unsigned long long next_merge_tag() {
     static std::atomic<unsigned long long> counter{0};
@@ -942,8 +957,9 @@ static unsigned long long next_merge_tag() {
 }
 
 
-void paged_fast_plan(PagedParams& p, void* workspace) {
+void paged_fast_plan(PagedParams& p, void* workspace, size_t workspace_bytes) {
     const bool overlap = overlap_wanted(p);  // asks whether the caller fixed num_waves: before it is filled in
+    const size_t shadow = p.no_side_stream ? 0 : paged_shadow_bytes(p);
     p.overlap = overlap ? 1 : 0;
     const bool fixed_waves = p.num_waves > 0;
     p.num_waves = choose_num_waves(p, overlap);
@@ -977,6 +993,13 @@ void paged_fast_plan(PagedParams& p, void* workspace) {
     w += align_up(slots * G * 2 * sizeof(float), 256);
     p.part_flag = (uint64_t*)w;
     w += align_up(slots * sizeof(uint64_t), 256);
+    if (shadow > 0 && (size_t)(w - (uint8_t*)workspace) + shadow <= workspace_bytes) {
+        w += (256 - (uintptr_t)w % 256) % 256;
+        const size_t rows = (size_t)(shadow_blocks(p) * (p.num_heads_kv / p.kv_share) * p.block_size) * 128;
+        p.shadow_k = (uint16_t*)w;
+        p.shadow_v = p.shadow_k + rows;
+        p.shadow_table = (int32_t*)(p.shadow_v + rows);
+    }
     // the head-256 kernel and on-demand pieces (whose order of completion is not that of their numbers) keep the merge launch
     // Built into the u8 kernels only (see kFusedBuilt).  Measured, whole steps on one machine: the 128-sequence
     // u8 batch 0.437 ms fused against 0.440 ms with the merge launch.  Where many pieces share a segment the one wavefront that
@@ -1187,8 +1210,9 @@ static void launch_decode(const PagedParams& p, const KvWriteParams& wp, int do_
     }
 }
 
-hipError_t launch_paged_fast(const PagedParams& p, const KvWriteParams* write, hipStream_t stream,
+hipError_t launch_paged_fast(const PagedParams& params, const KvWriteParams* write, hipStream_t stream,
                              const KernelProbe& probe) {
+    PagedParams p = params;
     KvWriteParams wp{};
     int write_blocks = 0;
     if (write) {
@@ -1196,6 +1220,10 @@ hipError_t launch_paged_fast(const PagedParams& p, const KvWriteParams* write, h
         if (wp.head_dim > 256) return hipErrorInvalidValue;  // the fast path is head sizes up to 256 only
         write_blocks = (int)((kv_write_wavefronts(wp) + 3) / 4);
     }
+    if (wp.vector_rows)
+        wp.shadow_k = p.shadow_k, wp.shadow_v = p.shadow_v, wp.shadow_table = p.shadow_table;
+    else
+        p.shadow_table = nullptr;  // (nobody to fill it)
     hipError_t e = hipSuccess;
     // A pure decode batch of few rows is one launch less: the decode wavefronts plan for themselves
     // and write the new rows (see kSelfPlanMaxRows).

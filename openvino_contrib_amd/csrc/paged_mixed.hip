@@ -25,7 +25,7 @@ __global__ __launch_bounds__(flash::kThreads) __attribute__((amdgpu_waves_per_eu
     }
     p.num_heads_kv = chunk_heads_kv;
     p.kv_share = 1;
-    flash::paged_prefill_item<kBf16, kU8, kPad>(p, (int)blockIdx.x - decode_workgroups, lds);
+    flash::paged_prefill_item<kBf16, kU8, kPad, kU8>(p, (int)blockIdx.x - decode_workgroups, lds);
 }
 
 template <bool kU8, bool kBf16, bool kPad>

@@ -45,3 +45,30 @@ def test_mixed_batches_in_one_launch(hip, oracle, batch, cache, block, size, hea
     finally:
         capi.check(capi.lib().hipattn_set_option(b"mixed_overlap", -1))
     assert H.scaled_bound_error(out, alone, "against one kernel after the other") <= tol
+
+
+@pytest.mark.parametrize("block,heads", [(32, (8, 2)), (16, (3, 3)), (128, (8, 8)), (32, (48, 1))])
+@pytest.mark.parametrize("seqs", [[(0, 384)], [(0, 33), (0, 1), (0, 417), (5, 400), (0, 0), (0, 383), (200, 1), (0, 640)], [(0, 511), (64, 2), (0, 385), (0, 0), (0, 700)]])
+def test_new_prompts_read_the_rows_that_the_writer_quantised(hip, oracle, seqs, block, heads):
+    """u8 caches: sequences of 384 new tokens or more without cached ones take their rows from the writer's dequantised copy, others from the cache, in one call: the
+    chunk rows bit for bit those of the kernel that dequantises the cache's rows itself, with whole and missing table entries
+    (the first block of a sequence among them)."""
+    case = W.make_paged_case(5, seqs, heads[0], heads[1], 128, block, W.BF16, W.BF16, W.U8)
+    for broken in (False, True):
+        if broken:  # every fifth entry names no block
+            case["block_indices"] = case["block_indices"].copy()
+            case["block_indices"][::5] = -7
+        ref = H.oracle_paged(oracle, case)[0]
+        results = []
+        for overlap in (-1, 0):
+            capi.check(capi.lib().hipattn_set_option(b"mixed_overlap", overlap))
+            try:
+                dev = H.PagedDeviceCase(hip, case)
+                results.append(dev.run()[0])
+                dev.free()
+            finally:
+                capi.check(capi.lib().hipattn_set_option(b"mixed_overlap", -1))
+        begins = case["subsequence_begins"]
+        chunk = np.concatenate([np.arange(begins[s], begins[s + 1]) for s in range(len(seqs)) if seqs[s][1] > 1])
+        np.testing.assert_array_equal(results[0][chunk], results[1][chunk])
+        assert H.scaled_bound_error(results[0], ref, "%s broken %d" % (seqs, broken)) <= 1e-2
