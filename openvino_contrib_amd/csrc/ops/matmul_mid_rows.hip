@@ -1,16 +1,16 @@
 // Products of 7 to 64 activation rows with a weight matrix stored [n, k] -- the projections of a decode step of a serving batch -- on
 // v_mfma_f32_16x16x32 with fp32 accumulation, instead of the library's kernels.
 //
-// What bounds it: the weights, read once from HBM.  A workgroup takes 16 weight rows to a wavefront, four or six wavefronts, and a part
+// What bounds it: the weights, read once from HBM.  A workgroup takes 64, 96 or 128 weight rows and a part
 // of k; weights and activations come to LDS 64 elements of k at a time (global_load_lds, a ring of kRing stages, one barrier to a stage),
 // because the matrix operands as they stand are not what a compute unit loads well: sixteen lanes in sixteen rows take
 // 64 clocks to an instruction, against 16 where eight lanes share 128 bytes (64 rows on 4,096 x 4,096 straight to registers: 21.2 us
 // against 11.4).  Rows are swizzled by 16-byte pieces so that a fragment's reads spread over the banks.  Short n: the parts of k leave fp32
 // sums in the workspace and a second launch adds them in their order.
-// Measured (bf16, weights from HBM, us; library -> this, 64 rows / 16 rows): n 28,672 k 4,096: 56.0 -> 51.2 (4.6 TB/s) / 56.1 -> 46.0;
-// 22,016 x 4,096: 50.2 -> 36.4 / 53.0 -> 35.1; 4,096 x 14,336: 37.5 -> 28.7 / 26.3 -> 25.0; 4,096 x 4,096: 13.9 -> 12.2 / 11.9 -> 11.0;
-// 1,024 x 4,096: 17.8 -> 9.4; 8,192 x 8,192: 34.3 -> 31.2 / 29.8 -> 28.8 (36.5 with all workgroups beginning at the same stage).  Tiles of
-// 112 rows on 28,672 (one workgroup to a compute unit): 50.6.
+// Measured (bf16, weights from HBM, us; library -> this, 64 rows / 16 rows): n 28,672 k 4,096: 52.7 -> 43.6 (5.4 TB/s) / 56.1 -> 46.0;
+// 22,016 x 4,096: 50.2 -> 37.1 / 53.0 -> 35.1; 4,096 x 14,336: 37.5 -> 28.7 / 26.3 -> 25.0; 4,096 x 4,096: 13.9 -> 12.2 / 11.9 -> 11.0;
+// 1,024 x 4,096: 17.8 -> 9.4; 8,192 x 8,192: 34.3 -> 31.2 / 29.8 -> 28.8 (36.5 with all workgroups beginning at the same stage).
+// Two tiles of 16 weight rows to a wavefront read its activations from LDS half as often: 50.2 -> 43.4 at 28,672 x 4,096, 64 rows.
 #include "ops/ops_common.hpp"
 #include "ops/vec8.hpp"
 
@@ -74,10 +74,10 @@ struct MidRowsParams {
 
 // kGlu: the weight rows are the two halves of a gated MLP; a wavefront's 16 are eight of the gate's and the same eight of the other half,
 // c is [m, n / 2].
-template <bool kBf16, bool kGlu, int kM, int kWaves, int kRing>
+template <bool kBf16, bool kGlu, int kM, int kWaves, int kN, int kRing>
 __global__ __launch_bounds__(64 * kWaves) void matmul_mid_rows_kernel(MidRowsParams p) {
-    constexpr int kTileN = 16 * kWaves, kRows = kTileN + 16 * kM, kSlot = kRows * kStageBytes;
-    constexpr int kXLoads = (2 * kM + kWaves - 1) / kWaves, kLoads = 2 + kXLoads;  // loads of a wavefront for a stage, eight rows each
+    constexpr int kTileN = 16 * kN * kWaves, kRows = kTileN + 16 * kM, kSlot = kRows * kStageBytes;
+    constexpr int kXLoads = (2 * kM + kWaves - 1) / kWaves, kLoads = 2 * kN + kXLoads;  // loads of a wavefront for a stage, eight rows each
     __shared__ __attribute__((aligned(128))) uint8_t lds[kRing * kSlot];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, row = lane & 15, quarter = lane >> 4;
     const int tile_of_all = (int)blockIdx.x % p.tiles, part = (int)blockIdx.x / p.tiles;
@@ -92,12 +92,13 @@ __global__ __launch_bounds__(64 * kWaves) void matmul_mid_rows_kernel(MidRowsPar
     int stage = (int)((uint32_t)tile_of_all * 37u % (uint32_t)max(count, 1));
     const char* const wbase = (const char*)(p.b[which] + 64 * (int64_t)first);
     const char* const xbase = (const char*)(p.a + 64 * (int64_t)first);
-    uint32_t w[2], x[kXLoads];
+    uint32_t w[2 * kN], x[kXLoads];
     int xrow[kXLoads];
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-        int r = min(kTileN * tile + 16 * wave + 8 * i + lrow, n - 1);
-        if constexpr (kGlu) r = min((kTileN * tile + 16 * wave) / 2 + lrow, n / 2 - 1) + (p.gate_first ? i : 1 - i) * (n / 2);
+    for (int i = 0; i < 2 * kN; i++) {
+        const int row0 = kTileN * tile + 16 * (kN * wave + i / 2);
+        int r = min(row0 + 8 * (i & 1) + lrow, n - 1);
+        if constexpr (kGlu) r = min(row0 / 2 + lrow, n / 2 - 1) + (p.gate_first ? i & 1 : 1 - (i & 1)) * (n / 2);
         w[i] = (uint32_t)r * (uint32_t)(2 * p.k) + 16 * piece;
     }
 #pragma unroll
@@ -109,22 +110,30 @@ __global__ __launch_bounds__(64 * kWaves) void matmul_mid_rows_kernel(MidRowsPar
     const auto load = [&](int slot) __attribute__((always_inline)) {
         const int64_t at = (int64_t)stage * kStageBytes;
 #pragma unroll
-        for (int i = 0; i < 2; i++) load_to_lds_16(wbase + at, w[i], base + slot * kSlot + (16 * wave + 8 * i) * kStageBytes);
+        for (int i = 0; i < 2 * kN; i++) load_to_lds_16(wbase + at, w[i], base + slot * kSlot + (16 * kN * wave + 8 * i) * kStageBytes);
 #pragma unroll
         for (int i = 0; i < kXLoads; i++) load_to_lds_16(xbase + at, x[i], base + slot * kSlot + (kTileN + xrow[i]) * kStageBytes);
         stage = stage + 1 == count ? 0 : stage + 1;
     };
-    float4_t acc[kM];
+    float4_t acc[kN][kM];
 #pragma unroll
-    for (int i = 0; i < kM; i++) acc[i] = (float4_t){0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < kN; t++)
+#pragma unroll
+        for (int i = 0; i < kM; i++) acc[t][i] = (float4_t){0.f, 0.f, 0.f, 0.f};
     const int at0 = 16 * (quarter ^ (row & 7)), at1 = 16 * ((quarter + 4) ^ (row & 7));
     const auto multiply = [&](int slot) __attribute__((always_inline)) {
         const uint8_t* const s = lds + slot * kSlot + row * kStageBytes;
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            const uint4_t wf = *(const uint4_t*)(s + 16 * wave * kStageBytes + (j ? at1 : at0));
+            uint4_t wf[kN];
 #pragma unroll
-            for (int i = 0; i < kM; i++) acc[i] = mma<kBf16>(wf, *(const uint4_t*)(s + (kTileN + 16 * i) * kStageBytes + (j ? at1 : at0)), acc[i]);
+            for (int t = 0; t < kN; t++) wf[t] = *(const uint4_t*)(s + 16 * (kN * wave + t) * kStageBytes + (j ? at1 : at0));
+#pragma unroll
+            for (int i = 0; i < kM; i++) {
+                const uint4_t xf = *(const uint4_t*)(s + (kTileN + 16 * i) * kStageBytes + (j ? at1 : at0));
+#pragma unroll
+                for (int t = 0; t < kN; t++) acc[t][i] = mma<kBf16>(wf[t], xf, acc[t][i]);
+            }
         }
     };
     for (int i = 0; i < kRing - 1 && i < count; i++) load(i);
@@ -139,35 +148,39 @@ __global__ __launch_bounds__(64 * kWaves) void matmul_mid_rows_kernel(MidRowsPar
         slot = slot + 1 == kRing ? 0 : slot + 1;
         fill = fill + 1 == kRing ? 0 : fill + 1;
     }
-    // register r: weight row 4 quarter + r of the wavefront's 16, activation row lane % 16
-    if constexpr (kGlu) {
-        const int at = (kTileN * tile + 16 * wave) / 2 + 4 * quarter;  // (of quarters 0 and 1; n / 2 is a multiple of 4)
+    // register r: weight row 4 quarter + r of the 16, activation row lane % 16
+#pragma unroll
+    for (int t = 0; t < kN; t++) {
+        const int row0 = kTileN * tile + 16 * (kN * wave + t);
+        if constexpr (kGlu) {
+            const int at = row0 / 2 + 4 * quarter;  // (of quarters 0 and 1; n / 2 is a multiple of 4)
+#pragma unroll
+            for (int i = 0; i < kM; i++) {
+                float4_t other, o;
+#pragma unroll
+                for (int r = 0; r < 4; r++) other[r] = __shfl_xor(acc[t][i][r], 32);
+                const int out_row = 16 * i + row;
+                if (quarter > 1 || at >= n / 2 || out_row >= p.m) continue;
+#pragma unroll
+                for (int r = 0; r < 4; r++) o[r] = activate(acc[t][i][r], p.activation, 1.0f) * other[r];
+                *(uint2_t*)((uint16_t*)p.c[0] + (int64_t)out_row * (n / 2) + at) = (uint2_t){cvt2<kBf16>(o[0], o[1]), cvt2<kBf16>(o[2], o[3])};
+            }
+            continue;
+        }
+        const int at = row0 + 4 * quarter;  // (n is a multiple of 4)
+        if (at >= n) continue;
 #pragma unroll
         for (int i = 0; i < kM; i++) {
-            float4_t other, o;
-#pragma unroll
-            for (int r = 0; r < 4; r++) other[r] = __shfl_xor(acc[i][r], 32);
             const int out_row = 16 * i + row;
-            if (quarter > 1 || at >= n / 2 || out_row >= p.m) continue;
-#pragma unroll
-            for (int r = 0; r < 4; r++) o[r] = activate(acc[i][r], p.activation, 1.0f) * other[r];
-            *(uint2_t*)((uint16_t*)p.c[0] + (int64_t)out_row * (n / 2) + at) = (uint2_t){cvt2<kBf16>(o[0], o[1]), cvt2<kBf16>(o[2], o[3])};
+            if (out_row >= p.m) break;
+            const int64_t o = (int64_t)out_row * n + at;
+            if (p.sums != nullptr)
+                *(float4_t*)(p.sums + ((int64_t)part * p.m + out_row) * p.columns + p.offset[which] + at) = acc[t][i];
+            else if (p.c_is_f32)
+                *(float4_t*)((float*)p.c[which] + o) = acc[t][i];
+            else
+                *(uint2_t*)((uint16_t*)p.c[which] + o) = (uint2_t){cvt2<kBf16>(acc[t][i][0], acc[t][i][1]), cvt2<kBf16>(acc[t][i][2], acc[t][i][3])};
         }
-        return;
-    }
-    const int at = kTileN * tile + 16 * wave + 4 * quarter;  // (n is a multiple of 4)
-    if (at >= n) return;
-#pragma unroll
-    for (int i = 0; i < kM; i++) {
-        const int out_row = 16 * i + row;
-        if (out_row >= p.m) break;
-        const int64_t o = (int64_t)out_row * n + at;
-        if (p.sums != nullptr)
-            *(float4_t*)(p.sums + ((int64_t)part * p.m + out_row) * p.columns + p.offset[which] + at) = acc[i];
-        else if (p.c_is_f32)
-            *(float4_t*)((float*)p.c[which] + o) = acc[i];
-        else
-            *(uint2_t*)((uint16_t*)p.c[which] + o) = (uint2_t){cvt2<kBf16>(acc[i][0], acc[i][1]), cvt2<kBf16>(acc[i][2], acc[i][3])};
     }
 }
 
@@ -291,49 +304,59 @@ __global__ __launch_bounds__(kNormThreads) void projection_norm_kernel(FinishPar
 }
 
 struct Split {
-    int waves, parts;
+    int rows, parts;
 };
-// Wavefronts to a workgroup and parts of k, by the bytes that the busiest compute unit moves: its share of the weights and, with parts, the
-// chip's traffic of their sums.  A part is five stages or more (64 rows: 1,024 x 4,096 in 16 / 12 parts 11.2 / 10.5 us; 2,048 x 2,048 in
-// 8 / 6 9.4 / 8.9), four wavefronts unless six deal the rows out better (22,016 x 4,096: 45.8 -> 39.6; 6,144 x 4,096: 17.0 -> 15.3).
+// Weight rows to a workgroup (64, 96 or 128) and parts of k, by the bytes that the busiest compute unit moves: its weights, a quarter of its
+// activations (they come from the L2) and, with parts, twice the chip's traffic of their sums, which the second launch waits for.  A part is
+// five stages or more.  (us without the second launch, 64 rows, 64 / 96 / 128 weight rows at their best parts: 28,672 x 4,096 50.2 / 53 / 43.4;
+// 22,016 x 4,096 42.2 / 35.8 / 38.4; 6,144 x 4,096 14.6 / 13.0 / 13.5; 4,096 x 4,096 9.6 / 10.8 / 10.5; 4,096 x 14,336 25.3 / 27 / 25.5.)
+// 128 rows for more than 16 activation rows only: with fewer the activations are no burden.
 Split split_of(int64_t m, const int64_t* n, int count, int64_t k, size_t workspace_bytes, bool whole_k) {
     constexpr int64_t kUnits = 256;
-    Split best{4, 1};
+    Split best{64, 1};
     int64_t least = INT64_MAX, columns = 0;
     for (int i = 0; i < count; i++) columns += n[i];
-    for (int waves = 4; waves <= 6; waves += 2) {
+    const int64_t activations = m <= 16 ? 16 : m <= 32 ? 32 : 64;
+    for (int rows = 64; rows <= (m > 16 ? 128 : 96); rows += 32) {
         int64_t tiles = 0;
-        for (int i = 0; i < count; i++) tiles += (n[i] + 16 * waves - 1) / (16 * waves);
+        for (int i = 0; i < count; i++) tiles += (n[i] + rows - 1) / rows;
         for (int64_t parts = 1; parts <= 16 && (parts == 1 || (!whole_k && parts * 5 <= k / 64 && parts * tiles <= 2 * kUnits)); parts++) {
             if (parts > 1 && (size_t)(parts * m * columns * 4) > workspace_bytes) break;
-            const int64_t cost = (tiles * parts + kUnits - 1) / kUnits * (16 * waves) * (2 * k / parts) + (parts > 1 ? parts * m * columns * 8 / kUnits : 0);
-            if (cost < least) least = cost, best = {waves, (int)parts};
+            const int64_t cost =
+                (tiles * parts + kUnits - 1) / kUnits * (rows + activations / 4) * (2 * k / parts) + (parts > 1 ? parts * m * columns * 16 / kUnits : 0);
+            if (cost < least) least = cost, best = {rows, (int)parts};
         }
     }
     return best;
 }
 
+// (rings: two workgroups to a compute unit, or three)
 template <bool kBf16, bool kGlu, int kM>
-void launch(const MidRowsParams& p, int waves, hipStream_t stream) {
+void launch(const MidRowsParams& p, int rows, hipStream_t stream) {
     const dim3 grid((unsigned)(p.tiles * p.parts));
-    constexpr int kRing4 = kM == 1 ? 5 : 4, kRing6 = kM == 4 ? 4 : 5;  // (two workgroups to a compute unit, or three)
-    if (waves == 4)
-        hipLaunchKernelGGL((matmul_mid_rows_kernel<kBf16, kGlu, kM, 4, kRing4>), grid, dim3(256), 0, stream, p);
+    if constexpr (kM > 1) {
+        if (rows == 128) {
+            hipLaunchKernelGGL((matmul_mid_rows_kernel<kBf16, kGlu, kM, 4, 2, kM == 4 ? 3 : 4>), grid, dim3(256), 0, stream, p);
+            return;
+        }
+    }
+    if (rows == 64)
+        hipLaunchKernelGGL((matmul_mid_rows_kernel<kBf16, kGlu, kM, 4, 1, kM == 1 ? 5 : 4>), grid, dim3(256), 0, stream, p);
     else
-        hipLaunchKernelGGL((matmul_mid_rows_kernel<kBf16, kGlu, kM, 6, kRing6>), grid, dim3(384), 0, stream, p);
+        hipLaunchKernelGGL((matmul_mid_rows_kernel<kBf16, kGlu, kM, 6, 1, kM == 4 ? 4 : 5>), grid, dim3(384), 0, stream, p);
 }
 
 template <bool kBf16, bool kGlu>
-void launch(const MidRowsParams& p, int waves, hipStream_t stream) {
+void launch(const MidRowsParams& p, int rows, hipStream_t stream) {
     if (p.m <= 16)
-        launch<kBf16, kGlu, 1>(p, waves, stream);
+        launch<kBf16, kGlu, 1>(p, rows, stream);
     else if (p.m <= 32)
-        launch<kBf16, kGlu, 2>(p, waves, stream);
+        launch<kBf16, kGlu, 2>(p, rows, stream);
     else
-        launch<kBf16, kGlu, 4>(p, waves, stream);
+        launch<kBf16, kGlu, 4>(p, rows, stream);
 }
 
-// the products of one input with `count` weights, as tiles of split.waves wavefronts
+// the products of one input with `count` weights, in tiles of split.rows
 MidRowsParams params_of(const void* a, const void* const* b, void* const* c, const int64_t* n, int count, int64_t m, int64_t k, const Split& split,
                         float* sums) {
     MidRowsParams p{};
@@ -343,7 +366,7 @@ MidRowsParams params_of(const void* a, const void* const* b, void* const* c, con
         if (i >= count) continue;
         p.b[i] = (const uint16_t*)b[i], p.c[i] = c[i], p.n[i] = (int)n[i];
         p.begin[i] = p.tiles, p.offset[i] = p.columns;
-        p.tiles += (int)((n[i] + 16 * split.waves - 1) / (16 * split.waves)), p.columns += (int)n[i];
+        p.tiles += (int)((n[i] + split.rows - 1) / split.rows), p.columns += (int)n[i];
     }
     return p;
 }
@@ -370,9 +393,9 @@ hipattn_status matmul_mid_rows(const hipops_matmul_desc* d, const void* a, const
     MidRowsParams p = params_of(a, &b, &c, &d->n, 1, d->m, d->k, split, split.parts > 1 ? (float*)workspace : nullptr);
     p.c_is_f32 = d->c_dtype == HIPATTN_F32 ? 1 : 0;
     if (bf16)
-        launch<true, false>(p, split.waves, stream);
+        launch<true, false>(p, split.rows, stream);
     else
-        launch<false, false>(p, split.waves, stream);
+        launch<false, false>(p, split.rows, stream);
     if (split.parts > 1) {
         const int64_t count = d->m * d->n;
         const dim3 grid((unsigned)((count / 4 + 255) / 256));
@@ -386,7 +409,7 @@ hipattn_status matmul_mid_rows(const hipops_matmul_desc* d, const void* a, const
 // Up to 64 rows: one launch for all the products of an input and one for what follows them, where the operators one by one are a
 // launch each.  Bounded by the weights, once launches are few: us, 4 / 64 rows of hidden 4,096, 32 / 8 heads of 128, MLP 14,336: q, k, v and
 // two rotary embeddings in five to eight launches 33 / 62 -> 15.6 / 20.1; o, residual and norm 18 / 34 -> 13.7 / 16.2; gate|up and SwiGLU
-// 47 / 57 -> 42.0 / 54.4; down and residual 26 / 42 -> 25.8 / 31.8.
+// 47 / 57 -> 42.0 / 46; down and residual 26 / 42 -> 25.8 / 31.8.
 hipattn_status projection(const hipops_projection_desc* d, const hipops_projection_args* t, void* workspace, size_t workspace_bytes, hipStream_t stream) {
     if (!d || !t) return fail(HIPATTN_INVALID_ARGUMENT, "projection: null descriptor");
     const auto refuse = [](const char* why) { return fail(HIPATTN_UNSUPPORTED, "projection: %s", why); };
@@ -412,9 +435,9 @@ hipattn_status projection(const hipops_projection_desc* d, const hipops_projecti
         MidRowsParams p = params_of(t->x, t->weights, t->outs, d->n, 1, d->rows, d->k, split, nullptr);
         p.activation = d->glu_activation, p.gate_first = d->glu_gate_first ? 1 : 0;
         if (bf16)
-            launch<true, true>(p, split.waves, stream);
+            launch<true, true>(p, split.rows, stream);
         else
-            launch<false, true>(p, split.waves, stream);
+            launch<false, true>(p, split.rows, stream);
     } else {
         const auto float_type = [](int x) { return x == HIPATTN_F32 || x == HIPATTN_F16 || x == HIPATTN_BF16; };
         if (add && (!t->residual || (t->gamma == nullptr) != (t->normalised == nullptr))) return fail(HIPATTN_INVALID_ARGUMENT, "projection: null pointer");
@@ -430,9 +453,9 @@ hipattn_status projection(const hipops_projection_desc* d, const hipops_projecti
         const Split split = split_of(d->rows, d->n, d->num_weights, d->k, workspace_bytes, false);
         const MidRowsParams p = params_of(t->x, t->weights, t->outs, d->n, d->num_weights, d->rows, d->k, split, (float*)workspace);
         if (bf16)
-            launch<true, false>(p, split.waves, stream);
+            launch<true, false>(p, split.rows, stream);
         else
-            launch<false, false>(p, split.waves, stream);
+            launch<false, false>(p, split.rows, stream);
         FinishParams f{};
         f.sums = p.sums, f.m = p.m, f.columns = p.columns, f.parts = p.parts, f.dtype = d->dtype;
         for (int i = 0; i < kMaxWeights; i++) {

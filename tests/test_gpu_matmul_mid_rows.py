@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dtype", [F16, BF16])
 @pytest.mark.parametrize("m,n,k", [(7, 4, 64), (16, 100, 4160), (17, 1024, 4096), (32, 6144, 320), (33, 68, 704), (48, 512, 640), (49, 4096, 1024), (64, 128, 14336),
-                                   (64, 22016, 128), (20, 6160, 768), (64, 36, 8192), (12, 5500, 192), (40, 64, 96)])
+                                   (64, 22016, 128), (20, 6160, 768), (64, 36, 8192), (12, 5500, 192), (40, 64, 96), (50, 33000, 64), (30, 28676, 320)])
 def test_matmul_mid_rows(hip, ops, oracle, m, n, k, dtype):  # noqa: F811
     rng = np.random.default_rng(m + n + k)
     da, a = upload(hip, rng.standard_normal((1, m, k)) * 0.5, dtype)

@@ -65,7 +65,8 @@ def test_product_residual_and_norm(hip, ops, oracle, m, n, k, dtype):  # noqa: F
 
 @pytest.mark.parametrize("dtype", [F16, BF16])
 @pytest.mark.parametrize("m,width,k,activation,gate_first", [(1, 4, 64, 0, True), (4, 14336, 4096, 0, True), (16, 100, 320, 1, False), (33, 1376, 512, 2, True),
-                                                             (64, 11008, 256, 0, False), (20, 44, 704, 0, True)])
+                                                             (64, 11008, 256, 0, False), (20, 44, 704, 0, True), (61, 14340, 128, 0, True),
+                                                             (25, 16420, 64, 0, False)])
 def test_product_and_glu(hip, ops, oracle, m, width, k, activation, gate_first, dtype):  # noqa: F811
     rng = np.random.default_rng(m + width + k)
     dx, x = upload(hip, rng.standard_normal((m, k)), dtype)
