@@ -106,6 +106,13 @@ HIPOPS_API hipattn_status hipops_projection(const hipops_projection_desc* desc, 
     return guarded("hipops_projection", [&] { return projection(desc, tensors, workspace, workspace_bytes, (hipStream_t)stream); });
 }
 
+HIPOPS_API hipattn_status hipops_residual_norm(const void* product, const void* residual, const void* gamma, void* out, void* normalised,
+                                               int64_t rows, int64_t n, float eps, int dtype, int gamma_dtype, hipattn_stream stream) {
+    return guarded("hipops_residual_norm", [&] {
+        return residual_norm(product, residual, gamma, out, normalised, rows, n, eps, dtype, gamma_dtype, (hipStream_t)stream);
+    });
+}
+
 HIPOPS_API hipattn_status hipops_glu(const void* x, void* out, int64_t rows, int64_t width, int activation, int gate_first,
                                      int dtype, hipattn_stream stream) {
     return guarded("hipops_glu", [&] { return glu(x, out, rows, width, activation, gate_first, dtype, (hipStream_t)stream); });

@@ -39,6 +39,8 @@ hipattn_status matmul_mid_rows(const hipops_matmul_desc* d, const void* a, const
                                hipStream_t stream);
 hipattn_status projection(const hipops_projection_desc* desc, const hipops_projection_args* tensors, void* workspace, size_t workspace_bytes,
                           hipStream_t stream);
+hipattn_status residual_norm(const void* product, const void* residual, const void* gamma, void* out, void* normalised, int64_t rows, int64_t n,
+                             float eps, int dtype, int gamma_dtype, hipStream_t stream);
 hipattn_status matmul_workspace_size(const hipops_matmul_desc* desc, size_t* bytes);
 hipattn_status matmul(const hipops_matmul_desc* desc, const void* a, const void* b, void* c, void* workspace,
                       size_t workspace_bytes, hipStream_t stream);

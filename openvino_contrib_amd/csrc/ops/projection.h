@@ -46,4 +46,11 @@ typedef struct hipops_projection_args {
 hipattn_status hipops_projection(const hipops_projection_desc* desc, const hipops_projection_args* device_tensors,
                                  void* device_workspace, size_t workspace_bytes, hipattn_stream stream);
 
+/* The second half of _ADD with gamma for any number of rows, behind a product that is there: out = product + residual, rounded, and
+ * normalised = hipops_rms_norm of it, all [rows, n] of `dtype` (HIPATTN_F16 / BF16); n a multiple of 8 up to 16,384, pointers 16-byte
+ * aligned (HIPATTN_UNSUPPORTED otherwise). */
+hipattn_status hipops_residual_norm(const void* device_product, const void* device_residual, const void* device_gamma, void* device_out,
+                                    void* device_normalised, int64_t rows, int64_t n, float eps, int dtype, int gamma_dtype,
+                                    hipattn_stream stream);
+
 }  // extern "C"

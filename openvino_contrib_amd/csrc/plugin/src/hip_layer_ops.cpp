@@ -505,7 +505,8 @@ public:
         for (size_t i = 0; i < products.size(); i++) {
             const auto& in = *t[product_at[i]].in;
             const hipops_matmul_desc m = products[i]->describe(in, nullptr);
-            if (m.batch != 1 || m.m < 1 || m.m > 64) return false;
+            if (m.batch != 1 || m.m < 1) return false;
+            if (m.m > 64) return kind == HIPOPS_PROJECTION_ADD && norm && product_then_norm(context, t, m);
             d.dtype = m.ab_dtype, d.rows = m.m, d.k = m.k, d.n[i] = m.n;
             a.x = in[0].device, a.weights[i] = in[1].device, a.outs[i] = (*t[product_at[i]].out)[0].device;
         }
@@ -536,6 +537,24 @@ public:
         const hipattn_status st = hipops_projection(&d, &a, wb.mutable_buffers[0], wb.mutable_sizes[0], context.stream.get());
         if (st == HIPATTN_UNSUPPORTED) return false;
         HIP_OPS_CHECK(st);
+        return true;
+    }
+
+private:
+    // more rows than the kernels of few take: the product as it is, the residual and the norm of it in one pass over memory
+    bool product_then_norm(const InferenceRequestContext& context, const std::vector<Tensors>& t, const hipops_matmul_desc& m) const {
+        const auto& add = *t[1].in;
+        hipops_projection_desc d{};
+        d.dtype = m.ab_dtype;
+        if (add[0].shape != add[1].shape || add[0].type != (*t[0].out)[0].type || add[1].type != add[0].type ||
+            !norm->describe_for_projection(*t[2].in, d) || m.n % 8 != 0 || m.n > 16384)
+            return false;
+        const void *product = (*t[0].out)[0].device, *residual = add[residual_input].device, *gamma = (*t[2].in)[1].device;
+        void *sum = (*t[1].out)[0].device, *normalised = (*t[2].out)[0].device;
+        for (const void* x : {product, residual, gamma, (const void*)sum, (const void*)normalised})
+            if (x == nullptr || (uintptr_t)x % 16 != 0) return false;
+        products[0]->Execute(context, *t[0].in, *t[0].out, *t[0].workbuffers);
+        HIP_OPS_CHECK(hipops_residual_norm(product, residual, gamma, sum, normalised, m.m, m.n, d.eps, d.dtype, d.gamma_dtype, context.stream.get()));
         return true;
     }
 };

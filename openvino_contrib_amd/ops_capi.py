@@ -153,6 +153,12 @@ def projection(kind, dtype, rows, k, n, x, weights, outs, workspace=None, stream
     check(entry(ctypes.byref(d), ctypes.byref(a), _ptr(workspace), workspace.nbytes if workspace is not None else 0, _h(stream)))
 
 
+def residual_norm(product, residual, gamma, out, normalised, rows, n, eps, dtype, gamma_dtype, stream=None):
+    entry = lib().hipops_residual_norm  # (the plugin's too)
+    entry.restype, entry.argtypes = _i, [_vp] * 5 + [_i64, _i64, _f, _i, _i, _vp]
+    check(entry(*[_ptr(b) for b in (product, residual, gamma, out, normalised)], rows, n, eps, dtype, gamma_dtype, _h(stream)))
+
+
 GLU_SWISH, GLU_GELU, GLU_GELU_TANH = 0, 1, 2
 
 

@@ -64,6 +64,25 @@ def test_product_residual_and_norm(hip, ops, oracle, m, n, k, dtype):  # noqa: F
 
 
 @pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("rows,n", [(65, 8), (300, 4096), (1000, 1000), (3, 16384), (70, 4104)])
+def test_residual_and_norm_behind_a_product(hip, ops, oracle, rows, n, dtype):  # noqa: F811
+    """The sum is the Add's bit for bit; the norm as a single RMS: fp32 and one rounding."""
+    rng = np.random.default_rng(rows + n)
+    (dp, p), (dr, r) = (upload(hip, rng.standard_normal((rows, n)), dtype) for _ in range(2))
+    dg, g = upload(hip, 1 + 0.1 * rng.standard_normal(n), F32)
+    out, normalised, alone = (hip.DeviceBuffer(rows * n * 2) for _ in range(3))
+    out.fill(0xFF), normalised.fill(0xFF)
+    ops.residual_norm(dp, dr, dg, out, normalised, rows, n, 1e-5, dtype, F32)
+    ops.binary(0, dp, dr, alone, [rows, n], [rows, n], [rows, n], dtype)
+    got = download(hip, out, dtype, (rows, n))
+    np.testing.assert_array_equal(got, download(hip, alone, dtype, (rows, n)))
+    assert scaled_error(download(hip, normalised, dtype, (rows, n)), oracle.rms_norm(got, g, 1e-5)) <= ROUND[dtype] + 1e-6
+    with pytest.raises(ops.HipOpsError) as e:
+        ops.residual_norm(dp, dr, dg, out, normalised, rows, n + 4, 1e-5, dtype, F32)
+    assert e.value.status == hip.UNSUPPORTED
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
 @pytest.mark.parametrize("m,width,k,activation,gate_first", [(1, 4, 64, 0, True), (4, 14336, 4096, 0, True), (16, 100, 320, 1, False), (33, 1376, 512, 2, True),
                                                              (64, 11008, 256, 0, False), (20, 44, 704, 0, True), (61, 14340, 128, 0, True),
                                                              (25, 16420, 64, 0, False)])
