@@ -450,6 +450,9 @@ hipattn_status projection(const hipops_projection_desc* d, const hipops_projecti
     if (glu) {
         if (d->glu_activation < HIPOPS_GLU_SWISH || d->glu_activation > HIPOPS_GLU_GELU_TANH)
             return fail(HIPATTN_INVALID_ARGUMENT, "projection: activation %d", d->glu_activation);
+        // (the operators one by one read x before they write over it; here other workgroups may still be reading)
+        const uintptr_t x = (uintptr_t)t->x, out = (uintptr_t)t->outs[0];
+        if (x < out + (uintptr_t)(d->rows * d->n[0]) && out < x + (uintptr_t)(2 * d->rows * d->k)) return refuse("results over the input");
         const Split split = split_of(d->rows, d->n, 1, d->k, 0, true);
         MidRowsParams p = params_of(t->x, t->weights, t->outs, d->n, 1, d->rows, d->k, split, nullptr);
         p.activation = d->glu_activation, p.gate_first = d->glu_gate_first ? 1 : 0;

@@ -14,7 +14,7 @@ extern "C" {
  *   _GLU   out[0] [rows, n[0] / 2] = hipops_glu of x * weights[0]^T
  * Everything is `dtype` (HIPATTN_F16 / BF16) but the tables and gamma; sums and what is done to them are
  * fp32, rounded once (the products are not rounded before).  n[i] is a multiple of 8, k of 64, pointers are
- * 16-byte aligned; HIPATTN_UNSUPPORTED, with nothing launched, for what the kernels do not take: the
+ * 16-byte aligned, and what _GLU writes is no part of x; HIPATTN_UNSUPPORTED, with nothing launched, for what the kernels do not take: the
  * operators one by one do.  The workspace holds rows * sum(n) floats or more (not needed for _GLU);
  * hipops_matmul_workspace_size's is enough for every split of k. */
 #define HIPOPS_PROJECTION_ROPE 0

@@ -101,7 +101,7 @@ def test_what_the_kernels_do_not_take_is_refused(hip, ops):  # noqa: F811
     buf, ws = hip.DeviceBuffer(1 << 20), hip.DeviceBuffer(1 << 20)
     for kwargs, status in ((dict(rows=65), hip.UNSUPPORTED), (dict(k=96), hip.UNSUPPORTED), (dict(n=(12,)), hip.UNSUPPORTED), (dict(dtype=F32), hip.UNSUPPORTED),
                            (dict(workspace=None), hip.UNSUPPORTED), (dict(residual=None), hip.INVALID_ARGUMENT), (dict(kind=7), hip.INVALID_ARGUMENT),
-                           (dict(gamma=buf, normalised=None), hip.INVALID_ARGUMENT)):
+                           (dict(gamma=buf, normalised=None), hip.INVALID_ARGUMENT), (dict(kind=ops.PROJECTION_GLU), hip.UNSUPPORTED)):
         call = dict(dict(kind=ops.PROJECTION_ADD, dtype=BF16, rows=8, k=64, n=(64,), x=buf, weights=[buf], outs=[buf], workspace=ws, residual=buf), **kwargs)
         with pytest.raises(ops.HipOpsError) as e:
             ops.projection(**call)
