@@ -160,6 +160,7 @@ struct PagedParams {
     uint16_t* shadow_k;
     uint16_t* shadow_v;
     int32_t* shadow_table;
+    int lone_tile;        // (paged_mixed.hip) one sequence, which gets query tiles also if it is a single token: no decode rows, no merge
     int tiles_only;       // (flash_small.hip) tile_prefix counts single-token sequences too: there are no decode rows
 };
 

@@ -23,14 +23,15 @@ __device__ __forceinline__ void plan_block(const PagedParams& p) {
     if (tid < 64) p.dyn_counter[tid] = 0;  // tickets for the dynamic pieces of this call, one counter per group
     const int per = (p.num_rows + 255) / 256;
     const int s0 = min(tid * per, p.num_rows), s1 = min(s0 + per, p.num_rows);
+    const int tiled = p.lone_tile ? 1 : 2;  // tokens of the shortest sequence that gets query tiles
     int blk = 0, tile = 0;
     float key_tiles = 0.0f;  // 64-key tiles the flash kernel works through, summed over 128-row query tiles
     for (int s = s0; s < s1; s++) {
         // (rows are sequences whenever the lengths matter here: max_q_tiles > 0)
         const int qlen = p.max_q_tiles > 0 ? p.subsequence_begins[s + 1] - p.subsequence_begins[s] : 1;
         blk += line_units(decode_range(p, s).nb, p.switch_cost);
-        tile += (qlen > 1 && p.max_q_tiles > 0) ? (qlen + 127) / 128 : 0;
-        if (p.overlap && qlen > 1) {
+        tile += (qlen >= tiled && p.max_q_tiles > 0) ? (qlen + 127) / 128 : 0;
+        if (p.overlap && qlen >= tiled) {
             const int past = p.past_lens[s];
             for (int r0 = 0; r0 < qlen; r0 += 128) {
                 int keys = past + min(qlen, r0 + 128);
@@ -94,7 +95,7 @@ __device__ __forceinline__ void plan_block(const PagedParams& p) {
         ((DecodeRange*)p.seq_info)[s] = rg;
         if (rg.empty_row) zero_output_row(p, rg.token);  // (rare: an empty block table) nothing will visit this row
         blk += line_units(rg.nb, p.switch_cost);
-        tile += (qlen > 1 && p.max_q_tiles > 0) ? (qlen + 127) / 128 : 0;
+        tile += (qlen >= tiled && p.max_q_tiles > 0) ? (qlen + 127) / 128 : 0;
     }
     if (s1 == p.num_rows && s0 < p.num_rows) {
         p.blk_prefix[p.num_rows] = blk;
@@ -872,9 +873,10 @@ static int resident_decode_waves() {
 // on the device): each such sequence has at least 2 tokens and wastes at most one tile.
 // 0 selects the row-per-token form of the plan, which takes the batch to hold as many rows as
 // sequences: only a batch with exactly that many tokens may get it (a single token spread over two
-// or more sequences, all but one of them empty, has a bound of 0 by the formula and must not).
+// or more sequences, all but one of them empty, has a bound of 0 by the formula and must not); and one
+// token in one sequence, which has no other length.
 static int query_tile_bound(const PagedParams& p) {
-    if (p.num_tokens == p.num_seqs && !p.any_lengths) return 0;  // one token per sequence: a pure decode batch
+    if (p.num_tokens == p.num_seqs && (!p.any_lengths || p.num_seqs == 1)) return 0;  // one token per sequence: a pure decode batch
     return std::max(1, p.num_tokens / 128 + std::min(p.num_seqs, p.num_tokens / 2));
 }
 
@@ -970,6 +972,11 @@ void paged_fast_plan(PagedParams& p, void* workspace, size_t workspace_bytes) {
     const int G = p.num_heads_q / p.num_heads_kv;
     p.max_q_tiles = query_tile_bound(p);
     p.num_rows = plan_rows(p);
+    // One sequence: its length is known to the device alone, and it may turn out to be a single token (a padded or a recorded call).  As a
+    // decode row that needs the decode workgroups and the merge, which cost every prompt 2 us (64 tokens 14.5 -> 16.5, 1,000 38.0 -> 40.1); as
+    // a query tile it needs neither, but walks its context alone (us, tile / decode row: 300 tokens 21 / 16, 2,000 54 / 19, 8,000 165 / 23; u8
+    // 22 / 18, 70 / 21, 236 / 23).  A tile while the bound on the context keeps it below 45 us, which two kernels took for any context.
+    p.lone_tile = overlap && p.num_seqs == 1 && most_blocks(p) <= 32 && paged_mixed_supported(p) ? 1 : 0;
     const int64_t segments = (int64_t)p.num_rows * p.num_heads_kv;
     // 16-bit caches: from 128 segments on all wavefronts (24 sequences of 400: 16.1 us against 17.4 with 512; 63 of 300, 504
     // segments: 23.1 against 23.8 with 768).  (On-demand pieces: every ticket group needs its wavefronts.)
@@ -1250,8 +1257,7 @@ hipError_t launch_paged_fast(const PagedParams& params, const KvWriteParams* wri
         if (probe.before) (void)hipEventRecord(probe.before, stream);
         e = launch_paged_mixed(p, p.num_heads_kv / p.kv_share, stream);
         if (probe.after) (void)hipEventRecord(probe.after, stream);
-        // (a batch of one sequence that is not a single token has no decode rows)
-        return e != hipSuccess || p.fused_merge || p.num_seqs == 1 ? e : launch_merge(p, stream);
+        return e != hipSuccess || p.fused_merge || p.lone_tile ? e : launch_merge(p, stream);
     }
     if (p.max_q_tiles > 0 && (p.overlap || beside)) {
         // Mixed batch of a shape that the kernel of both parts (paged_mixed.hip) does not take: the decode

@@ -3,7 +3,7 @@
 //
 // Both take whole compute units.  The first workgroups, which are dispatched first, are the decode part's; the plan on
 // the device has chosen how many of them work and the others leave at once, so that the chunks' workgroups find every
-// compute unit the decode part does not keep.  As two kernels, the chunks on a side stream, the fork and the join left
+// compute unit the decode part does not keep.  (One sequence of a short context: no decode part, p.lone_tile.)  As two kernels, the chunks on a side stream, the fork and the join left
 // the chip idle for some 25 us a step.  Measured (us a step, two kernels -> one; 32 heads on 8 kv heads of 128): a prompt of 64 tokens 46 -> 14,
 // of 1,000 60 -> 39; 8 prompts of 1,000 155 -> 138, of 2,000 364 -> 347; six uneven prompts into a u8 cache 193 -> 176; two chunks of 200 beside 20
 // decode rows 49 -> 38, beside 100 long ones 375 -> 368; 8 chunks of 512 beside 120 rows, 64 heads, 585 -> 579.
@@ -51,7 +51,7 @@ bool paged_mixed_supported(const PagedParams& p) {
 
 hipError_t launch_paged_mixed(const PagedParams& p, int chunk_heads_kv, hipStream_t stream) {
     // (workgroups go to the XCDs round-robin and the chunks' order counts on that: a multiple of eight in front of them)
-    const int decode_workgroups = p.num_seqs == 1 ? 0 : (p.num_waves / 8 + 7) / 8 * 8;
+    const int decode_workgroups = p.lone_tile ? 0 : (p.num_waves / 8 + 7) / 8 * 8;
     const int G = p.num_heads_q / chunk_heads_kv;
     const dim3 grid((unsigned)(decode_workgroups + (int64_t)p.max_q_tiles * ((G & 1) == 0 ? p.num_heads_q / 2 : p.num_heads_q)));
     const bool bf16 = p.cache_dtype == HIPATTN_BF16;
