@@ -79,7 +79,7 @@ hipattn_status hipops_rope(const hipops_rope_desc* desc, const void* device_x, c
 
 /* ---- MatMul -----------------------------------------------------------------------------
  * C[b] = op(A[b]) * op(B[b]), row-major, through hipBLASLt (up to 64 rows on weights
- * stored [n, k]: kernels of their own).  Replaces MatMulOp
+ * stored [n, k]: kernels of their own, where they are the faster ones).  Replaces MatMulOp
  * (src/ops/matmul.cpp:22-76 for the shape rules, :185-227 for cublasGemmStridedBatchedEx).
  * op(A) is m x k (A stored k x m when transpose_a), op(B) is k x n (B stored n x k when
  * transpose_b - the weight layout of a projection).  batch_stride_a / _b == 0 broadcasts that

@@ -1,6 +1,5 @@
 // MatMul: few rows (up to six, up to 16 on small weights) in the kernel of matmul_few_rows.hip, up to 64 in that of
-// matmul_mid_rows.hip, else through hipBLASLt: a
-// plain library GEMM with fp32 accumulation.  The operator's tensors are row-major; hipBLASLt is column-major, so the product is taken transposed
+// matmul_mid_rows.hip where it is the faster one, else through hipBLASLt: a plain library GEMM with fp32 accumulation.  The operator's tensors are row-major; hipBLASLt is column-major, so the product is taken transposed
 // (C^T = op(B)^T * op(A)^T) with the operands swapped and no data movement.  Descriptors and the
 // algorithm are kept per (device, shape), so a repeated shape costs one hipblasLtMatmul call; the
 // algorithm is the fastest of the heuristic's candidates, timed once when the shape is first seen
@@ -117,7 +116,7 @@ hipattn_status matmul(const hipops_matmul_desc* d, const void* a, const void* b,
     int device = 0;
     if (hipGetDevice(&device) != hipSuccess) return fail(HIPATTN_NO_DEVICE, "matmul: no current device");
     if (matmul_few_rows_supported(d, a, b, c)) return matmul_few_rows(d, a, b, c, stream);
-    if (matmul_mid_rows_supported(d, a, b, c)) return matmul_mid_rows(d, a, b, c, workspace, workspace_bytes, stream);
+    if (matmul_mid_rows_supported(d, a, b, c, workspace_bytes)) return matmul_mid_rows(d, a, b, c, workspace, workspace_bytes, stream);
 
     DeviceState* dev_ptr = nullptr;
     {

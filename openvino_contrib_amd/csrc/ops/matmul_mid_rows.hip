@@ -1,5 +1,6 @@
-// Products of 7 to 64 activation rows with a weight matrix stored [n, k] -- the projections of a decode step of a serving batch -- on
-// v_mfma_f32_16x16x32 with fp32 accumulation, instead of the library's kernels.
+// Products of few activation rows with a weight matrix stored [n, k] -- the projections of a decode step of a serving batch -- on
+// v_mfma_f32_16x16x32 with fp32 accumulation, instead of the library's kernels: of 7 to 64 rows by themselves, of 1 to 64 with what follows
+// them (projection()).
 //
 // What bounds it: the weights, read once from HBM.  A workgroup takes 64, 96 or 128 weight rows and a part
 // of k; weights and activations come to LDS 64 elements of k at a time (global_load_lds, a ring of kRing stages, one barrier to a stage),
@@ -314,6 +315,7 @@ __global__ __launch_bounds__(kNormThreads) void projection_norm_kernel(FinishPar
     }
 }
 
+constexpr int64_t kMaxParts = 16;
 struct Split {
     int rows, parts;
 };
@@ -331,7 +333,7 @@ Split split_of(int64_t m, const int64_t* n, int count, int64_t k, size_t workspa
     for (int rows = 64; rows <= (m > 16 ? 128 : 96); rows += 32) {
         int64_t tiles = 0;
         for (int i = 0; i < count; i++) tiles += (n[i] + rows - 1) / rows;
-        for (int64_t parts = 1; parts <= 16 && (parts == 1 || (!whole_k && parts * 5 <= k / 64 && parts * tiles <= 2 * kUnits)); parts++) {
+        for (int64_t parts = 1; parts <= kMaxParts && (parts == 1 || (!whole_k && parts * 5 <= k / 64 && parts * tiles <= 2 * kUnits)); parts++) {
             if (parts > 1 && (size_t)(parts * m * columns * 4) > workspace_bytes) break;
             const int64_t cost =
                 (tiles * parts + kUnits - 1) / kUnits * (rows + activations / 4) * (2 * k / parts) + (parts > 1 ? parts * m * columns * 16 / kUnits : 0);
@@ -391,6 +393,26 @@ MidRowsParams params_of(const void* a, const void* const* b, void* const* c, con
 }
 
 bool aligned16(const void* x) { return ((uintptr_t)x & 15) == 0; }
+
+// Where the library's kernels are the faster ones (us, library / this).
+bool library_is_faster(int64_t m, int64_t n, int64_t k, size_t workspace_bytes) {
+    // A workspace too small for the parts of k (or none): a workgroup's chain of k, where the workgroups are fewer than two thirds of the compute
+    // units (no workspace; 16 rows, 4,096 x 2,048 11.0 / 8.9, x 2,560 11.4 / 12.0, 8,192 x 4,096 16.1 / 17.5, 9,216 x 4,096 23.8 / 18.1, 16 x 8,192 11.0 / 26.1;
+    // 32 rows, 512 x 2,048 11.1 / 9.7, x 2,560 11.3 / 11.5, x 3,072 10.9 / 13.4; 64 rows, 512 x 1,536 11.1 / 9.8, x 2,048 11.1 / 12.2, 4,096 x 4,096 14.0 / 22.1,
+    // 11,008 x 4,096 27.0 / 25.0).
+    const int64_t longest = m <= 32 ? 2048 : 1536;
+    if (k > longest && n < 172 * 64 && workspace_bytes < (size_t)(kMaxParts * m * n * 4)) {
+        const int64_t parts = split_of(m, &n, 1, k, workspace_bytes, false).parts;
+        if (n * parts < 172 * 64 && k / parts > longest && parts < split_of(m, &n, 1, k, SIZE_MAX, false).parts) return true;
+    }
+    // Up to 16 rows on some middling weights (16 rows: 2,560 x 5,120 10.6 / 10.1, 2,816 x 5,120 10.6 / 11.2, 3,328 x 5,120 10.8 / 11.8, x 9,216 15.9 / 15.9,
+    // 4,096 x 8,192 15.8 / 17.6, x 10,240 19.5 / 19.3, 4,608 x 8,192 22.4 / 18.7; 24 rows: 3,328 x 5,120 12.9 / 12.2) and, to 32 rows from n = 7,168 on, on short k (16 rows:
+    // 5,632 x 3,072 11.2 / 11.6, 6,144 x 3,072 10.9 / 11.9, 8,192 x 4,096 15.7 / 17.8, x 6,144 23.7 / 21.3, 9,216 x 4,096 23.6 / 20.4; 32 rows: 6,144 x 4,096 14.8 / 14.3,
+    // 8,192 x 4,096 16.2 / 18.2).
+    if (m <= 16 && n >= 2816 && n <= 4096 && k >= 5120 && k <= 9216) return true;
+    return m <= (n < 7168 ? 16 : 32) && n >= 6144 && n <= 8192 && k >= 3072 && k <= 5120;
+}
+
 bool sizes_supported(int dtype, int64_t n, int64_t k) {
     return (dtype == HIPATTN_F16 || dtype == HIPATTN_BF16) && k % 64 == 0 && k < (1 << 24) && n * k <= (1 << 28);
 }
@@ -399,10 +421,10 @@ bool sizes_supported(int dtype, int64_t n, int64_t k) {
 
 // 16-bit operands, one matrix, the weights' rows along k in whole stages (and all of them within 32 bits of offset), 16-byte
 // aligned rows.  The sums of the parts need a workspace; without one k stays whole.  The largest weights are the library's
-// (128,256 x 4,096 with 7 / 16 / 64 rows: 180 / 191 / 202 us there, 186 / 188 / 206 here).
-bool matmul_mid_rows_supported(const hipops_matmul_desc* d, const void* a, const void* b, const void* c) {
+// (128,256 x 4,096 with 7 / 16 / 64 rows: 180 / 191 / 202 us there, 186 / 188 / 206 here), and so is what library_is_faster names.
+bool matmul_mid_rows_supported(const hipops_matmul_desc* d, const void* a, const void* b, const void* c, size_t workspace_bytes) {
     return sizes_supported(d->ab_dtype, d->n, d->k) && d->batch == 1 && !d->transpose_a && d->transpose_b && d->m > 6 && d->m <= 64 && d->n % 4 == 0 &&
-           aligned16(a) && aligned16(b) && aligned16(c);
+           aligned16(a) && aligned16(b) && aligned16(c) && !library_is_faster(d->m, d->n, d->k, workspace_bytes);
 }
 
 hipattn_status matmul_mid_rows(const hipops_matmul_desc* d, const void* a, const void* b, void* c, void* workspace, size_t workspace_bytes,

@@ -34,7 +34,7 @@ hipattn_status softmax(const void* x, void* out, int64_t outer, int64_t length, 
 bool matmul_few_rows_supported(const hipops_matmul_desc* d, const void* a, const void* b, const void* c);
 hipattn_status matmul_few_rows(const hipops_matmul_desc* d, const void* a, const void* b, void* c, hipStream_t stream);
 // 7 to 64 rows against weights stored [n, k] (matmul_mid_rows.hip)
-bool matmul_mid_rows_supported(const hipops_matmul_desc* d, const void* a, const void* b, const void* c);
+bool matmul_mid_rows_supported(const hipops_matmul_desc* d, const void* a, const void* b, const void* c, size_t workspace_bytes);
 hipattn_status matmul_mid_rows(const hipops_matmul_desc* d, const void* a, const void* b, void* c, void* workspace, size_t workspace_bytes,
                                hipStream_t stream);
 hipattn_status projection(const hipops_projection_desc* desc, const hipops_projection_args* tensors, void* workspace, size_t workspace_bytes,
