@@ -472,6 +472,12 @@ hipattn_status projection(const hipops_projection_desc* d, const hipops_projecti
     if (glu) {
         if (d->glu_activation < HIPOPS_GLU_SWISH || d->glu_activation > HIPOPS_GLU_GELU_TANH)
             return fail(HIPATTN_INVALID_ARGUMENT, "projection: activation %d", d->glu_activation);
+        // k stays whole: where the weights are too few rows for two thirds of the compute units a long one is a chain that the product in parts and
+        // the GLU as an operator are faster than (us, one by one / here; 4 rows: 512 x 2,048 7.7 / 9.3, 7,168 x 2,048 13.0 / 12.2; 16 rows: 512 x 2,048 8.9 / 9.1,
+        // x 4,096 12.5 / 15.4, x 8,192 11 / 28; 32 rows: 8,192 x 2,048 15.2 / 14.7, x 4,096 20.5 / 23.6; 64 rows: 2,048 x 2,048 12.1 / 14.0, 8,192 x 2,048
+        // 16.7 / 16.2, x 8,192 36 / 46; 11,264 x 4,096 28 / 29, 33 with the library's product)
+        const bool enough = (d->rows > 8 && d->rows <= 32) || d->n[0] >= (d->rows <= 8 ? 7168 : 4096);
+        if (d->n[0] < 172 * 64 && d->k > (enough ? 2048 : 1536)) return refuse("k too long for weights of few rows");
         // (the operators one by one read x before they write over it; here other workgroups may still be reading)
         const uintptr_t x = (uintptr_t)t->x, out = (uintptr_t)t->outs[0];
         if (x < out + (uintptr_t)(d->rows * d->n[0]) && out < x + (uintptr_t)(2 * d->rows * d->k)) return refuse("results over the input");

@@ -108,6 +108,22 @@ def test_what_the_kernels_do_not_take_is_refused(hip, ops):  # noqa: F811
         assert e.value.status == status, kwargs
 
 
+@pytest.mark.parametrize("m,n,k,taken", [(8, 7160, 1536, True), (8, 7160, 1600, False), (8, 7168, 2048, True), (1, 7168, 2112, False), (9, 8, 2048, True), (32, 11000, 2112, False),
+                                         (33, 4088, 1600, False), (33, 4096, 2048, True), (64, 11008, 2112, True), (64, 512, 8192, False), (4, 28672, 4096, True)])
+def test_glu_behind_a_long_k_goes_operator_by_operator(hip, ops, m, n, k, taken):  # noqa: F811
+    """Either side of the lines: weights of few rows on a long k are a product in parts and an operator."""
+    x, w, out = hip.DeviceBuffer(m * k * 2), hip.DeviceBuffer(n * k * 2), hip.DeviceBuffer(m * n)
+    x.fill(0), w.fill(0), out.fill(0xFF)
+    call = lambda: ops.projection(ops.PROJECTION_GLU, BF16, m, k, (n,), x, [w], [out])
+    if not taken:
+        with pytest.raises(ops.HipOpsError) as e:
+            call()
+        assert e.value.status == hip.UNSUPPORTED
+    else:
+        call()
+    assert (download(hip, out, BF16, (m, n // 2)) == 0).all() == taken
+
+
 def _model(tokens, hidden, ffn, heads, kv_heads, size, extra_reader):
     """norm -> q, k, v -> RoPE of q and k -> (their parts put together, as far as they are wide) -> o -> Add -> norm -> gate|up -> GLU -> down -> Add."""
     rng = np.random.default_rng(tokens + hidden)
