@@ -225,6 +225,7 @@ public:
         return true;
     }
     bool has_positions() const { return has_positions_; }
+    bool ReadsRowsOf(size_t input) const override { return input == 1 || input == 2; }
 
 private:
     ov::op::internal::RoPE::Config cfg_;
@@ -333,6 +334,7 @@ public:
             HIP_PLUGIN_THROW(who + "axis " + std::to_string(axis_) + " / batch_dims " + std::to_string(batch_dims_));
     }
     bool InputIsHostOnly(size_t input) const override { return input == 2; }  // the axis was read from its Constant
+    bool ReadsRowsOf(size_t input) const override { return input == 0; }
     std::vector<ov::Shape> InferOutputShapes(const std::vector<TensorView>& in, const InferenceRequestContext&) const override {
         const ov::Shape &d = in.at(0).shape, &i = in.at(1).shape;
         for (int64_t b = 0; b < batch_dims_; b++)

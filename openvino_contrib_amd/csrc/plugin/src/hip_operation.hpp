@@ -121,6 +121,8 @@ public:
     // When such an input was bound as a host tensor the request copies it back after the operator,
     // so the caller's memory holds the update; device-resident tensors need nothing.
     virtual std::vector<size_t> UpdatedInputs() const { return {}; }
+    // an input of which it reads single rows (an embedding table, the tables of a rotary embedding)
+    virtual bool ReadsRowsOf(size_t /*input*/) const { return false; }
     // True for an input the operator only ever reads through TensorView::host (a scale, a window, a
     // shape pattern, an order): a tensor all of whose consumers say so is not uploaded, and its
     // TensorView::device is null.

@@ -976,24 +976,48 @@ void InferRequest::execute_steps(const InferenceRequestContext& context, bool pr
     }
 }
 
-// True where the kernels are long enough that launching them one by one, ahead of the GPU, costs nothing: a graph's first kernel
-// starts 17 us behind its launch call, an operator's own launch takes 3 us.  (Decoder layers, us per infer, graph -> operators: 4
-// sequences, hidden 4,096, 34 MB of operands to an operator, 169 -> 151; 1 sequence, hidden 2,048, 7 MB, 87 -> 74; but 16 / 32 Adds of 1 KB
-// 61 / 111 -> 89 / 145.)  Buffers an operator updates in place do not count: of a KV cache it reads what the sequences hold.
+// True where the operators one by one are done sooner than a graph of them.  The GPU starts on the first of them while the host
+// is still launching, where a graph's first kernel starts 17 us behind its launch call.  But one by one they follow each other a microsecond
+// later than in a graph, and the host takes 3 to 5.5 us to a launch: where the GPU is done with one sooner it waits.  So the two are compared launch by
+// launch, by what each must read and write at 8 TB/s (tensors this small come from the caches) beside the least its kind takes; below
+// 4 MB to a launch the gain is within the noise and a graph costs the host less.  In effect models of up to some 12 launches with large operands
+// run without a graph.
+// (us per infer, graph / operators: decoder layers of hidden 4,096, 1 / 4 / 16 of them, 154 / 143, 502 / 528, 1,988 / 2,059; of hidden 2,048 92 / 89, 301 / 302,
+// 1,115 / 1,142; 16 / 32 Adds of 1 KB 57 / 86, 99 / 148, 14 / 32 of 4 MB 72 / 81, 138 / 163, 12 / 32 of 16 MB 145 / 135, 338 / 331.)
+// Not counted: buffers an operator updates in place (of a KV cache it reads what the sequences hold), tables it reads
+// rows of, and views, which are no launch either.
 bool InferRequest::outlasts_its_launches() const {
-    constexpr size_t kBytesPerOperator = 4 << 20;
+    constexpr size_t kBytesPerLaunch = 4 << 20;
+    constexpr float kGraphStart = 17.f, kGap = 0.9f, kHostPerLaunch = 5.5f, kBytesPerMicrosecond = 8e6f;
     const auto& sequence = compiled_->exec_sequence();
-    size_t bytes = 0, operators = 0;
+    size_t all_bytes = 0, launches = 0;
+    std::vector<int> seen(compiled_->groups().size(), 0);
+    float host = 0.f, gpu = 0.f, kernels = 0.f;
     for (size_t si = 0; si < prepared_.size(); si++) {
-        const std::string& type = sequence[si].op->GetTypeName();
-        if (type == "Parameter" || type == "Result" || type == "Constant") continue;
-        operators++;
-        const auto updated = sequence[si].op->UpdatedInputs();
+        const OperationBase& op = *sequence[si].op;
+        const std::string& type = op.GetTypeName();
+        if (type == "Parameter" || type == "Result" || type == "Constant" || (op.InplaceInputOf(0) >= 0 && prepared_[si].copies.empty())) continue;
+        size_t bytes = 0;
+        const auto updated = op.UpdatedInputs();
         for (size_t i = 0; i < prepared_[si].in.size(); i++)
-            if (prepared_[si].in[i].device && std::find(updated.begin(), updated.end(), i) == updated.end()) bytes += prepared_[si].in[i].byte_size();
+            if (prepared_[si].in[i].device && !op.ReadsRowsOf(i) && std::find(updated.begin(), updated.end(), i) == updated.end())
+                bytes += prepared_[si].in[i].byte_size();
         for (const auto& out : prepared_[si].out) bytes += out.byte_size();
+        const bool attention = type == "PagedAttentionExtension" || type == "ScaledDotProductAttention";
+        const float least = attention ? 12.f : type == "MatMul" || type == "RMS" ? 4.2f : 2.7f;
+        const int group = compiled_->group_of(si);
+        const bool launch = group < 0 || ++seen[group] <= 2;  // (a group is two launches)
+        const float us = (launch ? least : 0.f) + (float)bytes / kBytesPerMicrosecond;
+        if (launch) {
+            launches++;
+            host += kHostPerLaunch;
+            gpu = std::max(gpu + kGap, host);
+        }
+        all_bytes += bytes;
+        gpu += us;
+        kernels += us;
     }
-    return bytes >= operators * kBytesPerOperator;
+    return all_bytes >= launches * kBytesPerLaunch && gpu <= kGraphStart + kernels;
 }
 
 // Everything the operators of this infer were handed, as numbers: two infers with equal signatures
