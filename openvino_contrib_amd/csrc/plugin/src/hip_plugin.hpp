@@ -152,6 +152,7 @@ private:
     std::condition_variable wake_;
     std::deque<ov::threading::Task> queue_;
     std::atomic<size_t> queued_{0};  // of queue_, to be looked at without the lock
+    std::atomic<bool> looking_out_{false};  // a worker is, without the lock
     bool stopping_ = false;
     std::vector<std::thread> threads_;
 };
