@@ -278,7 +278,7 @@ RECORDED_TRAFFIC = {
     "c3": ((563582.6 * 2.0 + 3258.4) * 1024, "profiles/paged_decode_kernel_config3_fp16.txt"),
     "c4": ((1225872.7 * 2.0 + 12671.2) * 1024, "profiles/paged_decode_kernel_config4_u8.txt"),
     "c2": ((49302.7 * 2.0 + 65536.0) * 1024, "profiles/sdpa_flash_kernel_config2_bf16.txt"),
-    "c5": ((786147.1 * 2.0 + 6318.8) * 1024, "profiles/paged_attention_config5_mixed.txt"),  # the decode part of the mixed step
+    "c5": ((904840.2 * 2.0 + 71868.7) * 1024, "profiles/paged_attention_config5_mixed.txt"),  # decode rows and chunks, one kernel
 }
 
 
@@ -288,10 +288,11 @@ def recorded_traffic(w):
 
 
 def roofline_hbm(res, w):
-    a = res["decode_kv_bytes"] / (res["dominant_kernel_ms"] * 1e-3) / 1e9
+    mixed = w in ("c5", "c5u8")  # (one kernel for the decode rows and the chunks: the rows of both)
+    a = res["kv_bytes" if mixed else "decode_kv_bytes"] / (res["dominant_kernel_ms"] * 1e-3) / 1e9
     traffic, source = recorded_traffic(w)
     return {"bound": "hbm", "achieved": a, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": a / HBM_PEAK_GBS,
-            "traffic": traffic, "traffic_source": source, "kernel": "paged_mixed_kernel" if w == "c5" else "paged_decode_kernel"}
+            "traffic": traffic, "traffic_source": source, "kernel": "paged_mixed_kernel" if mixed else "paged_decode_kernel"}
 
 
 def roofline_mfma(res):
@@ -1010,8 +1011,8 @@ def main():
                 t_ideal = max(r["kv_bytes"] / (HBM_PEAK_GBS * 1e9), r["flops"] / (MFMA_BF16_PEAK_TFLOPS * 1e12))
                 r["ideal_ms"] = t_ideal * 1e3
                 r["frac_of_ideal"] = t_ideal * 1e3 / r["ms_per_step"]
-                r["roofline"]["note"] = ("mixed batch: the decode kernel runs beside the chunks' flash kernel on a share "
-                                         "of the compute units, so its duration is not a whole-chip figure; "
+                r["roofline"]["note"] = ("mixed batch: one kernel reads the cache for the decode rows on a share of the compute units and "
+                                         "works on the chunks, bound by the matrix cores, on the others; "
                                          "frac_of_ideal is the one for this step")
         log("%s: %.3f ms/step, dominant kernel %.3f ms, roofline frac %.3f"
             % (w, r["ms_per_step"], r["dominant_kernel_ms"], r["roofline"]["frac"]))
