@@ -393,6 +393,15 @@ MidRowsParams params_of(const void* a, const void* const* b, void* const* c, con
 }
 
 bool aligned16(const void* x) { return ((uintptr_t)x & 15) == 0; }
+bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+    return (uintptr_t)a < (uintptr_t)b + (uintptr_t)b_bytes && (uintptr_t)b < (uintptr_t)a + (uintptr_t)a_bytes;
+}
+// Operator by operator the sum of all rows is there before the norm of any is written; here another row's workgroup may still be reading.  (The
+// residual's own place is fine: what a lane writes there it has read.)
+bool norm_over_inputs(const void* residual, const void* gamma, int gamma_dtype, const void* out, const void* normalised, int64_t rows, int64_t n) {
+    const int64_t bytes = 2 * rows * n, gamma_bytes = n * (gamma_dtype == HIPATTN_F32 ? 4 : 2);
+    return (normalised != residual && overlap(normalised, bytes, residual, bytes)) || overlap(out, bytes, gamma, gamma_bytes);
+}
 
 // Where the library's kernels are the faster ones (us, library / this).
 bool library_is_faster(int64_t m, int64_t n, int64_t k, size_t workspace_bytes) {
@@ -479,8 +488,7 @@ hipattn_status projection(const hipops_projection_desc* d, const hipops_projecti
         const bool enough = (d->rows > 8 && d->rows <= 32) || d->n[0] >= (d->rows <= 8 ? 7168 : 4096);
         if (d->n[0] < 172 * 64 && d->k > (enough ? 2048 : 1536)) return refuse("k too long for weights of few rows");
         // (the operators one by one read x before they write over it; here other workgroups may still be reading)
-        const uintptr_t x = (uintptr_t)t->x, out = (uintptr_t)t->outs[0];
-        if (x < out + (uintptr_t)(d->rows * d->n[0]) && out < x + (uintptr_t)(2 * d->rows * d->k)) return refuse("results over the input");
+        if (overlap(t->x, 2 * d->rows * d->k, t->outs[0], d->rows * d->n[0])) return refuse("results over the input");
         const Split split = split_of(d->rows, d->n, 1, d->k, 0, true);
         MidRowsParams p = params_of(t->x, t->weights, t->outs, d->n, 1, d->rows, d->k, split, nullptr);
         p.activation = d->glu_activation, p.gate_first = d->glu_gate_first ? 1 : 0;
@@ -493,6 +501,7 @@ hipattn_status projection(const hipops_projection_desc* d, const hipops_projecti
         if (add && (!t->residual || (t->gamma == nullptr) != (t->normalised == nullptr))) return fail(HIPATTN_INVALID_ARGUMENT, "projection: null pointer");
         if (add && (!aligned16(t->residual) || !aligned16(t->gamma) || !aligned16(t->normalised))) return refuse("operands off 16 bytes");
         if (t->gamma && (!float_type(d->gamma_dtype) || columns > 8 * kNormThreads * kNormKeep)) return refuse("gamma or row length of the norm");
+        if (add && t->gamma && norm_over_inputs(t->residual, t->gamma, d->gamma_dtype, t->outs[0], t->normalised, d->rows, columns)) return refuse("results over an input");
         if (rope && d->rotated_outputs) {
             if (!t->cos || !t->sin) return fail(HIPATTN_INVALID_ARGUMENT, "projection: null pointer");
             if (d->head_size < 8 || d->head_size % 8 != 0 || !float_type(d->table_dtype)) return refuse("head size or table type");
@@ -535,6 +544,7 @@ hipattn_status residual_norm(const void* product, const void* residual, const vo
         return refuse("types");
     if (rows < 1 || rows > 0x7fffffffLL || n < 8 || n % 8 != 0 || n > 8 * kNormThreads * kNormKeep) return refuse("sizes");
     if (!aligned16(product) || !aligned16(residual) || !aligned16(gamma) || !aligned16(out) || !aligned16(normalised)) return refuse("operands off 16 bytes");
+    if (norm_over_inputs(residual, gamma, gamma_dtype, out, normalised, rows, n)) return refuse("results over an input");
     FinishParams f{};
     f.product = product, f.residual = residual, f.gamma = gamma, f.out[0] = out, f.normalised = normalised;
     f.columns = (int)n, f.m = (int)rows, f.dtype = dtype, f.gamma_dtype = gamma_dtype, f.eps = eps;

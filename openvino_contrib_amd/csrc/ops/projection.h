@@ -14,7 +14,8 @@ extern "C" {
  *   _GLU   out[0] [rows, n[0] / 2] = hipops_glu of x * weights[0]^T
  * Everything is `dtype` (HIPATTN_F16 / BF16) but the tables and gamma; sums and what is done to them are
  * fp32, rounded once (the products are not rounded before).  n[i] is a multiple of 8, k of 64, pointers are
- * 16-byte aligned, and what _GLU writes is no part of x; HIPATTN_UNSUPPORTED, with nothing launched, for what the kernels do not take: the
+ * 16-byte aligned, what _GLU writes is no part of x, and normalised none of residual
+ * (but may be all of it) nor out[0] of gamma; HIPATTN_UNSUPPORTED, with nothing launched, for what the kernels do not take: the
  * operators one by one do.  The workspace holds rows * sum(n) floats or more (not needed for _GLU);
  * hipops_matmul_workspace_size's is enough for every split of k. */
 #define HIPOPS_PROJECTION_ROPE 0
@@ -48,7 +49,7 @@ hipattn_status hipops_projection(const hipops_projection_desc* desc, const hipop
 
 /* The second half of _ADD with gamma for any number of rows, behind a product that is there: out = product + residual, rounded, and
  * normalised = hipops_rms_norm of it, all [rows, n] of `dtype` (HIPATTN_F16 / BF16); n a multiple of 8 up to 16,384, pointers 16-byte
- * aligned (HIPATTN_UNSUPPORTED otherwise). */
+ * aligned, normalised no part of residual (but it may be all of it) nor out of gamma (HIPATTN_UNSUPPORTED otherwise). */
 hipattn_status hipops_residual_norm(const void* device_product, const void* device_residual, const void* device_gamma, void* device_out,
                                     void* device_normalised, int64_t rows, int64_t n, float eps, int dtype, int gamma_dtype,
                                     hipattn_stream stream);

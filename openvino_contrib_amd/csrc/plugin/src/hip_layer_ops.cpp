@@ -556,7 +556,10 @@ private:
         for (const void* x : {product, residual, gamma, (const void*)sum, (const void*)normalised})
             if (x == nullptr || (uintptr_t)x % 16 != 0) return false;
         products[0]->Execute(context, *t[0].in, *t[0].out, *t[0].workbuffers);
-        HIP_OPS_CHECK(hipops_residual_norm(product, residual, gamma, sum, normalised, m.m, m.n, d.eps, d.dtype, d.gamma_dtype, context.stream.get()));
+        const hipattn_status st =
+            hipops_residual_norm(product, residual, gamma, sum, normalised, m.m, m.n, d.eps, d.dtype, d.gamma_dtype, context.stream.get());
+        if (st == HIPATTN_UNSUPPORTED) return false;  // (results over an input; the product is taken again)
+        HIP_OPS_CHECK(st);
         return true;
     }
 };

@@ -72,3 +72,24 @@ def test_new_prompts_read_the_rows_that_the_writer_quantised(hip, oracle, seqs, 
         chunk = np.concatenate([np.arange(begins[s], begins[s + 1]) for s in range(len(seqs)) if seqs[s][1] > 1])
         np.testing.assert_array_equal(results[0][chunk], results[1][chunk])
         assert H.scaled_bound_error(results[0], ref, "%s broken %d" % (seqs, broken)) <= 1e-2
+
+
+@pytest.mark.parametrize("room", [0, 1])
+def test_new_prompts_without_room_for_the_copy(hip, oracle, room):
+    """A caller with the workspace of a call without such prompts, or a byte less than the copy takes: the rows come from the cache, bit for bit the same."""
+    seqs = [(0, 640), (0, 33), (200, 1), (0, 417)]
+    case = W.make_paged_case(6, seqs, 8, 2, 128, 32, W.BF16, W.BF16, W.U8)
+    dev = H.PagedDeviceCase(hip, case)
+    with_copy = dev.run()[0]
+    desc = H.pa_desc(hip, case)
+    whole, without = hip.paged_attention_workspace_size(desc), hip.paged_attention_workspace_size(H.pa_desc(hip, case, max_context_len=100))
+    assert without < whole
+    ws = hip.DeviceBuffer(whole - 1 if room else without)
+    dev.out.fill(0xFF)
+    hip.paged_attention(desc, dev.q, dev.k_new, dev.v_new, dev.key_cache, dev.value_cache, dev.past_lens, dev.subsequence_begins, dev.block_indices,
+                        dev.block_indices_begins, dev.out, ws)
+    out = H.storage_to_f32(dev.out.download(np.uint16, with_copy.shape), W.BF16)
+    np.testing.assert_array_equal(out, with_copy)
+    assert H.scaled_bound_error(out, H.oracle_paged(oracle, case)[0], "no room") <= 1e-2
+    ws.free()
+    dev.free()

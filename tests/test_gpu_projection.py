@@ -174,3 +174,113 @@ def test_groups_of_the_plugin(hip, extra_reader, hidden, ffn, heads, kv_heads, s
             results.append([H.storage_to_f32(request.output(i)[0], BF16) for i in range(3 if extra_reader else 2)])
         for got, ref in zip(*results):
             assert np.isfinite(ref).all() and scaled_error(got, ref) <= 6 * ROUND[BF16], tokens
+
+
+def test_norms_over_a_part_of_their_inputs_are_refused(hip, ops):  # noqa: F811
+    m, n, k = 16, 512, 64
+    size = m * n * 2
+    memory, ws = hip.DeviceBuffer(8 * size), hip.DeviceBuffer(1 << 20)
+    memory.fill(0)
+
+    class At:
+        nbytes = size
+
+        def __init__(self, offset):
+            self.ptr = type(memory.ptr)(memory.ptr.value + offset)
+
+    x, w, product, residual, gamma = At(0), At(size), At(2 * size), At(3 * size), At(5 * size)
+    free, other = At(6 * size), At(7 * size)
+    for out, normalised, taken in ((free, other, True), (free, residual, True), (residual, other, True), (free, At(3 * size + 1024), False),
+                                   (free, At(4 * size), True), (free, At(2 * size + 16), False), (At(5 * size - 1024), other, False), (gamma, other, False),
+                                   (At(5 * size + 1024), other, True)):
+        calls = (lambda: ops.residual_norm(product, residual, gamma, out, normalised, m, n, 1e-5, BF16, BF16),
+                 lambda: ops.projection(ops.PROJECTION_ADD, BF16, m, k, (n,), x, [w], [out], ws, residual=residual, gamma=gamma, gamma_dtype=BF16,
+                                        normalised=normalised, eps=1e-5))
+        for call in calls:
+            if taken:
+                call()
+                continue
+            with pytest.raises(ops.HipOpsError) as e:
+                call()
+            assert e.value.status == hip.UNSUPPORTED
+    hip.DeviceBuffer(16).download(np.uint8, (1,))  # (waits for what was launched)
+
+
+def _bind(request, inputs, outputs):
+    for i, (buffer, dtype, shape, offset) in enumerate(inputs):
+        request.set_device_input(i, buffer.ptr.value + offset, dtype, shape)
+    for i, (buffer, dtype, shape, offset) in enumerate(outputs):
+        request.set_device_output(i, buffer.ptr.value + offset, dtype, shape)
+
+
+@pytest.mark.parametrize("tokens", [8, 64, 66, 6000])
+@pytest.mark.parametrize("where", ["sum over the residual", "norm over the residual", "norm half the rows behind the residual", "sum over gamma"])
+def test_norm_group_with_results_over_its_inputs(hip, where, tokens):
+    """The caller's device tensors may overlap as far as the operators one by one allow: against the same model run that way."""
+    n, k, row = 1024, 256, 2048
+    rng = np.random.default_rng(tokens)
+    g = P.GraphText("over")
+    x, r, gamma = g.parameter("x", BF16, [-1, k]), g.parameter("residual", BF16, [-1, n]), g.parameter("gamma", BF16, [n])
+    y = g.add("MatMul", "mm", [x, g.constant("w", storage(rng.standard_normal((n, k)) / 16, BF16)[0], "bf16")], transpose_a=False, transpose_b=True)
+    total = g.add("Add", "sum", [y, r])
+    g.result("norm", g.add("RMS", "rms", [total, gamma], epsilon=1e-5, output_type="dynamic"))
+    g.result("total", total)
+    text = g.text()
+    xs, rs, gs = (storage(rng.standard_normal(shape), BF16)[0] for shape in ((tokens, k), (tokens, n), (n,)))
+    results = []
+    for profiled in (False, True):
+        plugin = P.Plugin()
+        if profiled:
+            plugin.set_property("PERF_COUNT", "YES")
+        request = plugin.compile_model(P.Model.from_text(text)).create_infer_request()
+        # one allocation: [x][residual][half as many rows more][gamma, rows of space behind it][free, free]
+        at = [0, tokens * k * 2]
+        at += [at[1] + tokens * 3 // 2 * row]
+        at += [at[2] + tokens * row, at[2] + 2 * tokens * row]
+        memory = hip.DeviceBuffer(at[4] + tokens * row)
+        image = np.zeros(memory.nbytes, np.uint8)
+        for offset, a in zip(at, (xs, rs, gs)):
+            image[offset:offset + a.nbytes] = a.reshape(-1).view(np.uint8)
+        outs = {"sum over the residual": (at[4], at[1]), "norm over the residual": (at[1], at[3]), "norm half the rows behind the residual": (at[1] + tokens // 2 * row, at[3]),
+                "sum over gamma": (at[4], at[2])}[where]
+        _bind(request, [(memory, BF16, [tokens, k], at[0]), (memory, BF16, [tokens, n], at[1]), (memory, BF16, [n], at[2])],
+              [(memory, BF16, [tokens, n], o) for o in outs])
+        for _ in range(3):
+            memory.upload(image)
+            request.infer()
+            after = memory.download(np.uint8, (memory.nbytes,))
+            results.append([H.storage_to_f32(after[o:o + tokens * row].view(np.uint16), BF16) for o in outs])
+        memory.free()
+    for got in results[:3]:
+        for a, b in zip(got, results[3]):
+            assert np.isfinite(b).all() and scaled_error(a, b) <= 3 * ROUND[BF16]
+
+
+@pytest.mark.parametrize("tokens", [4, 33, 64])
+@pytest.mark.parametrize("shift", [0, -512, 512])
+def test_glu_group_with_its_result_over_its_input(hip, tokens, shift):
+    """Through the plugin: the result's device tensor is (in part) the input's, which the product of every column reads."""
+    k = 256
+    rng = np.random.default_rng(tokens)
+    g = P.GraphText("over")
+    x = g.parameter("x", BF16, [-1, k])
+    y = g.add("MatMul", "mm", [x, g.constant("w", storage(rng.standard_normal((2 * k, k)) / 16, BF16)[0], "bf16")], transpose_a=False, transpose_b=True)
+    g.result("out", g.add("GLU", "glu", [y], axis=-1, split_lengths=k, glu_type=0, split_to_glu_idx=0, output_type="dynamic"))
+    request = P.Plugin().compile_model(g.model()).create_infer_request()
+    xs = storage(rng.standard_normal((tokens, k)), BF16)[0]
+    size = tokens * k * 2
+    memory, apart = hip.DeviceBuffer(size + 1024), hip.DeviceBuffer(size)
+    results = []
+    for out in ((apart, BF16, [tokens, k], 0), (memory, BF16, [tokens, k], 512 + shift)):
+        _bind(request, [(memory, BF16, [tokens, k], 512)], [out])
+        for _ in range(3):
+            image = np.zeros(size + 1024, np.uint8)
+            image[512:512 + size] = xs.reshape(-1).view(np.uint8)
+            memory.upload(image)
+            request.infer()
+            whole = out[0].download(np.uint8, (out[0].nbytes,))
+            results.append(H.storage_to_f32(whole[out[3]:out[3] + size].view(np.uint16), BF16))
+    for got in results[1:3]:
+        np.testing.assert_array_equal(got, results[0])
+    for got in results[3:]:
+        assert scaled_error(got, results[0]) <= 3 * ROUND[BF16]
