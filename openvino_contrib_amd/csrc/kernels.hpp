@@ -160,8 +160,8 @@ struct PagedParams {
     uint16_t* shadow_k;
     uint16_t* shadow_v;
     int32_t* shadow_table;
-    int lone_tile;        // (paged_mixed.hip) one sequence, which gets query tiles also if it is a single token: no decode rows, no merge
     int tiles_only;       // (flash_small.hip) tile_prefix counts single-token sequences too: there are no decode rows
+    int lone_tile;        // (paged_mixed.hip) one sequence, which gets query tiles also if it is a single token: no decode rows, no merge
 };
 
 // A shorter prompt is read by few query tiles and costs the writer as much (32 heads on 8, us without -> with: 8 prompts of 100 21.2 -> 23.0, of 300

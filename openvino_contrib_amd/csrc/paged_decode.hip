@@ -29,7 +29,7 @@ __device__ __forceinline__ void plan_block(const PagedParams& p) {
     for (int s = s0; s < s1; s++) {
         // (rows are sequences whenever the lengths matter here: max_q_tiles > 0)
         const int qlen = p.max_q_tiles > 0 ? p.subsequence_begins[s + 1] - p.subsequence_begins[s] : 1;
-        blk += line_units(decode_range(p, s).nb, p.switch_cost);
+        if (!p.lone_tile) blk += line_units(decode_range(p, s).nb, p.switch_cost);
         tile += (qlen >= tiled && p.max_q_tiles > 0) ? (qlen + 127) / 128 : 0;
         if (p.overlap && qlen >= tiled) {
             const int past = p.past_lens[s];
@@ -91,7 +91,8 @@ __device__ __forceinline__ void plan_block(const PagedParams& p) {
         const int qlen = p.max_q_tiles > 0 ? p.subsequence_begins[s + 1] - p.subsequence_begins[s] : 1;
         p.blk_prefix[s] = blk;
         p.tile_prefix[s] = tile;
-        const DecodeRange rg = decode_range(p, s);
+        DecodeRange rg = decode_range(p, s);
+        if (p.lone_tile) rg.nb = 0, rg.empty_row = 0;
         ((DecodeRange*)p.seq_info)[s] = rg;
         if (rg.empty_row) zero_output_row(p, rg.token);  // (rare: an empty block table) nothing will visit this row
         blk += line_units(rg.nb, p.switch_cost);

@@ -128,7 +128,7 @@ __device__ __forceinline__ DecodeRange decode_range(const PagedParams& p, int i)
         single = i >= p.subsequence_begins[0] && i < p.subsequence_begins[p.num_seqs];
     } else {
         r.token = b0;
-        single = b1 - b0 == 1 && !p.lone_tile;
+        single = (b1 - b0 == 1);
     }
     const int table_tokens = (tb1 - tb0) * p.block_size;
     r.ctx = min(past + pos_in_seq + 1, table_tokens);
