@@ -206,8 +206,8 @@ hipattn_status hipattn_sdpa_masked(const hipattn_sdpa_desc* desc, const void* q,
  * nothing to attend is zeros.  No kernel reads outside the cache for such an entry.
  * A mixed batch (single-token and multi-token sequences) with decode_waves == 0 runs its two
  * parts side by side, in one launch at head size 128 and, with 16-bit caches on 16-byte aligned rows, between 64 and
- * 128.  Other shapes (and calls with sinks): the call forks from `stream` onto a side stream that the library keeps for
- * that stream (created by the first such call on it, default priority, destroyed by
+ * 128 (not fp16 queries on a bf16 cache, sinks or alibi_slopes).  Other calls whose kernels fit beside each other: the
+ * call forks from `stream` onto a side stream that the library keeps for that stream (created by the first such call on it, default priority, destroyed by
  * hipattn_stream_destroy; the library keeps at most 32, further streams share one) and joins before
  * it returns, so `stream` order is all the caller has to know, also under stream capture (make the
  * first such call on a stream outside a capture: creating a stream is not a capturable operation).  The

@@ -3,10 +3,10 @@
 //
 // Both take whole compute units.  The first workgroups, which are dispatched first, are the decode part's; the plan on
 // the device has chosen how many of them work and the others leave at once, so that the chunks' workgroups find every
-// compute unit the decode part does not keep.  (One sequence of a short context: no decode part, p.lone_tile.)  As two kernels, the chunks on a side stream, the fork and the join left
-// the chip idle for some 25 us a step.  Measured (us a step, two kernels -> one; 32 heads on 8 kv heads of 128): a prompt of 64 tokens 46 -> 14,
-// of 1,000 60 -> 39; 8 prompts of 1,000 155 -> 138, of 2,000 364 -> 347; six uneven prompts into a u8 cache 193 -> 176; two chunks of 200 beside 20
-// decode rows 49 -> 38, beside 100 long ones 375 -> 368; 8 chunks of 512 beside 120 rows, 64 heads, 585 -> 579.
+// compute unit the decode part does not keep.  (One sequence of a short context: no decode part, p.lone_tile.)  As two kernels, the chunks on a side stream, the fork and the join cost
+// 20 to 27 us where there are no decode rows and about 10 where both parts are long.  Measured (us a step, two kernels -> one; 32 heads on 8 kv heads of 128):
+// a prompt of 64 tokens 41 -> 14, of 1,000 58 -> 38, of 2,100 84 -> 67; 8 prompts of 1,000 142 -> 125, of 2,000 356 -> 339; two chunks of 200
+// beside 20 decode rows 46 -> 37, beside 100 long ones 451 -> 444; 8 chunks of 512 beside 120 rows, 64 heads, 577 -> 567.
 #include "flash_chunk.hpp"
 #include "paged_decode.hpp"
 
