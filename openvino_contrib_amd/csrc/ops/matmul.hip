@@ -1,5 +1,6 @@
 // MatMul: few rows (up to six, up to 16 on small weights) in the kernel of matmul_few_rows.hip, up to 64 in that of
-// matmul_mid_rows.hip where it is the faster one, else through hipBLASLt: a plain library GEMM with fp32 accumulation.  The operator's tensors are row-major; hipBLASLt is column-major, so the product is taken transposed
+// matmul_mid_rows.hip where it is the faster one, else through hipBLASLt: a plain library GEMM with fp32 accumulation.  The
+// operator's tensors are row-major; hipBLASLt is column-major, so the product is taken transposed
 // (C^T = op(B)^T * op(A)^T) with the operands swapped and no data movement.  Descriptors and the
 // algorithm are kept per (device, shape), so a repeated shape costs one hipblasLtMatmul call; the
 // algorithm is the fastest of the heuristic's candidates, timed once when the shape is first seen

@@ -460,6 +460,10 @@ hipattn_status matmul_mid_rows(const hipops_matmul_desc* d, const void* a, const
 // launch each.  Bounded by the weights, once launches are few: us, 4 / 64 rows of hidden 4,096, 32 / 8 heads of 128, MLP 14,336: q, k, v and
 // two rotary embeddings in five to eight launches 33 / 62 -> 15.6 / 20.1; o, residual and norm 18 / 34 -> 13.7 / 16.2; gate|up and SwiGLU
 // 47 / 57 -> 42.0 / 46; down and residual 26 / 42 -> 25.8 / 31.8.
+// Over the sizes (1 to 64 rows, n 64 to 8,192, k 256 to 16,384, weights from HBM, us in a recorded graph): with a rotary embedding 1.4 to 4 times
+// as fast everywhere, with the norm 1.05 to 2 times.  A residual alone is 0.9 to 1.9 times: two launches either way, and up to 8 rows the kernel of few rows
+// wins by up to 1.4 us where its wavefronts' k is whole rounds (4 rows: 512 x 1,024 5.8 / 6.6, 3,072 x 3,072 10.4 / 11.1, 4,096 x 8,192 18.1 / 19.3;
+// but 4,096 x 7,168 17.9 / 17.0, 5,120 x 8,192 28.1 / 20.9): too little, and of a model's last Add only, for a line of its own.
 hipattn_status projection(const hipops_projection_desc* d, const hipops_projection_args* t, void* workspace, size_t workspace_bytes, hipStream_t stream) {
     if (!d || !t) return fail(HIPATTN_INVALID_ARGUMENT, "projection: null descriptor");
     const auto refuse = [](const char* why) { return fail(HIPATTN_UNSUPPORTED, "projection: %s", why); };
